@@ -292,10 +292,10 @@ struct Impl : Base {
     void alloc_fields() {
         const size_t n = (size_t)ncells;
         for (StatePtrs<T>* s : {&cur, &nxt}) {
-            s->uth = dalloc<T>(n, owned);
-            s->uph = dalloc<T>(n, owned);
-            s->eta = dalloc<T>(n, owned);
-            s->gam = dalloc<T>(n, owned);
+            s->uth = dalloc<T>(n + kFieldPad, owned);
+            s->uph = dalloc<T>(n + kFieldPad, owned);
+            s->eta = dalloc<T>(n + kFieldPad, owned);
+            s->gam = dalloc<T>(n + kFieldPad, owned);
         }
         ua0 = dalloc<T>(n, owned);
         va0 = dalloc<T>(n, owned);
@@ -933,7 +933,7 @@ std::vector<X> xcd_order(const std::vector<X>& work, X pad, int nxcd) {
 void derive(const sf_bubble_desc& d, sf_derived& o) { sfh::derive_params(d, o); }
 
 void build_tables(Base& c, std::vector<void*>& owned) {
-    std::vector<double> sTc, cTc, sTf, cTf, sF, cscTc, sPc, cPc, sPh, cPh;
+    std::vector<double> sTc, cTc, sTf, cTf, sF, cscTc, sPc, cPc;
     for (int b = 0; b < c.nb; ++b) {
         const BubbleDev& B = c.bub_h[b];
         const double h = B.h;
@@ -952,8 +952,6 @@ void build_tables(Base& c, std::vector<void*>& owned) {
         for (int i = 0; i < B.nph; ++i) {
             sPc.push_back(std::sin((double)i * h));
             cPc.push_back(std::cos((double)i * h));
-            sPh.push_back(std::sin(((double)i - 0.5) * h));
-            cPh.push_back(std::cos(((double)i - 0.5) * h));
         }
     }
     auto up64 = [&](const std::vector<double>& v) {
@@ -971,8 +969,7 @@ void build_tables(Base& c, std::vector<void*>& owned) {
     t.sinTc = up64(sTc); t.cosTc = up64(cTc); t.sinTf = up64(sTf); t.cosTf = up64(cTf);
     t.sinFace = up64(sF); t.cscTc = up64(cscTc);
     t.sinTc32 = up32(sTc); t.cosTc32 = up32(cTc); t.sinTf32 = up32(sTf); t.cosTf32 = up32(cTf);
-    t.sinPc = up64(sPc); t.cosPc = up64(cPc); t.sinPh = up64(sPh); t.cosPh = up64(cPh);
-    t.sinPc32 = up32(sPc); t.cosPc32 = up32(cPc); t.sinPh32 = up32(sPh); t.cosPh32 = up32(cPh);
+    t.sinPc = up64(sPc); t.cosPc = up64(cPc);
 }
 
 template <typename T, typename Ti>
@@ -1089,6 +1086,8 @@ void setup(Base& c, int prec) {
         B.airflow = d.airflow;
         B.viscous = c.opt.viscous ? 1 : 0;
         B.re = c.der[b].re;
+        B.invh32 = (float)B.invh;
+        B.dt32 = (float)B.dt;
         // every bubble starts on a 256-byte boundary (the row kernels load
         // C consecutive cells as one aligned vector)
         off += ((long long)B.nth * B.nph + 63) / 64 * 64;
@@ -1145,6 +1144,8 @@ void setup(Base& c, int prec) {
         for (int w : {128, 64}) c.tile_cands.push_back(build_tiles(w));
     c.geom.tiles = c.tile_cands[0].tiles;
     c.geom.ntiles = c.tile_cands[0].ntiles;
+    c.geom.wide_tiles = true;
+    for (int b = 0; b < nb; ++b) c.geom.wide_tiles = c.geom.wide_tiles && c.bub_h[b].nph >= 64;
     c.geom.pow2_rows = true;
     for (int b = 0; b < nb; ++b) c.geom.pow2_rows = c.geom.pow2_rows && c.bub_h[b].mask >= 0;
     // Row blocks, one launch per row width: C consecutive cells per thread
@@ -1818,6 +1819,7 @@ int sf_set_dt(sf_ctx* ctx, int32_t b, double dt_seconds) {
                 drop_calibration(c);
             }
             c.bub_h[k].dt = dtn;
+            c.bub_h[k].dt32 = (float)dtn;
             c.time_h[k].dt_s = dt_seconds;
         }
         SF_HIP(hipMemcpy(c.bub_d, c.bub_h.data(), c.nb * sizeof(BubbleDev), hipMemcpyHostToDevice));

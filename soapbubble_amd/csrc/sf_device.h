@@ -21,6 +21,7 @@ struct BubbleDev {
     double h, invh, dt;          // grid spacing, 1/h, non-dimensional step
     double M, Cr, gs, gamma_max, eva;
     double re;                   // Re^-1 of the VISCOUS path
+    float invh32, dt32;          // 1/h and dt for the FP32 traces
     int gravity, evaporation, airflow, viscous;
 };
 
@@ -91,31 +92,26 @@ struct Tables {
     const double *sinTc, *cosTc, *sinTf, *cosTf, *sinFace, *cscTc;
     // per-row, FP32 copies
     const float *sinTc32, *cosTc32, *sinTf32, *cosTf32;
-    // per-column: phi = i h and phi = (i - 1/2) h
-    const double *sinPc, *cosPc, *sinPh, *cosPh;
-    const float *sinPc32, *cosPc32, *sinPh32, *cosPh32;
+    // per-column: phi = i h
+    const double *sinPc, *cosPc;
 };
 
 template <typename T> struct TabSel;
 template <> struct TabSel<double> {
+    static __device__ __forceinline__ double invh(const BubbleDev& B) { return B.invh; }
+    static __device__ __forceinline__ double dt(const BubbleDev& B) { return B.dt; }
     static __device__ __forceinline__ const double* sTc(const Tables& t) { return t.sinTc; }
     static __device__ __forceinline__ const double* cTc(const Tables& t) { return t.cosTc; }
     static __device__ __forceinline__ const double* sTf(const Tables& t) { return t.sinTf; }
     static __device__ __forceinline__ const double* cTf(const Tables& t) { return t.cosTf; }
-    static __device__ __forceinline__ const double* sPc(const Tables& t) { return t.sinPc; }
-    static __device__ __forceinline__ const double* cPc(const Tables& t) { return t.cosPc; }
-    static __device__ __forceinline__ const double* sPh(const Tables& t) { return t.sinPh; }
-    static __device__ __forceinline__ const double* cPh(const Tables& t) { return t.cosPh; }
 };
 template <> struct TabSel<float> {
+    static __device__ __forceinline__ float invh(const BubbleDev& B) { return B.invh32; }
+    static __device__ __forceinline__ float dt(const BubbleDev& B) { return B.dt32; }
     static __device__ __forceinline__ const float* sTc(const Tables& t) { return t.sinTc32; }
     static __device__ __forceinline__ const float* cTc(const Tables& t) { return t.cosTc32; }
     static __device__ __forceinline__ const float* sTf(const Tables& t) { return t.sinTf32; }
     static __device__ __forceinline__ const float* cTf(const Tables& t) { return t.cosTf32; }
-    static __device__ __forceinline__ const float* sPc(const Tables& t) { return t.sinPc32; }
-    static __device__ __forceinline__ const float* cPc(const Tables& t) { return t.cosPc32; }
-    static __device__ __forceinline__ const float* sPh(const Tables& t) { return t.sinPh32; }
-    static __device__ __forceinline__ const float* cPh(const Tables& t) { return t.cosPh32; }
 };
 
 // ---------------------------------------------------------------- math ----
@@ -155,16 +151,14 @@ __device__ __forceinline__ float tatan2(float y, float x) {
 }
 __device__ __forceinline__ double tatan2(double y, double x) { return atan2(y, x); }
 
-// Normalisation of a direction: returns |v| and 1/|v| from |v|^2. FP32 uses
-// the hardware reciprocal square root; FP64 the correctly rounded sqrt and
-// division.
-__device__ __forceinline__ void norm_inv(float s, float& n, float& inv) {
-    inv = __builtin_amdgcn_rsqf(s);
-    n = s > 0.0f ? s * inv : s;   // |0| = 0 as length() gives, not 0 * inf
-}
-__device__ __forceinline__ void norm_inv(double s, double& n, double& inv) {
-    n = sqrt(s);
-    inv = 1.0 / n;
+// 1 / sqrt(s) of a positive s: FP32 the hardware estimate (within an ulp);
+// FP64 that estimate r (about 1e-8) times 1 + e/2 + 3 e^2/8, e = 1 - s r^2
+// (the next term is below 1e-23), within an ulp or two.
+__device__ __forceinline__ float inv_root(float s) { return __builtin_amdgcn_rsqf(s); }
+__device__ __forceinline__ double inv_root(double s) {
+    const double r = __builtin_amdgcn_rsq(s);
+    const double e = fma(-(s * r), r, 1.0);
+    return fma(r * e, fma(e, 0.375, 0.5), r);
 }
 // FP64 reciprocal of a positive finite y: the hardware estimate refined by
 // two Newton steps r += r (1 - y r), each of which squares the relative
@@ -187,21 +181,14 @@ __device__ __forceinline__ double qdiv(double a, double y) {
     return a / y;
 }
 __device__ __forceinline__ float trcp(float x) { return __builtin_amdgcn_rcpf(x); }
-__device__ __forceinline__ double trcp(double x) { return 1.0 / x; }
+__device__ __forceinline__ double trcp(double x) { return rcp64(x); }
 
-// sin/cos of the great-circle step. The step is a small angle (|u| dt), so
-// FP32 uses the Taylor series to x^7 / x^6 below 1/16 rad (truncation below
-// 2e-16 / 6e-15, under FP32 rounding); FP64 and large steps use sincos.
-__device__ __forceinline__ void sincos_step(float x, float* s, float* c) {
-    if (fabsf(x) < 0.0625f) {
-        float x2 = x * x;
-        *s = x * (1.0f + x2 * (-1.0f / 6.0f + x2 * (1.0f / 120.0f + x2 * (-1.0f / 5040.0f))));
-        *c = 1.0f + x2 * (-0.5f + x2 * (1.0f / 24.0f + x2 * (-1.0f / 720.0f)));
-    } else {
-        sincosf(x, s, c);
-    }
-}
-__device__ __forceinline__ void sincos_step(double x, double* s, double* c) { sincos(x, s, c); }
+__device__ __forceinline__ void tsincos(float x, float* s, float* c) { sincosf(x, s, c); }
+__device__ __forceinline__ void tsincos(double x, double* s, double* c) { sincos(x, s, c); }
+__device__ __forceinline__ float tfma(float a, float b, float c) { return fmaf(a, b, c); }
+__device__ __forceinline__ double tfma(double a, double b, double c) { return fma(a, b, c); }
+__device__ __forceinline__ float tabs(float x) { return fabsf(x); }
+__device__ __forceinline__ double tabs(double x) { return fabs(x); }
 
 // bubbleLerp (bubble.cu:153-160): NaN operands are skipped. With NANS =
 // false the fields are known to hold no NaN (a per-bubble flag that every
@@ -281,62 +268,53 @@ struct Field {
     __device__ __forceinline__ T belt(int row, int lo, T a) const { return belt<true>(row, lo, a); }
 };
 
-// ------------------------------------------- FP32 interior fast path ----
+// ------------------------------------------------ interior fast path ----
 // Away from the polar rows every sampler reduces to one bilinear
 // interpolation between two adjacent rows with no reflection (validateCoord
-// leaves theta alone, no pole branch applies). For FP32 fields without NaNs
-// that case is evaluated directly: the phi wrap by one conditional add or
-// subtract (y + nPhi stays unrounded where the reference's fmod(y + nPhi,
-// nPhi) would round it at the magnitude of nPhi), byte offsets into a
-// buffer resource, and the next row through the scalar offset. A buffer
-// load outside the field returns 0, so no position, however malformed, can
-// read outside it.
-struct FastIdx {
-    int off, off1;   // byte offsets of the lower row's two phi neighbours
-    float aT, aP;
-};
-
-__device__ __forceinline__ __amdgpu_buffer_rsrc_t field_rsrc(const float* p, int rows, int nph) {
-    return __builtin_amdgcn_make_buffer_rsrc((void*)p, (short)0, rows * nph * 4, 0x00020000);
+// leaves theta alone, no pole branch applies). For fields without NaNs that
+// case is evaluated directly, in both precisions and for rows of any length:
+// byte offsets into a buffer resource, the next row through the scalar
+// offset, a corner's two phi neighbours as one 8-byte (FP64: 16-byte) load.
+// The pair of the row's last column takes its second value from the next
+// row: that column loads column 0 instead (few lanes of few waves). Two
+// loads an interpolation instead of four. A buffer load outside the field
+// returns 0, so no position, however malformed, can read outside it; the
+// resource of a field ends kFieldPad values after it (the last pair of its
+// last row), which the state arrays are allocated with.
+constexpr int kFieldPad = 4;
+template <typename T>
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t field_rsrc(const T* p, int cells) {
+    return __builtin_amdgcn_make_buffer_rsrc((void*)p, (short)0,
+                                             (cells + kFieldPad) * (int)sizeof(T), 0x00020000);
+}
+typedef unsigned int u32x2 __attribute__((ext_vector_type(2)));
+typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
+__device__ __forceinline__ void bload1(__amdgpu_buffer_rsrc_t r, int off, int soff, float& v) {
+    v = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(r, off, soff, 0));
+}
+__device__ __forceinline__ void bload1(__amdgpu_buffer_rsrc_t r, int off, int soff, double& v) {
+    v = __builtin_bit_cast(double, __builtin_amdgcn_raw_buffer_load_b64(r, off, soff, 0));
+}
+__device__ __forceinline__ void bload2(__amdgpu_buffer_rsrc_t r, int off, int soff, float& a,
+                                       float& b) {
+    const u32x2 v = __builtin_amdgcn_raw_buffer_load_b64(r, off, soff, 0);
+    a = __uint_as_float(v.x);
+    b = __uint_as_float(v.y);
+}
+__device__ __forceinline__ void bload2(__amdgpu_buffer_rsrc_t r, int off, int soff, double& a,
+                                       double& b) {
+    const u32x4 v = __builtin_amdgcn_raw_buffer_load_b128(r, off, soff, 0);
+    u32x2 lo, hi;
+    lo.x = v.x; lo.y = v.y; hi.x = v.z; hi.y = v.w;
+    a = __builtin_bit_cast(double, lo);
+    b = __builtin_bit_cast(double, hi);
 }
 
-__device__ __forceinline__ float bload(__amdgpu_buffer_rsrc_t r, int off, int soff) {
-    return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(r, off, soff, 0));
-}
-
-// x, y: sampler-relative index coordinates, x in [0, rows - 1). The phi
-// wrap acts on the integer column (the fast path serves rows whose length
-// is a power of two), so the weight y - floor(y) keeps every bit of y, also
-// for y < 0.
-__device__ __forceinline__ FastIdx fast_index(float x, float y, int nph, int mask) {
-    const float fx = floorf(x), fy = floorf(y);
-    FastIdx q;
-    q.aT = x - fx;
-    q.aP = y - fy;
-    const int row = (int)fx * nph, pI = (int)fy;
-    q.off = (row + (pI & mask)) * 4;
-    q.off1 = (row + ((pI + 1) & mask)) * 4;
-    return q;
-}
-
-// The three interpolations as v0 + a (v1 - v0): two operations each instead
-// of the reference's three for (1 - a) v0 + a v1, the same value within an
-// FP32 rounding.
-__device__ __forceinline__ float fast_bilerp(__amdgpu_buffer_rsrc_t r, const FastIdx& q, int row_bytes) {
-    const float v00 = bload(r, q.off, 0), v01 = bload(r, q.off1, 0);
-    const float v10 = bload(r, q.off, row_bytes), v11 = bload(r, q.off1, row_bytes);
-    const float lo = fmaf(q.aP, v01 - v00, v00);
-    const float hi = fmaf(q.aP, v11 - v10, v10);
-    return fmaf(q.aT, hi - lo, lo);
-}
-
-// A traced position in index coordinates, x = ix + fx, y = iy + fy. FP32
-// traces keep the start point's integer index apart from the fraction,
-// which holds the start point's half index and the increment turned along
-// the circle: the interpolation weights then carry the increment's
-// precision instead of the ulp of the absolute index (6e-5 of a cell at
-// index 1000). FP64 traces hold the absolute position in fx, fy (ix = iy =
-// 0).
+// A traced position in index coordinates, x = ix + fx, y = iy + fy: the
+// start point's integer index apart from the fraction, which holds the start
+// point's half index and the increment turned along the circle. The
+// interpolation weights then carry the increment's precision instead of the
+// ulp of the absolute index (FP32: 6e-5 of a cell at index 1000).
 template <typename T>
 struct TPos {
     int ix, iy;
@@ -345,27 +323,100 @@ struct TPos {
     __device__ __forceinline__ T y() const { return (T)iy + fy; }
 };
 
-// fast_index of the point p + (ox, oy) (ox, oy half-integers, added to the
-// fraction exactly): weights from the fraction, the row and column from the
-// integer parts. True when the lower row lies in [0, rows - 2], the case
-// the fast path serves (rows: the field's row count).
-__device__ __forceinline__ bool fast_index_rel(const TPos<float>& p, float ox, float oy, int rows,
-                                               int nph, int mask, FastIdx& q) {
-    const float rx = p.fx + ox, ry = p.fy + oy;
-    const float fx = floorf(rx), fy = floorf(ry);
-    q.aT = rx - fx;
-    q.aP = ry - fy;
-    const int tI = p.ix + (int)fx, pI = p.iy + (int)fy;
-    const int row = tI * nph;
-    q.off = (row + (pI & mask)) * 4;
-    q.off1 = (row + ((pI + 1) & mask)) * 4;
-    return (unsigned)tI < (unsigned)(rows - 1);
+// x split into its floor and the fraction above it.
+__device__ __forceinline__ void split_floor(float x, int& i, float& f) {
+    asm("v_cvt_flr_i32_f32 %0, %1" : "=v"(i) : "v"(x));
+    f = __builtin_amdgcn_fractf(x);
+}
+__device__ __forceinline__ void split_floor(double x, int& i, double& f) {
+    const double fl = floor(x);
+    i = (int)fl;
+    f = x - fl;
 }
 
-template <typename T, bool NANS>
-struct FastPath { static constexpr bool on = false; };
-template <>
-struct FastPath<float, false> { static constexpr bool on = true; };
+// The lower corner of a sample point: row, column (wrapped into the row) and
+// the weights above it.
+template <typename T>
+struct Corner {
+    int t, c;
+    T aT, aP;
+};
+
+// The corner of the point p + (OX, OY) / 2, added to the fraction exactly:
+// weights from the fraction, row and column from the integer parts.
+template <int OX, int OY, typename T, bool P2>
+__device__ __forceinline__ Corner<T> corner_at(const TPos<T>& p, int nph, int mask) {
+    Corner<T> q;
+    split_floor(OX ? p.fx + T(0.5 * OX) : p.fx, q.t, q.aT);
+    split_floor(OY ? p.fy + T(0.5 * OY) : p.fy, q.c, q.aP);
+    q.t += p.ix;
+    q.c += p.iy;
+    q.c = P2 ? (q.c & mask) : wrap_col(q.c, nph, mask);
+    return q;
+}
+
+// The lower row in [0, rows - 2]: no pole between the corners (rows: the
+// field's row count).
+template <typename T>
+__device__ __forceinline__ bool inside(const Corner<T>& q, int rows) {
+    return (unsigned)q.t < (unsigned)(rows - 1);
+}
+
+// The interpolation inside the field. The three interpolations as v0 + a (v1
+// - v0): two operations each instead of the reference's three for (1 - a) v0
+// + a v1, the same value within a rounding.
+template <typename T>
+__device__ __forceinline__ T corner_bilerp(__amdgpu_buffer_rsrc_t r, const Corner<T>& q, int nph) {
+    const int rb = nph * (int)sizeof(T);
+    const int row = __mul24(q.t, nph);
+    const int off = (row + q.c) * (int)sizeof(T);
+    T v00, v01, v10, v11;
+    bload2(r, off, 0, v00, v01);
+    bload2(r, off, rb, v10, v11);
+    if (q.c == nph - 1) {
+        bload1(r, row * (int)sizeof(T), 0, v01);
+        bload1(r, row * (int)sizeof(T), rb, v11);
+    }
+    const T lo = tfma(q.aP, v01 - v00, v00);
+    const T hi = tfma(q.aP, v11 - v10, v10);
+    return tfma(q.aT, hi - lo, lo);
+}
+
+// The interpolation of a field of `rows` rows whose lower or upper row is
+// the one across a pole: the field's first or last row at phi + pi, with the
+// sign SIGN (values that flip across the pole); HALF (u_theta, whose rows
+// stand a whole row from the pole): the two rows two apart, so the distance
+// from the row on this side counts half. What the samplers below give for
+// any point of the sphere, theta in [0, pi].
+template <int SIGN, bool HALF, typename T, bool P2>
+__device__ __forceinline__ T pole_bilerp(__amdgpu_buffer_rsrc_t r, Corner<T> q, int rows, int nph,
+                                         int mask) {
+    auto opposite = [&](int c) {
+        return P2 ? ((c + (nph >> 1)) & mask) : wrap_col(c + nph / 2, nph, mask);
+    };
+    if (q.t < -1) { q.t = -1; q.aT = T(0); }
+    if (q.t > rows - 1) { q.t = rows - 1; q.aT = T(1); }
+    T w0 = T(1) - q.aT, w1 = q.aT;
+    int c0 = q.c, c1 = q.c;
+    if (q.t < 0) {
+        c0 = opposite(q.c);
+        w0 = (HALF ? T(0.5) : T(1)) * T(SIGN) * w0;
+        if (HALF) w1 = T(0.5) + T(0.5) * w1;
+    }
+    if (q.t >= rows - 1) {
+        c1 = opposite(q.c);
+        w1 = (HALF ? T(0.5) : T(1)) * T(SIGN) * w1;
+        if (HALF) w0 = T(0.5) + T(0.5) * w0;
+    }
+    const int r0 = max(q.t, 0) * nph, r1 = min(q.t + 1, rows - 1) * nph;
+    auto at = [&](int row, int c) {
+        T v;
+        bload1(r, (row + (c == nph ? 0 : c)) * (int)sizeof(T), 0, v);
+        return v;
+    };
+    const T l0 = at(r0, c0), l1 = at(r0, c0 + 1), h0 = at(r1, c1), h1 = at(r1, c1 + 1);
+    return w0 * tfma(q.aP, l1 - l0, l0) + w1 * tfma(q.aP, h1 - h0, h0);
+}
 
 // Split a sample position into indices and weights; the phi index is
 // clamped into range so a NaN position cannot address memory outside the
@@ -381,13 +432,8 @@ __device__ __forceinline__ void split_index(T x, T y, int nph, int& tI, int& pI,
 }
 
 // sampleCentered (bubble.cu:320-376)
-template <typename T, bool NANS = true, bool P2 = false, bool FAST = true>
-__device__ T sample_centered(const Field<T, P2>& f, int nth, T rx, T ry) {
-    if constexpr (FAST && FastPath<T, NANS>::on) {
-        if (rx >= 0.5f && rx < (float)nth - 0.5f && f.pow2())
-            return fast_bilerp(field_rsrc(f.p, nth, f.nph), fast_index(rx - 0.5f, ry, f.nph, f.mask),
-                               f.nph * 4);
-    }
+template <typename T, bool NANS = true, bool P2 = false>
+__device__ __forceinline__ T sample_centered(const Field<T, P2>& f, int nth, T rx, T ry) {
     if constexpr (sizeof(T) == 8 && !NANS) {
         // FP64 fields without NaNs, away from the polar rows: the bilinear
         // interpolation of rows floor(x) and floor(x) + 1 that the general
@@ -427,17 +473,9 @@ __device__ T sample_centered(const Field<T, P2>& f, int nth, T rx, T ry) {
 
 // sampleCentered of two fields at one point (the eta and Gamma samples of
 // advectionAllCentered, bubble.cu:957-960) sharing the index computation.
-template <typename T, bool NANS = true, bool P2 = false, bool FAST = true>
-__device__ void sample_centered2(const Field<T, P2>& f, const Field<T, P2>& g, int nth, T rx, T ry, T& of,
+template <typename T, bool NANS = true, bool P2 = false>
+__device__ __forceinline__ void sample_centered2(const Field<T, P2>& f, const Field<T, P2>& g, int nth, T rx, T ry, T& of,
                                  T& og) {
-    if constexpr (FAST && FastPath<T, NANS>::on) {
-        if (rx >= 0.5f && rx < (float)nth - 0.5f && f.pow2()) {
-            const FastIdx q = fast_index(rx - 0.5f, ry, f.nph, f.mask);
-            of = fast_bilerp(field_rsrc(f.p, nth, f.nph), q, f.nph * 4);
-            og = fast_bilerp(field_rsrc(g.p, nth, g.nph), q, g.nph * 4);
-            return;
-        }
-    }
     T x = rx - T(0.5), y = ry;
     const int nph = f.nph;
     bool fl = validate_coord(x, y, nth, nph);
@@ -456,13 +494,8 @@ __device__ void sample_centered2(const Field<T, P2>& f, const Field<T, P2>& g, i
 }
 
 // sampleVPhi (bubble.cu:178-240): values taken across the pole flip sign.
-template <typename T, bool NANS = true, bool P2 = false, bool FAST = true>
-__device__ T sample_vphi(const Field<T, P2>& f, int nth, T rx, T ry) {
-    if constexpr (FAST && FastPath<T, NANS>::on) {
-        if (rx >= 0.5f && rx < (float)nth - 0.5f && f.pow2())
-            return fast_bilerp(field_rsrc(f.p, nth, f.nph),
-                               fast_index(rx - 0.5f, ry + 0.5f, f.nph, f.mask), f.nph * 4);
-    }
+template <typename T, bool NANS = true, bool P2 = false>
+__device__ __forceinline__ T sample_vphi(const Field<T, P2>& f, int nth, T rx, T ry) {
     T x = rx - T(0.5), y = ry + T(0.5);
     const int nph = f.nph;
     bool fl = validate_coord(x, y, nth, nph);
@@ -490,13 +523,8 @@ __device__ T sample_vphi(const Field<T, P2>& f, int nth, T rx, T ry) {
 // interpolate between the first/last row and its phi+pi mirror with half
 // weight. A sample exactly at theta = pi (which the reference reads past
 // the array for) takes the south-cap branch.
-template <typename T, bool NANS = true, bool P2 = false, bool FAST = true>
-__device__ T sample_vtheta(const Field<T, P2>& f, int nth, T rx, T ry) {
-    if constexpr (FAST && FastPath<T, NANS>::on) {
-        if (rx >= 1.0f && rx < (float)nth - 1.0f && f.pow2())
-            return fast_bilerp(field_rsrc(f.p, nth - 1, f.nph),
-                               fast_index(rx - 1.0f, ry, f.nph, f.mask), f.nph * 4);
-    }
+template <typename T, bool NANS = true, bool P2 = false>
+__device__ __forceinline__ T sample_vtheta(const Field<T, P2>& f, int nth, T rx, T ry) {
     T x = rx - T(1), y = ry;
     const int nph = f.nph;
     bool fl = validate_coord(x, y, nth, nph);
@@ -527,213 +555,199 @@ __device__ T sample_vtheta(const Field<T, P2>& f, int nth, T rx, T ry) {
     return fl ? -v : v;
 }
 
-// The samplers at a traced position: the FP32 interior fast path from the
-// split position, else the general sampler at the absolute one.
-template <typename T, bool NANS = true, bool P2 = false>
-__device__ __forceinline__ T sample_vtheta(const Field<T, P2>& f, int nth, const TPos<T>& p) {
-    if constexpr (FastPath<T, NANS>::on) {
-        FastIdx q;
-        if (f.pow2() && fast_index_rel(p, -1.0f, 0.0f, nth - 1, f.nph, f.mask, q))
-            return fast_bilerp(field_rsrc(f.p, nth - 1, f.nph), q, f.nph * 4);
-    }
-    return sample_vtheta<T, NANS, P2, false>(f, nth, p.x(), p.y());
-}
-template <typename T, bool NANS = true, bool P2 = false>
-__device__ __forceinline__ T sample_vphi(const Field<T, P2>& f, int nth, const TPos<T>& p) {
-    if constexpr (FastPath<T, NANS>::on) {
-        FastIdx q;
-        if (f.pow2() && fast_index_rel(p, -0.5f, 0.5f, nth, f.nph, f.mask, q))
-            return fast_bilerp(field_rsrc(f.p, nth, f.nph), q, f.nph * 4);
-    }
-    return sample_vphi<T, NANS, P2, false>(f, nth, p.x(), p.y());
-}
-template <typename T, bool NANS = true, bool P2 = false>
-__device__ __forceinline__ void sample_centered2(const Field<T, P2>& f, const Field<T, P2>& g, int nth,
-                                                 const TPos<T>& p, T& of, T& og) {
-    if constexpr (FastPath<T, NANS>::on) {
-        FastIdx q;
-        if (f.pow2() && fast_index_rel(p, -0.5f, 0.0f, nth, f.nph, f.mask, q)) {
-            of = fast_bilerp(field_rsrc(f.p, nth, f.nph), q, f.nph * 4);
-            og = fast_bilerp(field_rsrc(g.p, nth, g.nph), q, g.nph * 4);
-            return;
+// The samplers at a traced position. NANS: the reference's NaN-skipping
+// interpolation at the absolute position; without it (fields that hold no
+// NaN) one bilinear interpolation from the split position.
+template <typename T, bool NANS, bool P2>
+__device__ __forceinline__ void sample_velocity(const Field<T, P2>& uth, const Field<T, P2>& uph,
+                                                int nth, const TPos<T>& p, T& vt, T& vp) {
+    if constexpr (NANS) {
+        vt = sample_vtheta<T, true, P2>(uth, nth, p.x(), p.y());
+        vp = sample_vphi<T, true, P2>(uph, nth, p.x(), p.y());
+    } else {
+        const int nph = uth.nph, m = uth.mask;
+        const Corner<T> a = corner_at<-2, 0, T, P2>(p, nph, m);
+        const Corner<T> b = corner_at<-1, 1, T, P2>(p, nph, m);
+        const auto ra = field_rsrc(uth.p, (nth - 1) * nph), rp = field_rsrc(uph.p, nth * nph);
+        if (inside(a, nth - 1) && inside(b, nth)) {
+            vt = corner_bilerp(ra, a, nph);
+            vp = corner_bilerp(rp, b, nph);
+        } else {
+            vt = pole_bilerp<-1, true, T, P2>(ra, a, nth - 1, nph, m);
+            vp = pole_bilerp<-1, false, T, P2>(rp, b, nth, nph, m);
         }
     }
-    sample_centered2<T, NANS, P2, false>(f, g, nth, p.x(), p.y(), of, og);
+}
+template <typename T, bool NANS, bool P2>
+__device__ __forceinline__ void sample_centred_at(const Field<T, P2>& f, const Field<T, P2>& g, int nth,
+                                                  const TPos<T>& p, T& of, T& og) {
+    if constexpr (NANS) {
+        sample_centered2<T, true, P2>(f, g, nth, p.x(), p.y(), of, og);
+    } else {
+        const int nph = f.nph, m = f.mask;
+        const Corner<T> q = corner_at<-1, 0, T, P2>(p, nph, m);
+        const auto rf = field_rsrc(f.p, nth * nph), rg = field_rsrc(g.p, nth * nph);
+        if (inside(q, nth)) {
+            of = corner_bilerp(rf, q, nph);
+            og = corner_bilerp(rg, q, nph);
+        } else {
+            of = pole_bilerp<1, false, T, P2>(rf, q, nth, nph, m);
+            og = pole_bilerp<1, false, T, P2>(rg, q, nth, nph, m);
+        }
+    }
 }
 
 // ------------------------------------------------------ great circle ----
-// The start frame (w, u_, v_) and speed after the transported midpoint
-// velocity, i.e. the first two stages shared by traceGreatCircle
-// (bubble.cu:416-496) and the vector advection kernels (bubble.cu:651-731,
-// 787-867). Positions on the sphere are kept Cartesian: the sin/cos of a
-// traced point's theta and phi are its z, rho, x/rho and y/rho, which is
-// the reference's cos(acos(z)), sin(acos(z)), cos(atan2(y,x)), sin(atan2(y,x))
-// without the round trip.
+// One leg of a back-trace (traceGreatCircle, bubble.cu:416-506, and the
+// vector advection kernels, bubble.cu:651-766, 787-902), in the coordinates
+// of the start point: x towards its meridian's point of the equator, y east,
+// z the pole, so the start point is w = (sin t0, 0, cos t0), its frame e_theta
+// = (cos t0, 0, -sin t0), e_phi = (0, 1, 0), and no trigonometry of phi enters.
+// Moving by `step` against the velocity (a, b) reaches
+//   q = w cos(s) + (a e_theta + b e_phi) k,   s = |u| step, k = -step sin(s) / s,
+// with sin(s) / s and cos(s) by their series in s^2 (no root of |u|^2, no
+// unit direction). Its angles from the start point are
+//   sin dphi   = q_y / rho,
+//   sin dtheta = rho cos t0 - q_z sin t0 = a k + cos t0 q_y tan(dphi / 2)
+// (the second form free of the first one's cancellation: it keeps the
+// increment's relative precision in FP32). The velocity sampled at q is
+// carried back along the circle by v - (v . w)(q + w) / (1 + q . w), in the
+// two points' frames a rotation by g with
+//   cos g (1 + cos s) = cos dphi (1 + q_z cos t0) + rho sin t0,
+//   sin g (1 + cos s) = sin dphi (q_z + cos t0).
+// The reference forms the same points and components from Cartesian
+// vectors, a unit direction and its cross products: about 340 vector
+// instructions a velocity trace, this form about 170.
 template <typename T>
-struct Circle {
-    T w0, w1, w2, u0, u1, u2, v0, v1, v2, unorm;
-    T gx, gy, sT, cT, sP, cP;   // start point: index coordinates and trig
-    TPos<T> start;              // start point, split as the traced positions
+struct TraceStart {
+    int ix, iy;
+    T hx, hy;      // index coordinates ix + hx, iy + hy (hx, hy 0 or 1/2)
+    T sT, cT;      // sin, cos of the start point's theta
+};
+template <typename T>
+struct Leg {
+    TPos<T> p;     // the point reached
+    T cg, sg;      // rotation of its frame's components into the start frame's
 };
 
-template <typename T, bool P2 = false>
-struct VelCtx {
-    Field<T, P2> uth, uph;
-    int nth;
-    T invh, dt;
-};
+// sin(s) / s, cos(s) and 1 / (1 + cos(s)) = sec^2(s/2) / 2 from s^2 below
+// 1/256, truncated below the rounding (first term left out: s^6 / 7! =
+// 1e-11, s^6 / 6!, 17 s^6 / 5760 = 2e-10 in FP32; s^12 / 13! and the like in
+// FP64, the third through the reciprocal).
+__device__ __forceinline__ void small_step(float s2, float& sc, float& c, float& in) {
+    sc = fmaf(s2, fmaf(s2, 1.0f / 120.0f, -1.0f / 6.0f), 1.0f);
+    c = fmaf(s2, fmaf(s2, 1.0f / 24.0f, -0.5f), 1.0f);
+    in = fmaf(s2, fmaf(s2, 1.0f / 48.0f, 0.125f), 0.5f);
+}
+__device__ __forceinline__ void small_step(double s2, double& sc, double& c, double& in) {
+    sc = 1.0 + s2 * (-1.0 / 6 + s2 * (1.0 / 120 + s2 * (-1.0 / 5040 + s2 * (1.0 / 362880 +
+                                                                           s2 * (-1.0 / 39916800)))));
+    c = 1.0 + s2 * (-0.5 + s2 * (1.0 / 24 + s2 * (-1.0 / 720 + s2 * (1.0 / 40320 +
+                                                                     s2 * (-1.0 / 3628800)))));
+    in = rcp64(1.0 + c);
+}
+// asin(s) and tan(asin(s) / 2) = s / (1 + sqrt(1 - s^2)) for |s| below 0.1
+// (FP64: 0.063), cos(asin(s)) above CosMin: by their series (truncated at
+// 5e-9 rad and 4e-8 relative in FP32; at 1e-19 in FP64, the second through
+// the cosine)
+template <typename T> struct CosMin;
+template <> struct CosMin<float> { static constexpr float v = 0.995f; };
+template <> struct CosMin<double> { static constexpr double v = 0.998; };
+__device__ __forceinline__ float asin_small(float s) {
+    const float s2 = s * s;
+    return s * fmaf(s2, fmaf(s2, 3.0f / 40.0f, 1.0f / 6.0f), 1.0f);
+}
+__device__ __forceinline__ double asin_small(double s) {
+    const double s2 = s * s;
+    return s * (1.0 + s2 * (1.0 / 6 + s2 * (3.0 / 40 + s2 * (5.0 / 112 + s2 * (35.0 / 1152 +
+                                                              s2 * (63.0 / 2816 + s2 * (231.0 / 13312)))))));
+}
+__device__ __forceinline__ float tan_half(float s, float) {
+    const float y = s * s;
+    return s * fmaf(y, fmaf(y, 0.0625f, 0.125f), 0.5f);
+}
+__device__ __forceinline__ double tan_half(double s, double c) { return s * rcp64(1.0 + c); }
 
-// The small angle a = atan2(n, d) between a traced point and its start
-// point, given (n, d) = k (sin a, cos a) and k_inv = 1 / k: with s = n k_inv
-// = sin a, the odd series s + s^3/6 + 3 s^5/40 of asin(s) below |s| = 1/10
-// (truncation under 5e-9 rad; no division, the scale k is 1 or the 1/rho
-// that the tangent frame needs anyway), the general atan2 otherwise (a
-// large step, or the phi change of a trace that passes close to a pole).
-__device__ __forceinline__ float small_angle(float n, float d, float k_inv) {
-    const float sn = n * k_inv, cs = d * k_inv;
-    if (cs > 0.0f && fabsf(sn) < 0.1f) {
-        const float s2 = sn * sn;
-        return sn * (1.0f + s2 * (1.0f / 6.0f + s2 * (3.0f / 40.0f)));
+template <typename T>
+__device__ __forceinline__ void trace_leg(const TraceStart<T>& o, T a, T b, T step, T invh,
+                                          Leg<T>& g) {
+    const T s2 = tfma(a, a, b * b) * (step * step);
+    T sc, c, in;
+    small_step(s2, sc, c, in);
+    const T k = -step * sc;
+    T qx, qy = b * k, qz, rho, ir;
+    const T ak = a * k;
+    qx = tfma(o.cT, ak, o.sT * c);
+    qz = tfma(-o.sT, ak, o.cT * c);
+    const T r2 = tfma(qx, qx, qy * qy);
+    ir = inv_root(r2);
+    rho = r2 * ir;
+    T sf = qy * ir, cf = qx * ir;
+    T dth = asin_small(tfma(o.cT * qy, tan_half(sf, cf), ak)), dph = asin_small(sf);
+    g.cg = tfma(cf, tfma(qz, o.cT, T(1)), rho * o.sT) * in;
+    g.sg = sf * (qz + o.cT) * in;
+    // cos dphi above CosMin bounds |sin dphi|, and s below 1/16 leaves
+    // |sin dtheta| <= s + s |tan(dphi / 2)| < 0.066
+    if (!(s2 < T(1.0 / 256) && cf > CosMin<T>::v)) {
+        // a large step, or a trace that passes close to a pole: the same
+        // angles by atan2, and the rotation from the tangents of the circle
+        // at both points (1 + cos(s) loses its digits near the antipode)
+        const T un = tsqrt(tfma(a, a, b * b)), iu = un > T(0) ? T(1) / un : T(0);
+        const T ua = a * iu, ub = b * iu;
+        T sn;
+        tsincos(-un * step, &sn, &c);
+        qx = tfma(o.cT * ua, sn, o.sT * c);
+        qy = ub * sn;
+        qz = tfma(-(o.sT * ua), sn, o.cT * c);
+        rho = tsqrt(tfma(qx, qx, qy * qy));
+        cf = T(1);    // at a pole: the start point's meridian
+        sf = T(0);
+        if (rho > T(0)) {
+            cf = qx / rho;
+            sf = qy / rho;
+        }
+        dth = tatan2(rho * o.cT - qz * o.sT, qz * o.cT + rho * o.sT);
+        dph = tatan2(sf, cf);
+        const T t0 = o.cT * ua * c - o.sT * sn, t1 = ub * c, t2 = -(o.sT * ua) * c - o.cT * sn;
+        const T et = qz * (cf * t0 + sf * t1) - rho * t2, ep = cf * t1 - sf * t0;
+        g.cg = et * ua + ep * ub;
+        g.sg = et * ub - ep * ua;
     }
-    return tatan2(n, d);
+    g.p.ix = o.ix;
+    g.p.iy = o.iy;
+    g.p.fx = tfma(dth, invh, o.hx);
+    g.p.fy = tfma(dph, invh, o.hy);
 }
 
-// Index-space coordinates of a traced point (x, y, z), rho = sin(theta) and
-// ir = 1 / rho (used where rho > 0). FP64: theta = atan2(rho, z), phi =
-// atan2(y, x). FP32: theta and phi as the start point's plus the angles
-// turned from it, theta - theta0 = atan2(rho z0 - z rho0, z z0 + rho rho0) in
-// the meridian half-plane (a unit vector: scale 1) and phi - phi0 =
-// atan2(y x0 - x y0, x x0 + y y0) (x0, y0 the start point's cos phi0,
-// sin phi0; scale rho): the same angles, with the grid-exact start index
-// carrying the magnitude so FP32 keeps the small increment's precision.
+// A velocity (vt, vp) at the leg's point, in the start point's frame.
 template <typename T>
-__device__ __forceinline__ void point_index(const Circle<T>& o, T x, T y, T z, T invh, TPos<T>& p,
-                                            T& rho, T& ir);
-template <>
-__device__ __forceinline__ void point_index(const Circle<double>& o, double x, double y, double z,
-                                            double invh, TPos<double>& p, double& rho, double& ir) {
-    rho = sqrt(x * x + y * y);
-    ir = 1.0 / rho;
-    p.ix = p.iy = 0;
-    p.fx = atan2(rho, z) * invh;
-    p.fy = atan2(y, x) * invh;
-}
-template <>
-__device__ __forceinline__ void point_index(const Circle<float>& o, float x, float y, float z,
-                                            float invh, TPos<float>& p, float& rho, float& ir) {
-    const float r2 = x * x + y * y;
-    ir = __builtin_amdgcn_rsqf(r2);
-    rho = r2 > 0.0f ? r2 * ir : 0.0f;
-    p.ix = o.start.ix;
-    p.iy = o.start.iy;
-    p.fx = o.start.fx + small_angle(rho * o.cT - z * o.sT, z * o.cT + rho * o.sT, 1.0f) * invh;
-    p.fy = o.start.fy + small_angle(y * o.cP - x * o.sP, x * o.cP + y * o.sP, ir) * invh;
+__device__ __forceinline__ void carry_back(const Leg<T>& g, T vt, T vp, T& a, T& b) {
+    a = tfma(vt, g.cg, -(vp * g.sg));
+    b = tfma(vt, g.sg, vp * g.cg);
 }
 
-// The start point (index coordinates gx, gy: multiples of 1/2) in the split
-// form of the traced positions.
-template <typename T>
-__device__ __forceinline__ TPos<T> start_pos(T gx, T gy) {
-    TPos<T> p;
-    if constexpr (sizeof(T) == 4) {
-        const T fx = tfloor(gx), fy = tfloor(gy);
-        p.ix = (int)fx;
-        p.iy = (int)fy;
-        p.fx = gx - fx;
-        p.fy = gy - fy;
-    } else {
-        p.ix = p.iy = 0;
-        p.fx = gx;
-        p.fy = gy;
+// The back-trace from a start point with velocity (a, b): the half step's
+// velocity carried back, the full step with it. Returns whether the point
+// moves (the reference returns the start point, and a zero or NaN speed for
+// the velocity, where either speed is not positive); `speed2` that speed
+// squared where it does not.
+template <typename T, bool NANS, bool P2>
+__device__ __forceinline__ bool back_trace(const Field<T, P2>& uth, const Field<T, P2>& uph, int nth,
+                                           const TraceStart<T>& o, T a, T b, T dt, T invh, Leg<T>& g,
+                                           T& speed2) {
+    speed2 = a * a + b * b;
+    bool moves = speed2 > T(0);
+    if (moves) {
+        T vt, vp;
+        trace_leg(o, a, b, T(0.5) * dt, invh, g);
+        sample_velocity<T, NANS, P2>(uth, uph, nth, g.p, vt, vp);
+        carry_back(g, vt, vp, a, b);
+        speed2 = a * a + b * b;
+        moves = speed2 > T(0);
+        if (moves) trace_leg(o, a, b, dt, invh, g);
     }
-    return p;
-}
-
-// The components along uc and along vc = q x uc of the tangent vector with
-// (e_theta, e_phi) components (vT, vP) at the unit point q = (x, y, z)
-// (rho = sin theta, ir = 1 / rho), uc a unit tangent at q. (e_theta,
-// e_phi, q) is right-handed, so vc = (e_theta . uc) e_phi - (e_phi . uc)
-// e_theta and the two components are a plane rotation of (vT, vP): the
-// reference's dot products with the Cartesian vector (bubble.cu:476-487,
-// 754-765) without forming it. At a pole (rho = 0) the frame of phi = 0.
-template <typename T>
-__device__ __forceinline__ void circle_components(T x, T y, T z, T rho, T ir, T vT, T vP, T uc0,
-                                                  T uc1, T uc2, T& along, T& across) {
-    T cp = T(1), sp = T(0);
-    if (rho > T(0)) { cp = x * ir; sp = y * ir; }
-    const T ct = z * (cp * uc0 + sp * uc1) - rho * uc2;   // e_theta . uc
-    const T cf = cp * uc1 - sp * uc0;                       // e_phi . uc
-    along = vT * ct + vP * cf;
-    across = vP * ct - vT * cf;
-}
-
-template <typename T, bool NANS = true, bool P2 = false>
-__device__ __forceinline__ bool circle_mid(const VelCtx<T, P2>& c, T gx, T gy, T sinT, T cosT, T sinP,
-                                           T cosP, T guT, T guP, Circle<T>& o) {
-    o.gx = gx; o.gy = gy; o.sT = sinT; o.cT = cosT; o.sP = sinP; o.cP = cosP;
-    o.start = start_pos(gx, gy);
-    T u0 = guT * (cosT * cosP) - guP * sinP;
-    T u1 = guT * (cosT * sinP) + guP * cosP;
-    T u2 = -guT * sinT;
-    o.w0 = cosP * sinT; o.w1 = sinP * sinT; o.w2 = cosT;
-    T inv;
-    norm_inv(u0 * u0 + u1 * u1 + u2 * u2, o.unorm, inv);
-    if (!(o.unorm > T(0))) return false;
-    o.u0 = u0 * inv; o.u1 = u1 * inv; o.u2 = u2 * inv;
-    T s, co;
-    sincos_step(T(-0.5) * o.unorm * c.dt, &s, &co);
-    T mx = o.u0 * s + o.w0 * co, my = o.u1 * s + o.w1 * co, mz = o.u2 * s + o.w2 * co;
-    TPos<T> mp;
-    T rho, ir;
-    point_index(o, mx, my, mz, c.invh, mp, rho, ir);
-    T muT = sample_vtheta<T, NANS>(c.uth, c.nth, mp);
-    T muP = sample_vphi<T, NANS>(c.uph, c.nth, mp);
-    // the midpoint velocity along the circle (mguP) and across it (mguT)
-    T uc0 = o.u0 * co - o.w0 * s, uc1 = o.u1 * co - o.w1 * s, uc2 = o.u2 * co - o.w2 * s;
-    T mguP, mguT;
-    circle_components(mx, my, mz, rho, ir, muT, muP, uc0, uc1, uc2, mguP, mguT);
-    // v_ of the start frame = w x u_
-    T v0 = o.w1 * o.u2 - o.w2 * o.u1, v1 = o.w2 * o.u0 - o.w0 * o.u2, v2 = o.w0 * o.u1 - o.w1 * o.u0;
-    u0 = mguP * o.u0 + mguT * v0;
-    u1 = mguP * o.u1 + mguT * v1;
-    u2 = mguP * o.u2 + mguT * v2;
-    norm_inv(u0 * u0 + u1 * u1 + u2 * u2, o.unorm, inv);
-    if (!(o.unorm > T(0))) return false;
-    o.u0 = u0 * inv; o.u1 = u1 * inv; o.u2 = u2 * inv;
-    o.v0 = o.w1 * o.u2 - o.w2 * o.u1;
-    o.v1 = o.w2 * o.u0 - o.w0 * o.u2;
-    o.v2 = o.w0 * o.u1 - o.w1 * o.u0;
-    return true;
-}
-
-// Departure point of the full step: returns its index-space coordinates and
-// the Cartesian point (bubble.cu:498-505, 734-743).
-template <typename T, bool P2>
-__device__ __forceinline__ void circle_depart(const VelCtx<T, P2>& c, const Circle<T>& o, T& s, T& co,
-                                              T& px, T& py, T& pz, TPos<T>& pos, T& rho, T& ir) {
-    sincos_step(-o.unorm * c.dt, &s, &co);
-    px = o.u0 * s + o.w0 * co;
-    py = o.u1 * s + o.w1 * co;
-    pz = o.u2 * s + o.w2 * co;
-    point_index(o, px, py, pz, c.invh, pos, rho, ir);
-}
-
-// Velocity at the departure point transported back along the circle into
-// the start frame (bubble.cu:745-766, 881-902).
-template <typename T, bool NANS = true, bool P2 = false>
-__device__ __forceinline__ void transport_back(const VelCtx<T, P2>& c, const Circle<T>& o, T& r0, T& r1,
-                                               T& r2) {
-    T s, co, px, py, pz, rho, ir;
-    TPos<T> pp;
-    circle_depart(c, o, s, co, px, py, pz, pp, rho, ir);
-    T puT = sample_vtheta<T, NANS>(c.uth, c.nth, pp);
-    T puP = sample_vphi<T, NANS>(c.uph, c.nth, pp);
-    T uc0 = o.u0 * co - o.w0 * s, uc1 = o.u1 * co - o.w1 * s, uc2 = o.u2 * co - o.w2 * s;
-    T b, a;
-    circle_components(px, py, pz, rho, ir, puT, puP, uc0, uc1, uc2, b, a);
-    r0 = b * o.u0 + a * o.v0;
-    r1 = b * o.u1 + a * o.v1;
-    r2 = b * o.u2 + a * o.v2;
+    if (!moves) g.p = TPos<T>{o.ix, o.iy, o.hx, o.hy};
+    return moves;
 }
 
 // ------------------------------------------------------------ BIMOCQ ----
@@ -780,11 +794,6 @@ struct CellRef {
 __device__ __forceinline__ CellRef cell_ref(const Tables& tab, const BubbleDev& B, int j, int i) {
     return CellRef{j + 0.5, (double)i, tab.sinTc[B.rt0 + j], tab.cosTc[B.rt0 + j],
                    tab.sinPc[B.ct0 + i], tab.cosPc[B.ct0 + i]};
-}
-__device__ __forceinline__ double asin_small(double s) {
-    const double s2 = s * s;
-    return s * (1.0 + s2 * (1.0 / 6 + s2 * (3.0 / 40 + s2 * (5.0 / 112 + s2 * (35.0 / 1152 +
-                                                                              s2 * (63.0 / 2816))))));
 }
 __device__ __forceinline__ P2d index_near(double invh, const U3& r, const CellRef& o) {
     const double rho = sqrt(r.x * r.x + r.y * r.y);
@@ -846,7 +855,7 @@ __device__ __forceinline__ U3 slerp_u(const U3& f, const U3& t, double alpha) {
 
 // sampleMapping (bubble.cu:539-603) on a unit-vector map: the corner
 // selection of the reference, three spherical interpolations.
-__device__ U3 sample_map_u(const UMap& M, size_t off, int nth, int nph, double rx, double ry) {
+__device__ __forceinline__ U3 sample_map_u(const UMap& M, size_t off, int nth, int nph, double rx, double ry) {
     const int m = (nph & (nph - 1)) == 0 ? nph - 1 : -1;
     if (rx >= 0.5 && rx < (double)nth - 0.5 && m >= 0) {
         // away from the polar rows: the corners of rows floor(x), floor(x) + 1

@@ -21,111 +21,108 @@
 #include "sf_device.h"
 #include "sf_launch.h"
 
+#include <type_traits>
+
 namespace sfk {
 
 constexpr double kEps = 1e-7;   // bubble.cu:28
 constexpr double kThresh = 0.0; // bubble.cu:27
 
 // ------------------------------------------------------------ advection ----
-// One cell: eta and Gamma at the centre (j+1/2, i), u_phi at the west face
-// (j+1/2, i-1/2), u_theta at the south face (j+1, i). NANS selects the
-// reference's NaN-skipping interpolation; without it the fields hold no NaN.
-// P2: every bubble of the launch has rows whose length is a power of two.
-template <typename T, bool NANS, bool P2>
-__device__ __forceinline__ void advect_cell(const BubbleDev& B, const Tables& tab,
-                                            const StatePtrs<T>& in, const StatePtrs<T>& out, int j,
-                                            int i) {
-    const size_t c = (size_t)j * B.nph + i;
-    VelCtx<T, P2> v;
-    v.uth = Field<T, P2>{in.uth + B.off, B.nph, B.mask, B.nth - 2};
-    v.uph = Field<T, P2>{in.uph + B.off, B.nph, B.mask, B.nth - 1};
-    v.nth = B.nth;
-    v.invh = (T)B.invh;
-    v.dt = (T)B.dt;
-    const Field<T, P2> feta{in.eta + B.off, B.nph, B.mask, B.nth - 1};
-    const Field<T, P2> fgam{in.gam + B.off, B.nph, B.mask, B.nth - 1};
-
-    const T sinTc = TabSel<T>::sTc(tab)[B.rt0 + j], cosTc = TabSel<T>::cTc(tab)[B.rt0 + j];
-    const T sinPc = TabSel<T>::sPc(tab)[B.ct0 + i], cosPc = TabSel<T>::cPc(tab)[B.ct0 + i];
-
-    // Start-point samples. Away from the two polar rows the sample positions
-    // are grid-aligned, and the samplers reduce to their interior branch with
-    // weights 0 or 1/2 (exactly the values the general path computes); the
-    // polar rows go through the general samplers.
-    const bool interior = j > 0 && j < B.nth - 1;
-
-    // eta, Gamma at the cell centre: traceGreatCircle + two samples
-    {
-        const T gx = (T)j + T(0.5), gy = (T)i;
-        T guT, guP;
-        if (interior && !NANS) {
-            // the same samples without their zero-weight terms (which add
-            // 0 x finite: nothing, in fields that hold no NaN)
-            guT = lerp_s<T, false>(v.uth.at(j - 1, i), v.uth.at(j, i), T(0.5));
-            guP = v.uph.template belt<false>(j, i, T(0.5));
-        } else if (interior) {
-            guT = lerp_s<T, NANS>(v.uth.template belt<NANS>(j - 1, i, T(0)),
-                                  v.uth.template belt<NANS>(j, i, T(0)), T(0.5));
-            guP = lerp_s<T, NANS>(v.uph.template belt<NANS>(j, i, T(0.5)),
-                                  v.uph.template belt<NANS>(j + 1, i, T(0.5)), T(0));
-        } else {
-            guT = sample_vtheta<T, NANS>(v.uth, B.nth, gx, gy);
-            guP = sample_vphi<T, NANS>(v.uph, B.nth, gx, gy);
-        }
-        Circle<T> o;
-        TPos<T> tp;
-        if (circle_mid<T, NANS>(v, gx, gy, sinTc, cosTc, sinPc, cosPc, guT, guP, o)) {
-            T s, co, px, py, pz, rho, ir;
-            circle_depart(v, o, s, co, px, py, pz, tp, rho, ir);
-        } else {
-            tp = o.start;
-        }
-        T en, gn;
-        sample_centered2<T, NANS>(feta, fgam, B.nth, tp, en, gn);
-        out.eta[B.off + c] = en;
-        out.gam[B.off + c] = gn;
-    }
-    // u_phi at the west face
-    {
-        const T gx = (T)j + T(0.5), gy = (T)i - T(0.5);
-        const T sinP = TabSel<T>::sPh(tab)[B.ct0 + i], cosP = TabSel<T>::cPh(tab)[B.ct0 + i];
-        T guT = interior ? lerp_s<T, NANS>(v.uth.template belt<NANS>(j - 1, i - 1, T(0.5)),
-                                           v.uth.template belt<NANS>(j, i - 1, T(0.5)), T(0.5))
-                         : sample_vtheta<T, NANS>(v.uth, B.nth, gx, gy);
-        T guP = in.uph[B.off + c];
-        Circle<T> o;
-        T res;
-        if (!circle_mid<T, NANS>(v, gx, gy, sinTc, cosTc, sinP, cosP, guT, guP, o)) {
-            res = o.unorm;
-        } else {
-            T r0, r1, r2;
-            transport_back<T, NANS>(v, o, r0, r1, r2);
-            res = -sinP * r0 + cosP * r1;
-        }
-        out.uph[B.off + c] = res;
-    }
-    // u_theta at the south face; sampleVPhi there is always the interior
-    // branch with weights 1/2
-    if (j < B.nth - 1) {
-        const T gx = (T)j + T(1), gy = (T)i;
-        const T sinT = TabSel<T>::sTf(tab)[B.rt0 + j + 1], cosT = TabSel<T>::cTf(tab)[B.rt0 + j + 1];
-        T guT = in.uth[B.off + c];
-        T guP = lerp_s<T, NANS>(v.uph.template belt<NANS>(j, i, T(0.5)),
-                                v.uph.template belt<NANS>(j + 1, i, T(0.5)), T(0.5));
-        Circle<T> o;
-        T res;
-        if (!circle_mid<T, NANS>(v, gx, gy, sinT, cosT, sinPc, cosPc, guT, guP, o)) {
-            res = o.unorm;
-        } else {
-            T r0, r1, r2;
-            transport_back<T, NANS>(v, o, r0, r1, r2);
-            res = r0 * (cosT * cosPc) + r1 * (cosT * sinPc) - r2 * sinT;
-        }
-        out.uth[B.off + c] = res;
+// The start point and velocity of a cell's back-traces: KIND 0 from the
+// centre (j+1/2, i) for eta and Gamma, 1 from the west face (j+1/2, i-1/2) for
+// u_phi, 2 from the south face (j+1, i) for u_theta. The start points are
+// grid-aligned, so the samplers reduce to averages of two or four values
+// (the values the general path computes, without its terms of weight 0,
+// which add 0 x finite in fields that hold no NaN); in the two polar rows
+// u_theta's average is 3/4 of the row's own face and -1/4 of the one across
+// the pole. NANS selects the reference's NaN-skipping samplers.
+template <int KIND, typename T, bool NANS, bool P2>
+__device__ __forceinline__ void trace_start(const BubbleDev& B, const Tables& tab,
+                                            const Field<T, P2>& uth, const Field<T, P2>& uph, int j,
+                                            int i, TraceStart<T>& o, T& a, T& b) {
+    const int nth = B.nth;
+    o.ix = KIND == 2 ? j + 1 : j;
+    o.iy = KIND == 1 ? i - 1 : i;
+    o.hx = KIND == 2 ? T(0) : T(0.5);
+    o.hy = KIND == 1 ? T(0.5) : T(0);
+    const T* s = KIND == 2 ? TabSel<T>::sTf(tab) : TabSel<T>::sTc(tab);
+    const T* c = KIND == 2 ? TabSel<T>::cTf(tab) : TabSel<T>::cTc(tab);
+    o.sT = s[B.rt0 + o.ix];
+    o.cT = c[B.rt0 + o.ix];
+    if constexpr (KIND == 2) {
+        a = uth.at(j, i);
+        b = lerp_s<T, NANS>(uph.template belt<NANS>(j, i, T(0.5)),
+                            uph.template belt<NANS>(j + 1, i, T(0.5)), T(0.5));
+    } else if constexpr (NANS) {
+        a = sample_vtheta<T, true>(uth, nth, o.ix + o.hx, o.iy + o.hy);
+        b = KIND == 1 ? uph.at(j, i) : sample_vphi<T, true>(uph, nth, o.ix + o.hx, o.iy + o.hy);
+    } else {
+        // rows north and south of the centres; in a polar row the one across
+        const bool pole = j == 0 || j == nth - 1;
+        const int r0 = j == 0 ? 0 : j - 1, r1 = j == nth - 1 ? nth - 2 : j;
+        const int s0 = j == 0 ? nth : 0, s1 = j == nth - 1 ? nth : 0;
+        auto face = [&](int r, int sh) {
+            if constexpr (KIND == 1)
+                return lerp_s<T, false>(uth.at(r, i - 1 + sh), uth.at(r, i + sh), T(0.5));
+            else
+                return uth.at(r, i + sh);
+        };
+        const T n = face(r0, s0), w = face(r1, s1);
+        a = T(0.5) * n + T(0.5) * w;
+        if (pole) a = j == 0 ? T(0.75) * w - T(0.25) * n : T(0.75) * n - T(0.25) * w;
+        b = KIND == 1 ? uph.at(j, i) : uph.template belt<false>(j, i, T(0.5));
     }
 }
 
-template <typename T, bool P2>
+template <int KIND, typename T, bool NANS, bool P2>
+__device__ __forceinline__ void advect_kind(const BubbleDev& B, const Tables& tab,
+                                            const StatePtrs<T>& in, const StatePtrs<T>& out, int j,
+                                            int i) {
+    const int nth = B.nth;
+    if (KIND == 2 && j >= nth - 1) return;
+    const size_t c = (size_t)B.off + (size_t)j * B.nph + i;
+    const Field<T, P2> uth{in.uth + B.off, B.nph, B.mask, nth - 2};
+    const Field<T, P2> uph{in.uph + B.off, B.nph, B.mask, nth - 1};
+    TraceStart<T> o;
+    T a, b;
+    trace_start<KIND, T, NANS, P2>(B, tab, uth, uph, j, i, o, a, b);
+    Leg<T> g;
+    T speed2;
+    const bool moves = back_trace<T, NANS, P2>(uth, uph, nth, o, a, b, TabSel<T>::dt(B),
+                                               TabSel<T>::invh(B), g, speed2);
+    if constexpr (KIND == 0) {
+        const Field<T, P2> feta{in.eta + B.off, B.nph, B.mask, nth - 1};
+        const Field<T, P2> fgam{in.gam + B.off, B.nph, B.mask, nth - 1};
+        T en, gn;
+        sample_centred_at<T, NANS>(feta, fgam, nth, g.p, en, gn);
+        out.eta[c] = en;
+        out.gam[c] = gn;
+    } else {
+        T rt = speed2, rp = speed2;
+        if (moves) {
+            T vt, vp;
+            sample_velocity<T, NANS>(uth, uph, nth, g.p, vt, vp);
+            carry_back(g, vt, vp, rt, rp);
+        }
+        if constexpr (KIND == 1) out.uph[c] = rp;
+        else out.uth[c] = rt;
+    }
+}
+
+// Bound by vector issue at the large sizes: 658 VALU instructions a wave of 64
+// cells at developed flow (962 before the traces took the start point's
+// frame), at four cycles each 35 us of the 37.6 us a 1024x2048 launch takes
+// (45.6 before; FP64 172 -> 72 us, 1000x2000 78 -> 41 us, the 96-bubble batch
+// 115 -> 94 us, 2048x4096 165 -> 132 us), and by the length of one thread's
+// dependent chain at the small ones.
+// SPLIT: a block does one of the three traces of its tile's cells
+// (blockIdx.y), else all of them: a third of the chain where the launch
+// leaves the chip idle, but the tile set-up three times and the velocities
+// through the caches three times where it fills it. WIDE: no tile is narrower than a wave, so
+// a wave's cells share their row: said to the compiler, the row's table
+// entries and offsets load and compute in scalar registers.
+template <typename T, bool P2, bool SPLIT, bool WIDE>
 __global__ __launch_bounds__(256) void k_advect(const int4* __restrict__ tiles,
                                                 const BubbleDev* __restrict__ bub,
                                                 BubbleTime* __restrict__ btime, Tables tab,
@@ -135,7 +132,7 @@ __global__ __launch_bounds__(256) void k_advect(const int4* __restrict__ tiles,
     const BubbleDev B = bub[tl.x];
     // the previous step's time advance lands here, before any kernel of this
     // step reads the time
-    if (tl.y == 0 && tl.z == 0 && threadIdx.x == 0) {
+    if (tl.y == 0 && tl.z == 0 && threadIdx.x == 0 && blockIdx.y == 0) {
         if (btime[tl.x].pending) {
             btime[tl.x].t += btime[tl.x].dt_s;
             btime[tl.x].pending = 0;
@@ -147,11 +144,16 @@ __global__ __launch_bounds__(256) void k_advect(const int4* __restrict__ tiles,
     }
     int j, i;
     tile_cell(tl, j, i);
+    if (WIDE) j = __builtin_amdgcn_readfirstlane(j);
     if (j >= B.nth || i >= B.nph) return;
-    if (btime[tl.x].nans)
-        advect_cell<T, true, P2>(B, tab, in, out, j, i);
-    else
-        advect_cell<T, false, P2>(B, tab, in, out, j, i);
+    auto run = [&](auto nans) {
+        constexpr bool N = decltype(nans)::value;
+        if (!SPLIT || blockIdx.y == 0) advect_kind<0, T, N, P2>(B, tab, in, out, j, i);
+        if (!SPLIT || blockIdx.y == 1) advect_kind<1, T, N, P2>(B, tab, in, out, j, i);
+        if (!SPLIT || blockIdx.y == 2) advect_kind<2, T, N, P2>(B, tab, in, out, j, i);
+    };
+    if (btime[tl.x].nans) run(std::true_type{});
+    else run(std::false_type{});
 }
 
 // ---------------------------------------------------------- air flow ----
@@ -1969,25 +1971,18 @@ __global__ __launch_bounds__(256) void k_bm_init(const int4* __restrict__ tiles,
 
 // traceGreatCircle from the cell centre (j + 1/2, i) over dt (either sign)
 template <typename T, bool NANS>
-__device__ __forceinline__ void trace_centre(const VelCtx<T>& v, const Tables& tab,
-                                             const BubbleDev& B, int j, int i, double& tx,
-                                             double& ty) {
-    const T gx = (T)j + T(0.5), gy = (T)i;
-    const T sinTc = TabSel<T>::sTc(tab)[B.rt0 + j], cosTc = TabSel<T>::cTc(tab)[B.rt0 + j];
-    const T sinPc = TabSel<T>::sPc(tab)[B.ct0 + i], cosPc = TabSel<T>::cPc(tab)[B.ct0 + i];
-    const T guT = sample_vtheta<T, NANS>(v.uth, B.nth, gx, gy);
-    const T guP = sample_vphi<T, NANS>(v.uph, B.nth, gx, gy);
-    Circle<T> o;
-    TPos<T> tp;
-    if (circle_mid<T, NANS>(v, gx, gy, sinTc, cosTc, sinPc, cosPc, guT, guP, o)) {
-        T s, co, px, py, pz, rho, ir;
-        circle_depart(v, o, s, co, px, py, pz, tp, rho, ir);
-    } else {
-        tp = o.start;
-    }
+__device__ __forceinline__ void trace_centre(const Field<T>& uth, const Field<T>& uph,
+                                             const Tables& tab, const BubbleDev& B, T dt, int j,
+                                             int i, double& tx, double& ty) {
+    TraceStart<T> o;
+    T a, b;
+    trace_start<0, T, NANS, false>(B, tab, uth, uph, j, i, o, a, b);
+    Leg<T> g;
+    T speed2;
+    back_trace<T, NANS, false>(uth, uph, B.nth, o, a, b, dt, TabSel<T>::invh(B), g, speed2);
     // the split position summed in FP64 (exact)
-    tx = (double)tp.ix + (double)tp.fx;
-    ty = (double)tp.iy + (double)tp.fy;
+    tx = (double)g.p.ix + (double)g.p.fx;
+    ty = (double)g.p.iy + (double)g.p.fy;
 }
 
 // updateForward / updateBackward (bubble.cu:1049-1118 with
@@ -1997,16 +1992,13 @@ template <typename T, bool NANS>
 __device__ __forceinline__ void bm_maps_cell(const BubbleDev& B, const Tables& tab,
                                              const StatePtrs<T>& cur, const BimocqPtrs& P, int j,
                                              int i) {
-    VelCtx<T> v;
-    v.uth = Field<T>{cur.uth + B.off, B.nph, B.mask, B.nth - 2};
-    v.uph = Field<T>{cur.uph + B.off, B.nph, B.mask, B.nth - 1};
-    v.nth = B.nth;
-    v.invh = (T)B.invh;
+    const Field<T> uth{cur.uth + B.off, B.nph, B.mask, B.nth - 2};
+    const Field<T> uph{cur.uph + B.off, B.nph, B.mask, B.nth - 1};
     const size_t o = (size_t)B.off, c = o + (size_t)j * B.nph + i;
     for (int dir = 0; dir < 2; ++dir) {
-        v.dt = dir == 0 ? (T)(-B.dt) : (T)B.dt;
         double tx, ty;
-        trace_centre<T, NANS>(v, tab, B, j, i, tx, ty);
+        trace_centre<T, NANS>(uth, uph, tab, B, dir == 0 ? -TabSel<T>::dt(B) : TabSel<T>::dt(B),
+                              j, i, tx, ty);
         const U3 s = sample_map_u(dir == 0 ? P.fwd : P.bwd, o, B.nth, B.nph, tx, ty);
         const UMap& out = dir == 0 ? P.nfwd : P.nbwd;
         out.x[c] = s.x;
@@ -2273,12 +2265,25 @@ __global__ __launch_bounds__(256) void k_bm_finish(const int4* __restrict__ tile
 template <typename T>
 void launch_advect(hipStream_t s, const LaunchGeom& g, const BubbleDev* bub, BubbleTime* bt,
                    const Tables& tab, StatePtrs<T> in, StatePtrs<T> out) {
-    if (g.pow2_rows)
-        hipLaunchKernelGGL((k_advect<T, true>), dim3(g.ntiles), dim3(256), 0, s, g.tiles, bub, bt,
-                           tab, in, out);
-    else
-        hipLaunchKernelGGL((k_advect<T, false>), dim3(g.ntiles), dim3(256), 0, s, g.tiles, bub, bt,
-                           tab, in, out);
+    // Both sides measured: 101x202 4.2 us split, 8.0 whole; 256x512 (512
+    // tiles) 5.2, 6.5; 384x768 (1152) 9.1, 9.8; 512x1024 (2048) 12.2, 12.0;
+    // 1024x2048 (8192) 40.7, 37.6; the 96-bubble batch (21504) 117, 94. The
+    // chip holds 2048 blocks of 256 threads (eight waves a SIMD).
+    const bool split = g.ntiles < 2048;
+#define SF_ADV1(P, S, W)                                                                          \
+    hipLaunchKernelGGL((k_advect<T, P, S, W>), dim3(g.ntiles, S ? 3 : 1), dim3(256), 0, s,        \
+                       g.tiles, bub, bt, tab, in, out)
+#define SF_ADV(P, S)                                                                              \
+    do {                                                                                          \
+        if (g.wide_tiles) SF_ADV1(P, S, true); else SF_ADV1(P, S, false);                         \
+    } while (0)
+    if (g.pow2_rows) {
+        if (split) SF_ADV(true, true); else SF_ADV(true, false);
+    } else {
+        if (split) SF_ADV(false, true); else SF_ADV(false, false);
+    }
+#undef SF_ADV1
+#undef SF_ADV
 }
 
 #define SF_CASES(CALL)                                 \

@@ -110,6 +110,7 @@ struct LaunchGeom {
     size_t lds_bytes;    // dynamic LDS of a row block (the reduced line system)
     bool pow2_rows;      // every bubble's row length is a power of two
     bool packed;         // some block holds several rows (RowSeg)
+    bool wide_tiles;     // no cell tile is narrower than a wave
 };
 
 template <typename T>
