@@ -100,6 +100,12 @@ std::vector<X> xcd_order(const std::vector<X>& work, X pad, int nxcd);
 // host-driven instead of as a graph of hundreds of mostly skipped launches.
 constexpr int kCaptureMaxInner = 48;
 
+// The condition bound up to which the automatic inner method takes the
+// spectral preconditioner: at 16 an inner PCG iteration gains a factor 0.6,
+// 27 iterations for the 1e-6 of an FP32 solve in 5 launches each, against
+// about 8 multigrid ones in 34.
+constexpr double kSpMaxCondition = 16.0;
+
 // Everything that does not depend on the precision.
 struct Base {
     sf_options opt{};
@@ -185,6 +191,13 @@ struct Base {
     std::vector<int> sched;   // inner iterations per refinement of the fixed schedule
     int method = 1;           // inner solver: 1 PCG, 2 Chebyshev
     bool mg = false;          // PCG preconditioned by the multigrid V-cycle
+    bool spectral = false;    // PCG preconditioned by the row-mean operator
+    bool method_changed = false;   // ... since the executable graphs were captured
+    // captured spectral steps watch for a schedule that has become too short,
+    // until a calibration gives the same one again
+    bool sp_watch = true;
+    bool sp_recal = false;         // a state was uploaded: its film sets the rate
+    std::vector<int> sp_short;
     bool trace_solve = std::getenv("SF_SOLVE_TRACE") != nullptr;
     int steps_done = 0;
     int stage = 0;            // 0 idle, 1 advected, 2 assembled, 3 solved
@@ -286,7 +299,122 @@ struct Impl : Base {
     void enable_mg() override {
         if (mgp.empty()) alloc_mg();
         mg = true;
+        spectral = false;
         method = 1;
+    }
+
+    // spectral preconditioner (FP32 inner solves): bases per row width, the
+    // spectral array, the row-constant operator, and per row width the item
+    // lists of the transforms and of the theta line solves
+    struct SpLaunch {
+        int4 *fwd = nullptr, *line = nullptr;
+        int nfwd = 0, nline = 0, threads = 0;
+        size_t lds = 0;
+    };
+    std::vector<SpLaunch> spl;
+    SpPtrs spp{};
+    void alloc_spectral() {
+        std::vector<SpDev> dev(nb);
+        long long tot = 0;
+        spl.assign(rgeo.size(), SpLaunch{});
+        for (size_t w = 0; w < rgeo.size(); ++w) {
+            const int nph = rgeo_nph[w], n = nph / 2;
+            int R = 4;
+            while (R * kSpCells < n) R *= 2;
+            const int npad = R * kSpCells, wv = (R + 63) / 64 * 64;
+            SpLaunch& L = spl[w];
+            // at least two modes a block, so the blocks of a bubble are at
+            // most its rows (the r.z slots)
+            L.threads = std::max(256, 2 * wv);
+            const int modes = L.threads / wv;
+            L.lds = (size_t)modes * 6 * R * sizeof(float);
+            std::vector<double> cs(4 * (size_t)nph);
+            for (int t = 0; t < 4 * nph; ++t) cs[t] = std::cos(2.0 * kPi * t / (4.0 * nph));
+            std::vector<float> lam(nph);
+            for (int m = 0; m < nph; ++m) {
+                const double q = std::sin(kPi * ((m + 1) / 2) / nph);
+                lam[m] = (float)(4.0 * q * q);
+            }
+            double* cs_d = dalloc<double>(cs.size(), owned);
+            SF_HIP(hipMemcpy(cs_d, cs.data(), cs.size() * sizeof(double), hipMemcpyHostToDevice));
+            float* lam_d = dalloc<float>(lam.size(), owned);
+            SF_HIP(hipMemcpy(lam_d, lam.data(), lam.size() * sizeof(float), hipMemcpyHostToDevice));
+            float* Qt = dalloc<float>((size_t)nph * nph, owned);
+            float* Q = dalloc<float>((size_t)nph * nph, owned);
+            launch_sp_basis(stream, nph, cs_d, Qt, Q);
+            std::vector<int4> fwd, line;
+            for (int b = 0; b < nb; ++b) {
+                if (bub_h[b].nph != nph) continue;
+                dev[b] = SpDev{Qt, Q, lam_d, tot, npad, 0};
+                tot += (long long)nph * npad;
+                for (int c = 0; c * kSpCols < nph; ++c)
+                    for (int j = 0; j * kSpRows < n; ++j) fwd.push_back(make_int4(b, j, c, 0));
+                for (int g = 0; g * modes < nph; ++g) line.push_back(make_int4(b, g, 0, 0));
+            }
+            auto up = [&](const std::vector<int4>& v, int4*& p, int& k) {
+                k = (int)v.size();
+                p = dalloc<int4>(v.size(), owned);
+                SF_HIP(hipMemcpy(p, v.data(), v.size() * sizeof(int4), hipMemcpyHostToDevice));
+            };
+            up(fwd, L.fwd, L.nfwd);
+            up(line, L.line, L.nline);
+        }
+        SpDev* d = dalloc<SpDev>(nb, owned);
+        SF_HIP(hipMemcpy(d, dev.data(), nb * sizeof(SpDev), hipMemcpyHostToDevice));
+        spp.d = d;
+        spp.Y = dalloc<float>((size_t)tot, owned);
+        spp.coef = dalloc<float>(5 * (size_t)stride, owned);
+    }
+    // The row-constant operator of the assembled system.
+    void sp_coef() {
+        if constexpr (sizeof(Ti) == 4)
+            launch_sp_coef<T>(stream, sgeo, bub_d, tab, nxt.gam, wN, wW, spp, stride);
+    }
+    // The bound on the condition of the preconditioned operator, over all
+    // bubbles (after sp_coef).
+    double sp_condition() {
+        std::vector<float> h(2 * (size_t)stride);
+        SF_HIP(hipMemcpyAsync(h.data(), spp.coef + 3 * stride, h.size() * sizeof(float),
+                              hipMemcpyDeviceToHost, stream));
+        SF_HIP(hipStreamSynchronize(stream));
+        double worst = 0.0;
+        for (int b = 0; b < nb; ++b) {
+            double hi = 0.0, lo = 0.0;
+            for (int j = 0; j < bub_h[b].nth; ++j) {
+                hi = std::max(hi, (double)h[bub_h[b].pr0 + j]);
+                lo = std::max(lo, (double)h[stride + bub_h[b].pr0 + j]);
+            }
+            worst = std::max(worst, hi * lo);
+        }
+        return worst;
+    }
+    // z <- M^-1 r, the partials of r.z to rz_out; gates as mg_vcycle.
+    void sp_apply(bool start, double* rz_out) {
+        if constexpr (sizeof(Ti) == 4) {
+            const int gate = start ? 0 : kMgGateInner;
+            for (const SpLaunch& L : spl) {
+                launch_sp_gemm(stream, L.fwd, L.nfwd, bub_d, ctl_d, spp, r, z, false,
+                               start ? kMgGateStart : gate, sp, partR, stride);
+                launch_sp_line(stream, L.line, L.nline, L.threads, L.lds, bub_d, ctl_d, spp, gate,
+                               rz_out, stride);
+                launch_sp_gemm(stream, L.fwd, L.nfwd, bub_d, ctl_d, spp, r, z, true, gate, sp, partR,
+                               stride);
+            }
+        }
+    }
+    // The spectral preconditioner serves rows up to its largest basis, of
+    // films whose condition bound stays below kSpMaxCondition.
+    bool try_spectral() {
+        if (sizeof(Ti) != 4) return false;
+        for (int b = 0; b < nb; ++b)
+            if (bub_h[b].nth > kSpMaxTheta) return false;
+        if (spl.empty()) alloc_spectral();
+        sp_coef();
+        if (!(sp_condition() <= kSpMaxCondition)) return false;
+        spectral = true;
+        mg = false;
+        method = 1;
+        return true;
     }
 
     void alloc_fields() {
@@ -515,6 +643,10 @@ struct Impl : Base {
             mg_coarsen();
             mg_vcycle(true, partR + 2 * stride);
         }
+        if (spectral) {
+            sp_coef();
+            sp_apply(true, partR + 2 * stride);
+        }
     }
 
     // FP64 residual evaluation k >= 1: x64[k&1] = x64[(k-1)&1] + ecorr (k = 1:
@@ -530,12 +662,12 @@ struct Impl : Base {
         double* xn = x64[k & 1];
         SysPtrs<Ti> s = sys(x64[0]);
         s.e = ecorr;
-        if (last) s.z = nullptr;
+        if (last || spectral) s.z = nullptr;
         for (const LaunchGeom& rg : pgeo)
             launch_resid<T, Ti>(stream, rg, bub_d, time_d, tab, nxt, ctl_d, s, gnext, xo, xn, k,
-                                partR, stride, partB, sp, method == 2 ? sh : nullptr,
-                                check_prev ? 1 : 0);
+                                partR, stride, partB, sp, sh, check_prev ? 1 : 0);
         if (mg && !last) mg_vcycle(true, partR + 2 * stride);
+        if (spectral && !last) sp_apply(true, partR + 2 * stride);
     }
     // Chebyshev iterates: e_1 is z; e_k for k >= 2 rotates over e, Ap, p[0]
     // (k mod 3), so e_{k-1}, e_k and e_{k+1} are distinct.
@@ -653,20 +785,22 @@ struct Impl : Base {
         }
         return all;
     }
-    void inner(int it) {
+    void inner(int it, bool last = false) {
         for (const LaunchGeom& rg : pgeo)
             launch_spmv<Ti>(stream, rg, bub_d, ctl_d, sys(x64[0]), p[(it + 1) & 1], p[it & 1], it, sp,
                             partR, partB, partA, stride);
-        cgstep(it);
+        cgstep(it, last);
     }
     // x, r update and z = M^-1 r of inner PCG iteration `it` (with the
     // multigrid preconditioner: the line-Jacobi z is the V-cycle's first
-    // half-sweep)
-    void cgstep(int it) {
+    // half-sweep); `last`: no iteration follows that reads z
+    void cgstep(int it, bool last = false) {
+        SysPtrs<Ti> s = sys(x64[0]);
+        if (last || spectral) s.z = nullptr;
         for (const LaunchGeom& rg : pgeo)
-            launch_cgstep<Ti>(stream, rg, bub_d, ctl_d, sys(x64[0]), p[it & 1], it, partA, partB,
-                              stride);
-        if (mg) mg_vcycle(false, partB);
+            launch_cgstep<Ti>(stream, rg, bub_d, ctl_d, s, p[it & 1], it, partA, partB, stride);
+        if (mg && !last) mg_vcycle(false, partB);
+        if (spectral && !last) sp_apply(false, partB);
     }
 
     bool all_flags(std::vector<SolveCtl>& c, bool inner_flag) {
@@ -686,10 +820,24 @@ struct Impl : Base {
     // skip the work (graph capture).
     void solve(bool host_driven, bool finalize) override {
         if (host_driven && method == 2 && auto_method() && stiff_for_chebyshev()) {
-            // the automatic inner method continues with multigrid: its
-            // coarse levels and first cycle for this solve, then the PCG
-            // branch below
-            if (trace_solve) std::fprintf(stderr, "[sf solve] stiff operator: multigrid from here on\n");
+            // the automatic inner method continues with PCG, preconditioned
+            // by the row-mean operator or, for an uneven film, by multigrid:
+            // its operator and first application for this solve, then the
+            // PCG branch below
+            method_changed = true;
+            if (try_spectral()) {
+                if (trace_solve) std::fprintf(stderr, "[sf solve] stiff operator: spectral preconditioner\n");
+                sp_apply(true, partR + 2 * stride);
+            } else {
+                if (trace_solve) std::fprintf(stderr, "[sf solve] stiff operator: multigrid from here on\n");
+                enable_mg();
+                mg_coarsen();
+                mg_vcycle(true, partR + 2 * stride);
+            }
+        } else if (host_driven && spectral && !(sp_condition() <= kSpMaxCondition)) {
+            // the film has become too uneven since
+            method_changed = true;
+            if (trace_solve) std::fprintf(stderr, "[sf solve] uneven film: multigrid from here on\n");
             enable_mg();
             mg_coarsen();
             mg_vcycle(true, partR + 2 * stride);
@@ -759,7 +907,7 @@ struct Impl : Base {
                 cgstep(0);
                 for (int it = 1; it < max_inner; ++it) {
                     inner(it);
-                    if ((mg || (it & 3) == 3) && all_flags(c, true)) break;
+                    if ((mg || spectral || (it & 3) == 3) && all_flags(c, true)) break;
                 }
                 all_flags(c, true);
                 int mx = 0;
@@ -771,8 +919,11 @@ struct Impl : Base {
             }
         } else {
             for (size_t k = 0; k < sched.size(); ++k) {
-                for (int it = 0; it < sched[k]; ++it) inner(it);
-                resid((int)k + 1, e, nullptr);
+                for (int it = 0; it < sched[k]; ++it) inner(it, it + 1 == sched[k]);
+                // (statistics of the spare refinement alone, for a schedule
+                // that has become too short)
+                const bool end = k + 1 == sched.size();
+                resid((int)k + 1, e, spectral && end ? sstat_d : nullptr, end);
             }
         }
         if (host_driven && recording) {
@@ -819,6 +970,7 @@ struct Impl : Base {
         SF_HIP(hipMemcpyAsync(dst + B.off, tmp.data(), N * sizeof(T), hipMemcpyHostToDevice, stream));
         if (field == SF_FIELD_ETA || field == SF_FIELD_GAMMA) bimocq_dirty = true;
         if (field <= SF_FIELD_GAMMA) reset_guess(b);
+        if (field <= SF_FIELD_GAMMA && spectral) sp_recal = true;
         if (field <= SF_FIELD_GAMMA) {
             // a new state steps again after a failed solve; the advection
             // samples a state with NaNs by NaN-skipping interpolation
@@ -1543,6 +1695,26 @@ void adapt_schedule(Base& c, const SchedStat* st, int ran) {
     c.sched[0] = n;
 }
 
+// The executable graphs hold the launches of the inner method they were
+// captured with: a host-driven step that changed it drops them (and the
+// schedule of the old one). Returns whether it did.
+bool drop_stale_graphs(Base& c) {
+    if (!c.method_changed) return false;
+    SF_HIP(hipStreamSynchronize(c.stream));
+    for (auto& g : c.graphs) (void)hipGraphExecDestroy(g.second.exec);
+    c.graphs.clear();
+    c.method_changed = false;
+    return true;
+}
+
+// Whether a step of the chunk needed its spare refinement (PCG schedules,
+// which do not adapt: the next steps calibrate again).
+bool spare_ran(const Base& c, const SchedStat* st) {
+    for (int b = 0; b < c.nb; ++b)
+        if (st[b].extra > 0) return true;
+    return false;
+}
+
 void check_index(sf_ctx* ctx, int b) {
     if (!ctx || !ctx->impl) throw Status{SF_ERR_INVALID, "null context"};
     if (b < 0 || b >= ctx->impl->nb) throw Status{SF_ERR_INVALID, "bubble index out of range"};
@@ -1816,6 +1988,8 @@ int sf_set_dt(sf_ctx* ctx, int32_t b, double dt_seconds) {
                 // to the old step
                 c.time_h[k].ghist = c.time_h[k].gpend = 0;
                 c.host_hist = 0;
+                c.sp_watch = true;
+                c.sp_short.clear();
                 drop_calibration(c);
             }
             c.bub_h[k].dt = dtn;
@@ -1848,115 +2022,143 @@ int sf_step(sf_ctx* ctx, int32_t nsteps) {
             c.graphs.clear();
             drop_calibration(c);
         }
-        for (int pass = 0; pass < 2 && want_graph && !c.calibrated; ++pass) {
-            const bool was_mg = c.mg;
-            // calibration: one host-driven step with the guess in effect sets
-            // the first schedule
-            for (; k < nsteps && c.calib_steps < 1; ++k) {
-                c.recording = c.host_hist >= warm;
-                eager_step(c, true);
-                if (c.recording) ++c.calib_steps;
-                c.recording = false;
-            }
-            if (c.calib_steps == 1) {
-                // schedule: per refinement one inner iteration fewer than the
-                // host-driven step ran (it stopped at the first n whose
-                // residual met the target, and launch n - 1 already produces
-                // that iterate e_n), then one spare refinement of one
-                // iteration (a further factor of about ten) that catches a
-                // step needing more; a bubble that converged skips the
-                // remaining kernels
-                c.sched.clear();
-                for (int n : c.calib)
-                    c.sched.push_back(c.opt.max_inner > 0 ? c.opt.max_inner
-                                                          : std::max(c.method == 2 ? n - 1 : n, 1));
-                if (c.sched.empty()) c.sched.push_back(1);
-                // a solve that misses its tolerance stops the bubble when
-                // halt_on_failure is set: one more refinement of margin
-                if (c.opt.halt_on_failure) c.sched.push_back(1);
-                c.sched.push_back(1);
-                if (c.opt.max_outer > 0) c.sched.resize((size_t)c.opt.max_outer, 1);
-                if (c.sched.size() > (size_t)kAccRefine) c.sched.resize(kAccRefine);
-                // Chebyshev: the last refinement (run only when those before
-                // missed the tolerance) takes the line solve z = M^-1 r that
-                // the residual before it produced as its correction, with no
-                // inner launch (the start-residual test moves into its
-                // residual launch): one skipped launch per step fewer
-                if (c.method == 2 && c.sched.size() >= 2) c.sched.back() = 0;
-                c.calibrated = true;
-                if (c.sched[0] > kGraphMaxInner) {
-                    drop_calibration(c);
-                    // the calibration step switched to multigrid: calibrate
-                    // that schedule
-                    if (c.mg && !was_mg) continue;
-                }
-                if (c.trace_solve) {
-                    std::fprintf(stderr, "[sf solve] graph schedule:");
-                    for (int n : c.sched) std::fprintf(stderr, " %d", n);
-                    std::fprintf(stderr, "\n");
-                }
-                if (c.calibrated) {
-                    const bool adapt = c.method == 2 && c.opt.max_inner <= 0;
-                    (void)step_graph(c, kGraphSteps, -1);
-                    if (adapt) {
-                        // the graphs of the calibrated schedule and of one
-                        // inner iteration fewer (where the schedule usually
-                        // settles as the extrapolated guess improves), so
-                        // that no instantiation falls between replays
-                        const int n0 = c.sched[0];
-                        for (int n : {n0, n0 - 1}) {
-                            if (n < 1) continue;
-                            c.sched[0] = n;
-                            (void)step_graph(c, kGraphSteps, 0);
-                            (void)step_graph(c, kGraphSteps, 1);
-                        }
-                        c.sched[0] = n0;
-                    }
-                }
-            }
+        if (c.sp_recal) {
+            c.sp_recal = false;
+            c.sp_watch = true;
+            c.sp_short.clear();
+            drop_calibration(c);
         }
-        if (want_graph && c.calibrated) {
-            for (; k < nsteps && c.host_hist < warm; ++k) eager_step(c, true);
-            // replays in chunks of kAdaptChunk steps, one graph launch each;
-            // with the automatic schedule each chunk's graph ends by handing
-            // its statistics to the host, which reads them one chunk later,
-            // so the device never waits for the host
-            const bool adapt = c.method == 2 && c.opt.max_inner <= 0;
-            if (k < nsteps) {
-                SF_HIP(hipEventRecord(c.ev[0], c.stream));
-                int chunk = 0;
-                while (k < nsteps && c.sched[0] <= kGraphMaxInner) {
-                    const int n = std::min(nsteps - k, kAdaptChunk);
-                    const int p = chunk & 1;
-                    // kGraphSteps steps per launch, the chunk's last launch
-                    // ending with the statistics hand-off
-                    for (int q = 0; q < n; q += kGraphSteps) {
-                        const int m = std::min(kGraphSteps, n - q);
-                        const bool last = q + m == n;
-                        SF_HIP(hipGraphLaunch(step_graph(c, m, adapt && last ? p : -1), c.stream));
-                    }
-                    k += n;
-                    c.host_hist += n;
-                    if (!adapt) continue;
-                    SF_HIP(hipEventRecord(c.cev[p], c.stream));
-                    c.chunk_sched[p] = c.sched[0];
-                    if (chunk > 0) {
-                        SF_HIP(hipEventSynchronize(c.cev[p ^ 1]));
-                        adapt_schedule(c, c.sstat_h + (p ^ 1) * c.nb, c.chunk_sched[p ^ 1]);
-                    }
-                    ++chunk;
+        // calibration, then replays; once more where the spectral
+        // preconditioner's schedule has become too short on the way
+        for (bool again = true; again && k < nsteps;) {
+            again = false;
+            for (int pass = 0; pass < 2 && want_graph && !c.calibrated; ++pass) {
+                const bool was_mg = c.mg || c.spectral;
+                // calibration: one host-driven step with the guess in effect sets
+                // the first schedule
+                for (; k < nsteps && c.calib_steps < 1; ++k) {
+                    c.recording = c.host_hist >= warm;
+                    eager_step(c, true);
+                    if (c.recording) ++c.calib_steps;
+                    c.recording = false;
                 }
-                SF_HIP(hipEventRecord(c.ev[5], c.stream));
-                SF_HIP(hipEventSynchronize(c.ev[5]));
-                if (adapt && chunk > 0) {
-                    const int p = (chunk - 1) & 1;
-                    adapt_schedule(c, c.sstat_h + p * c.nb, c.chunk_sched[p]);
+                (void)drop_stale_graphs(c);
+                if (c.calib_steps == 1) {
+                    // schedule: per refinement one inner iteration fewer than the
+                    // host-driven step ran (it stopped at the first n whose
+                    // residual met the target, and launch n - 1 already produces
+                    // that iterate e_n), then one spare refinement of one
+                    // iteration (a further factor of about ten) that catches a
+                    // step needing more; a bubble that converged skips the
+                    // remaining kernels
+                    c.sched.clear();
+                    for (int n : c.calib)
+                        c.sched.push_back(c.opt.max_inner > 0 ? c.opt.max_inner
+                                                              : std::max(c.method == 2 ? n - 1 : n, 1));
+                    if (c.sched.empty()) c.sched.push_back(1);
+                    // a solve that misses its tolerance stops the bubble when
+                    // halt_on_failure is set: one more refinement of margin
+                    if (c.opt.halt_on_failure) c.sched.push_back(1);
+                    // (the spectral preconditioner's rate follows the film: one more
+                    // iteration of margin in each refinement)
+                    if (c.spectral && c.opt.max_inner <= 0)
+                        for (int& n : c.sched) n += 1;
+                    c.sched.push_back(1);
+                    if (c.opt.max_outer > 0) c.sched.resize((size_t)c.opt.max_outer, 1);
+                    if (c.sched.size() > (size_t)kAccRefine) c.sched.resize(kAccRefine);
+                    // Chebyshev: the last refinement (run only when those before
+                    // missed the tolerance) takes the line solve z = M^-1 r that
+                    // the residual before it produced as its correction, with no
+                    // inner launch (the start-residual test moves into its
+                    // residual launch): one skipped launch per step fewer
+                    if (c.method == 2 && c.sched.size() >= 2) c.sched.back() = 0;
+                    c.calibrated = true;
+                    if (c.sched == c.sp_short) c.sp_watch = false;
+                    if (c.sched[0] > kGraphMaxInner) {
+                        drop_calibration(c);
+                        // the calibration step switched to multigrid: calibrate
+                        // that schedule
+                        if ((c.mg || c.spectral) && !was_mg) continue;
+                    }
+                    if (c.trace_solve) {
+                        std::fprintf(stderr, "[sf solve] graph schedule:");
+                        for (int n : c.sched) std::fprintf(stderr, " %d", n);
+                        std::fprintf(stderr, "\n");
+                    }
+                    if (c.calibrated) {
+                        const bool adapt = c.method == 2 && c.opt.max_inner <= 0;
+                        (void)step_graph(c, kGraphSteps, -1);
+                        if (adapt) {
+                            // the graphs of the calibrated schedule and of one
+                            // inner iteration fewer (where the schedule usually
+                            // settles as the extrapolated guess improves), so
+                            // that no instantiation falls between replays
+                            const int n0 = c.sched[0];
+                            for (int n : {n0, n0 - 1}) {
+                                if (n < 1) continue;
+                                c.sched[0] = n;
+                                (void)step_graph(c, kGraphSteps, 0);
+                                (void)step_graph(c, kGraphSteps, 1);
+                            }
+                            c.sched[0] = n0;
+                        }
+                    }
                 }
-                float ms = 0.f;
-                SF_HIP(hipEventElapsedTime(&ms, c.ev[0], c.ev[5]));
-                c.timing.step_ms += ms;
             }
-            if (c.sched[0] > kGraphMaxInner) drop_calibration(c);
+            if (want_graph && c.calibrated) {
+                for (; k < nsteps && c.host_hist < warm; ++k) eager_step(c, true);
+                if (drop_stale_graphs(c)) {
+                    drop_calibration(c);
+                    again = true;
+                    continue;
+                }
+                // replays in chunks of kAdaptChunk steps, one graph launch each;
+                // with the automatic schedule each chunk's graph ends by handing
+                // its statistics to the host, which reads them one chunk later,
+                // so the device never waits for the host
+                const bool adapt = c.method == 2 && c.opt.max_inner <= 0;
+                const bool watch = adapt || (c.spectral && c.sp_watch && c.opt.max_inner <= 0);
+                if (k < nsteps) {
+                    SF_HIP(hipEventRecord(c.ev[0], c.stream));
+                    int chunk = 0;
+                    while (k < nsteps && c.sched[0] <= kGraphMaxInner && !again) {
+                        const int n = std::min(nsteps - k, kAdaptChunk);
+                        const int p = chunk & 1;
+                        // kGraphSteps steps per launch, the chunk's last launch
+                        // ending with the statistics hand-off
+                        for (int q = 0; q < n; q += kGraphSteps) {
+                            const int m = std::min(kGraphSteps, n - q);
+                            const bool last = q + m == n;
+                            SF_HIP(hipGraphLaunch(step_graph(c, m, watch && last ? p : -1), c.stream));
+                        }
+                        k += n;
+                        c.host_hist += n;
+                        if (!watch) continue;
+                        SF_HIP(hipEventRecord(c.cev[p], c.stream));
+                        c.chunk_sched[p] = c.sched[0];
+                        if (chunk > 0) {
+                            SF_HIP(hipEventSynchronize(c.cev[p ^ 1]));
+                            const SchedStat* st = c.sstat_h + (p ^ 1) * c.nb;
+                            if (adapt) adapt_schedule(c, st, c.chunk_sched[p ^ 1]);
+                            else again = spare_ran(c, st);
+                        }
+                        ++chunk;
+                    }
+                    SF_HIP(hipEventRecord(c.ev[5], c.stream));
+                    SF_HIP(hipEventSynchronize(c.ev[5]));
+                    if (watch && chunk > 0) {
+                        const int p = (chunk - 1) & 1;
+                        const SchedStat* st = c.sstat_h + p * c.nb;
+                        if (adapt) adapt_schedule(c, st, c.chunk_sched[p]);
+                        else again = again || spare_ran(c, st);
+                    }
+                    float ms = 0.f;
+                    SF_HIP(hipEventElapsedTime(&ms, c.ev[0], c.ev[5]));
+                    c.timing.step_ms += ms;
+                }
+                if (again) c.sp_short = c.sched;
+                if (c.sched[0] > kGraphMaxInner || again) drop_calibration(c);
+            }
         }
         for (; k < nsteps; ++k) eager_step(c, true);
         c.steps_done += nsteps;

@@ -1264,11 +1264,14 @@ __global__ void k_cgstep(const int2* __restrict__ rows, const BubbleDev* __restr
         op.load(sys, row, i0, m, nph, j > 0, j < nth - 1);
         op.line(rv, a, cc, d);
     }
-    line_solve<Ti, C>(a, cc, d, nph, steps, reinterpret_cast<Ti*>(lds_raw), redf, sg);
-    if (act) {
-        st_row<C>(sys.z + row + i0, d);
+    // (without z: another preconditioner's launches follow)
+    if (sys.z) {
+        line_solve<Ti, C>(a, cc, d, nph, steps, reinterpret_cast<Ti*>(lds_raw), redf, sg);
+        if (act) {
+            st_row<C>(sys.z + row + i0, d);
 #pragma unroll
-        for (int q = 0; q < C; ++q) acc[0] += (double)rv[q] * (double)d[q];
+            for (int q = 0; q < C; ++q) acc[0] += (double)rv[q] * (double)d[q];
+        }
     }
     seg_sum<2>(acc, red, sg);
     if (valid && sg.lt == 0) {
@@ -1452,6 +1455,271 @@ __global__ void k_mg_line(const int2* __restrict__ rows, const BubbleDev* __rest
         block_sum<1>(acc, red);
         if (threadIdx.x == 0) rz_out[B.pr0 + j] = acc[0];
     }
+}
+
+// --------------------------------------- spectral preconditioner ----
+// z = M^-1 r for the inner PCG of a stiff system whose film is not too uneven:
+// M is the operator with every face weight and mass term replaced by its
+// row's mean over phi. Each of its theta-row blocks is circulant, so the real
+// Fourier basis Q of the row diagonalises them all at once:
+//   z = Q T^-1 Q^t r,  T one tridiagonal theta system per mode k,
+//   diag m_j + wN_j + wN_{j+1} + 4 sin^2(pi k / nph) wW_j, off-diagonal -wN_j.
+// The eigenvalues of M^-1 A lie between the smallest and the largest ratio of
+// a weight to its row's mean (k_sp_coef measures both), so PCG gains a factor
+// (sqrt(K) - 1) / (sqrt(K) + 1) an iteration, K their quotient: 0.05-0.15 on the
+// films of the driver's default parameters, against about 0.2 for a V-cycle
+// of the multigrid preconditioner, in 3 launches instead of 32 (a V-cycle of
+// 256 rows). The transforms are products with a dense matrix on the matrix
+// cores (FP32 MFMA): any row length. Measured at 256x512, radius 0.05 m, 0.005
+// s a step: 5.5 + 5.0 + 5.1 us an application (each launch bound by its
+// latency: loads, four dependent rounds of MFMA, the LDS sum; the 134 MFLOP of
+// a transform are a microsecond of the chip), a captured step 2.5 -> 0.36 ms
+// against the V-cycle's 8 + 5 + 1 iterations of 32 launches.
+
+// Means over phi of one row's face weights and mass term sin(theta) / (dt
+// Gamma), and the ratios to them. A broken cell's zero weights give an
+// infinite ratio.
+template <typename T>
+__global__ __launch_bounds__(256) void k_sp_coef(const int2* __restrict__ rows,
+                                                 const BubbleDev* __restrict__ bub, Tables tab,
+                                                 const T* __restrict__ gam,
+                                                 const float* __restrict__ wN,
+                                                 const float* __restrict__ wW, SpPtrs P,
+                                                 long stride) {
+    __shared__ double red[16 * 3];
+    const int2 rw = rows[blockIdx.x];
+    if (rw.x < 0) return;
+    const BubbleDev B = bub[rw.x];
+    const int j = rw.y, nph = B.nph;
+    const size_t row = (size_t)B.off + (size_t)j * nph;
+    double s[3] = {0.0, 0.0, 0.0};
+    for (int i = threadIdx.x; i < nph; i += blockDim.x) {
+        s[0] += (double)wW[row + i];
+        s[1] += (double)wN[row + i];
+        s[2] += 1.0 / (double)gam[row + i];
+    }
+    block_sum<3>(s, red);
+    const double inv = 1.0 / nph;
+    for (double& v : s) v *= inv;
+    float hi = 0.0f, lo = 0.0f;
+    for (int i = threadIdx.x; i < nph; i += blockDim.x) {
+        const float q[3] = {(float)((double)wW[row + i] / s[0]),
+                            j > 0 ? (float)((double)wN[row + i] / s[1]) : 1.0f,
+                            (float)(1.0 / ((double)gam[row + i] * s[2]))};
+#pragma unroll
+        for (int k = 0; k < 3; ++k) {
+            // a NaN or negative ratio counts as infinite
+            hi = q[k] >= 0.0f ? fmaxf(hi, q[k]) : __builtin_inff();
+            lo = q[k] > 0.0f ? fmaxf(lo, 1.0f / q[k]) : __builtin_inff();
+        }
+    }
+    const double mh = block_max((double)hi, red), ml = block_max((double)lo, red);
+    if (threadIdx.x == 0) {
+        float* c = P.coef + B.pr0 + j;
+        c[0] = (float)s[0];
+        c[stride] = j > 0 ? (float)s[1] : 0.0f;
+        c[2 * stride] = (float)(tab.sinTc[B.rt0 + j] / B.dt * s[2]);
+        c[3 * stride] = (float)mh;
+        c[4 * stride] = (float)ml;
+    }
+}
+
+// Row m of the basis: the constant, then cosine and sine of wave number k =
+// (m + 1) / 2 (the last mode: the alternating one), normalised.
+__global__ __launch_bounds__(256) void k_sp_basis(int nph, const double* __restrict__ cosines,
+                                                  float* __restrict__ Qt, float* __restrict__ Q) {
+    const int m = blockIdx.x, k = (m + 1) / 2;
+    const double s = m == 0 || m == nph - 1 ? sqrt(1.0 / nph) : sqrt(2.0 / nph);
+    // sin(x) = cos(x - pi/2): a quarter of the row's period, in units of a
+    // quarter column
+    for (int i = threadIdx.x; i < nph; i += blockDim.x) {
+        long long t = 4LL * k * i;
+        if (m != 0 && (m & 1) == 0) t += 3LL * nph;
+        const float v = (float)(s * cosines[t % (4LL * nph)]);
+        Qt[(size_t)m * nph + i] = v;
+        Q[(size_t)i * nph + m] = v;
+    }
+}
+
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+struct alignas(4) Quad {
+    float v[4];
+};
+
+// One tile of kSpRows theta rows x kSpCols columns of the forward transform
+// (columns: modes, Y[m][j] = sum_i r[j][i] Qt[m][i]) or the inverse one
+// (columns: cells, z[j][i] = sum_m Y[m][j] Qt[m][i]). The four waves of a
+// block take a quarter of the sum each (the sum is as long as a row, and the
+// tiles of one film alone do not fill the chip) and add up in LDS. Two
+// column tiles a wave share the row operand. Lane (g, l) holds summands k0 +
+// 4 g .. + 3 of row or column l: four products of depth 4 per load. Gates as
+// k_mg_line.
+template <bool INV>
+__global__ __launch_bounds__(256) void k_sp_gemm(const int4* __restrict__ items,
+                                                 const BubbleDev* __restrict__ bub,
+                                                 SolveCtl* __restrict__ ctl, SpPtrs P,
+                                                 const float* __restrict__ r, float* __restrict__ z,
+                                                 int flags, SolveParams sp,
+                                                 const double* __restrict__ partR, long stride) {
+    __shared__ double red[16 * 2];
+    __shared__ f32x4 part[3][2][64];
+    const int4 it = items[blockIdx.x];
+    const int b = it.x;
+    SolveCtl* Cb = ctl + b;
+    if (flag_load(&Cb->outer_done)) return;
+    if ((flags & kMgGateInner) && Cb->inner_done) return;
+    const BubbleDev B = bub[b];
+    if (flags & kMgGateStart) {
+        double sm[2];
+        sum_partials<2>(partR, stride, B.pr0, B.nth, sm, red);
+        if (residual_norm(sm[0], sm[1], sp.absolute) <= sp.tol) {
+            if (it.y == 0 && it.z == 0 && threadIdx.x == 0) flag_store(&Cb->outer_done, 1);
+            return;
+        }
+    }
+    const SpDev D = P.d[b];
+    float* __restrict__ Y = P.Y + D.yoff;
+    const int N = B.nph, n = B.nth;
+    const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6, l = lane & 15, g = lane >> 4;
+    const int j0 = it.y * kSpRows, c0 = it.z * kSpCols;
+    const int quarter = ((N + 63) / 64) * 16;
+    const int kend = min(N, (wid + 1) * quarter);
+    const float* __restrict__ rrow = r + B.off + (size_t)min(j0 + l, n - 1) * N;
+    const bool jin = j0 + l < n;
+    f32x4 acc[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
+    // the column operand's row of this lane's two columns: the summand is
+    // contiguous in it both ways (basis and its transpose)
+    const float* __restrict__ col[2];
+#pragma unroll
+    for (int t = 0; t < 2; ++t)
+        col[t] = (INV ? D.Q : D.Qt) + (size_t)min(c0 + 16 * t + l, N - 1) * N;
+    auto load16 = [&](int k, float (&a)[4], float (&w)[2][4]) {
+        if (INV) {
+#pragma unroll
+            for (int q = 0; q < 4; ++q) a[q] = Y[(size_t)(k + q) * D.npad + j0 + l];
+        } else {
+            const Quad v = *reinterpret_cast<const Quad*>(rrow + k);
+#pragma unroll
+            for (int q = 0; q < 4; ++q) a[q] = jin ? v.v[q] : 0.0f;
+        }
+#pragma unroll
+        for (int t = 0; t < 2; ++t) {
+            const Quad u = *reinterpret_cast<const Quad*>(col[t] + k);
+#pragma unroll
+            for (int q = 0; q < 4; ++q) w[t][q] = u.v[q];
+        }
+    };
+    auto mul16 = [&](const float (&a)[4], const float (&w)[2][4]) {
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+#pragma unroll
+            for (int t = 0; t < 2; ++t)
+                acc[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[q], w[t][q], acc[t], 0, 0, 0);
+    };
+    int k0 = wid * quarter;
+    // four loads of depth 16 in flight
+    for (; k0 + 64 <= kend; k0 += 64) {
+        float a[4][4], w[4][2][4];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) load16(k0 + 16 * u + 4 * g, a[u], w[u]);
+#pragma unroll
+        for (int u = 0; u < 4; ++u) mul16(a[u], w[u]);
+    }
+    for (; k0 + 16 <= kend; k0 += 16) {
+        float a[4], w[2][4];
+        load16(k0 + 4 * g, a, w);
+        mul16(a, w);
+    }
+    if (k0 < kend) {
+        // the sum's last few terms
+        float a[4], w[2][4];
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            const int k = k0 + 4 * g + q, kk = min(k, N - 1);
+            a[q] = k >= N ? 0.0f : INV ? Y[(size_t)kk * D.npad + j0 + l] : jin ? rrow[kk] : 0.0f;
+#pragma unroll
+            for (int t = 0; t < 2; ++t) w[t][q] = col[t][kk];
+        }
+        mul16(a, w);
+    }
+    if (wid > 0) {
+        part[wid - 1][0][lane] = acc[0];
+        part[wid - 1][1][lane] = acc[1];
+    }
+    __syncthreads();
+    if (wid > 0) return;
+#pragma unroll
+    for (int t = 0; t < 2; ++t) {
+#pragma unroll
+        for (int w = 0; w < 3; ++w) acc[t] += part[w][t][lane];
+        // lane (g, l) holds rows 4 g .. + 3 of column l
+        const int c = c0 + 16 * t + l;
+        if (c >= N) continue;
+        if (INV) {
+#pragma unroll
+            for (int q = 0; q < 4; ++q)
+                if (j0 + 4 * g + q < n) z[B.off + (size_t)(j0 + 4 * g + q) * N + c] = acc[t][q];
+        } else {
+            *reinterpret_cast<f32x4*>(Y + (size_t)c * D.npad + j0 + 4 * g) = acc[t];
+        }
+    }
+}
+
+// The theta line solves of the modes of one block (a segment of whole waves
+// each, kSpCells rows a thread; the rows past nth up to npad are empty), in
+// place in the spectral array, by the phi line solver with no coupling
+// around the ends. r.z is the same sum in the basis (Q is orthogonal), in
+// FP64 per block: rz_out slot g of the bubble, g the block; the slots past
+// the last block are cleared.
+__global__ void k_sp_line(const int4* __restrict__ items, const BubbleDev* __restrict__ bub,
+                          SolveCtl* __restrict__ ctl, SpPtrs P, int flags,
+                          double* __restrict__ rz_out, long stride) {
+    extern __shared__ __align__(16) unsigned char lds_raw[];
+    __shared__ double red[16];
+    __shared__ float redf[16];
+    constexpr int C = kSpCells;
+    const int4 it = items[blockIdx.x];
+    const int b = it.x;
+    SolveCtl* Cb = ctl + b;
+    if (flag_load(&Cb->outer_done)) return;
+    if ((flags & kMgGateInner) && Cb->inner_done) return;
+    const BubbleDev B = bub[b];
+    const SpDev D = P.d[b];
+    const int n = B.nth, npad = D.npad;
+    const RowSeg sg = row_seg<true>(npad / C);
+    const int m = it.y * sg.nseg + sg.seg;
+    const bool act = sg.seg < sg.nseg && m < B.nph && sg.lt < npad / C;
+    const int j0 = C * sg.lt;
+    float* __restrict__ y = P.Y + D.yoff + (size_t)min(m, B.nph - 1) * npad + j0;
+    float a[C], c[C], d[C], r[C];
+#pragma unroll
+    for (int q = 0; q < C; ++q) a[q] = c[q] = d[q] = r[q] = 0.0f;
+    if (act) {
+        const float lam = D.lam[m];
+        const float* __restrict__ cf = P.coef + B.pr0;
+        ld_row<C>(y, r);
+#pragma unroll
+        for (int q = 0; q < C; ++q) {
+            const int j = j0 + q;
+            if (j >= n) continue;
+            const float wn = cf[stride + j], ws = j + 1 < n ? cf[stride + j + 1] : 0.0f;
+            const float inv = pre_rcp(cf[2 * stride + j] + wn + ws + lam * cf[j]);
+            a[q] = -wn * inv;
+            c[q] = -ws * inv;
+            d[q] = r[q] * inv;
+        }
+    }
+    line_solve<float, C>(a, c, d, npad, 64, reinterpret_cast<float*>(lds_raw), redf, sg);
+    double acc[1] = {0.0};
+    if (act) {
+        st_row<C>(y, d);
+#pragma unroll
+        for (int q = 0; q < C; ++q) acc[0] += (double)r[q] * (double)d[q];
+    }
+    block_sum<1>(acc, red);
+    const int blocks = (B.nph + sg.nseg - 1) / sg.nseg;
+    for (int k = it.y + (int)threadIdx.x * blocks; k < n; k += (int)blockDim.x * blocks)
+        rz_out[B.pr0 + k] = k == it.y ? acc[0] : 0.0;
 }
 
 // ------------------------------------------- inner Chebyshev iteration ----
@@ -2427,6 +2695,34 @@ void launch_mg_line(hipStream_t s, const LaunchGeom& g, const BubbleDev* bub, So
                        stride)
     SF_CASES(SF_CALL)
 #undef SF_CALL
+}
+
+template <typename T>
+void launch_sp_coef(hipStream_t s, const LaunchGeom& g, const BubbleDev* bub, const Tables& tab,
+                    const T* gam, const float* wN, const float* wW, const SpPtrs& sp, long stride) {
+    hipLaunchKernelGGL(k_sp_coef<T>, dim3(g.nrows), dim3(256), 0, s, g.rows, bub, tab, gam, wN, wW,
+                       sp, stride);
+}
+template void launch_sp_coef<float>(hipStream_t, const LaunchGeom&, const BubbleDev*, const Tables&,
+                                    const float*, const float*, const float*, const SpPtrs&, long);
+void launch_sp_gemm(hipStream_t s, const int4* items, int nitems, const BubbleDev* bub,
+                    SolveCtl* ctl, const SpPtrs& P, const float* r, float* z, bool inverse,
+                    int flags, const SolveParams& sp, const double* partR, long stride) {
+    if (inverse)
+        hipLaunchKernelGGL(k_sp_gemm<true>, dim3(nitems), dim3(256), 0, s, items, bub, ctl, P, r, z,
+                           flags, sp, partR, stride);
+    else
+        hipLaunchKernelGGL(k_sp_gemm<false>, dim3(nitems), dim3(256), 0, s, items, bub, ctl, P, r, z,
+                           flags, sp, partR, stride);
+}
+void launch_sp_line(hipStream_t s, const int4* items, int nitems, int threads, size_t lds,
+                    const BubbleDev* bub, SolveCtl* ctl, const SpPtrs& P, int flags,
+                    double* rz_out, long stride) {
+    hipLaunchKernelGGL(k_sp_line, dim3(nitems), dim3(threads), lds, s, items, bub, ctl, P, flags,
+                       rz_out, stride);
+}
+void launch_sp_basis(hipStream_t s, int nph, const double* cosines, float* Qt, float* Q) {
+    hipLaunchKernelGGL(k_sp_basis, dim3(nph), dim3(256), 0, s, nph, cosines, Qt, Q);
 }
 
 void launch_finalize(hipStream_t s, int nb, const BubbleDev* bub, SolveCtl* ctl, SolveHist* hist,

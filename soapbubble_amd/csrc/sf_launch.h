@@ -96,6 +96,30 @@ struct MgPtrs {
 constexpr int kMgZeroNb = 1, kMgProlong = 2, kMgRestrict = 4, kMgRz = 8, kMgGateInner = 16,
               kMgGateStart = 32;
 
+// The spectral preconditioner (k_sp_coef, k_sp_gemm, k_sp_line). Per bubble:
+// the real Fourier basis of its row width (nph x nph, mode-major and
+// transposed), the eigenvalues of the phi difference, and its nph x npad block of the spectral
+// array (npad: the row count padded for the theta line solve).
+struct SpDev {
+    const float* Qt;
+    const float* Q;
+    const float* lam;
+    long long yoff;
+    int npad;
+    int pad_;
+};
+// The row-constant operator, per row (pr0 layout, `stride` apart): west and
+// north face weights, mass term, and the largest ratio of a cell's value to
+// its row's mean and of the mean to the value.
+struct SpPtrs {
+    const SpDev* d;
+    float* Y;
+    float* coef;
+};
+constexpr int kSpCells = 4;       // rows a thread of the theta line solve
+constexpr int kSpRows = 16, kSpCols = 32;   // output tile of k_sp_gemm
+constexpr int kSpMaxTheta = 2048; // the basis of a row is at most 4096 x 4096
+
 // Threads of a row block at most: one per C consecutive cells of the widest
 // row, C in {2, 4, 8, 16}.
 constexpr int kRowThreadsMax = 1024;
@@ -153,6 +177,21 @@ void launch_mg_line(hipStream_t s, const LaunchGeom& g, const BubbleDev* bub, So
                     MgPtrs<Ti> lvl, MgPtrs<Ti> coarse, const Ti* r0, int level, int flags,
                     const int* rsteps, const SolveParams& sp, const double* partR,
                     double* rz_out, long stride);
+// spectral preconditioner: the row-constant operator of a system; the
+// transform of r into the basis (`inverse`: of the spectral array into z);
+// the theta line solves of every mode, with the partials of r.z. Item lists:
+// rows as LaunchGeom::rows; (bubble, row tile, column tile); (bubble, block)
+template <typename T>
+void launch_sp_coef(hipStream_t s, const LaunchGeom& g, const BubbleDev* bub, const Tables& tab,
+                    const T* gam, const float* wN, const float* wW, const SpPtrs& sp, long stride);
+void launch_sp_gemm(hipStream_t s, const int4* items, int nitems, const BubbleDev* bub,
+                    SolveCtl* ctl, const SpPtrs& P, const float* r, float* z, bool inverse,
+                    int flags, const SolveParams& sp, const double* partR, long stride);
+void launch_sp_line(hipStream_t s, const int4* items, int nitems, int threads, size_t lds,
+                    const BubbleDev* bub, SolveCtl* ctl, const SpPtrs& P, int flags,
+                    double* rz_out, long stride);
+// the basis of rows of nph columns from the cosines cos(2 pi t / nph)
+void launch_sp_basis(hipStream_t s, int nph, const double* cosines, float* Qt, float* Q);
 void launch_finalize(hipStream_t s, int nb, const BubbleDev* bub, SolveCtl* ctl, SolveHist* hist,
                      const SolveParams& sp, const double* partR, long stride);
 void launch_sched_stats(hipStream_t s, SchedStat* d, SchedStat* h, int nb);
