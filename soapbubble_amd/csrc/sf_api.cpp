@@ -49,13 +49,38 @@ constexpr double kPi = 3.14159265358979323846;
 
 // A caller-provided device region that the set-up carves its arrays from
 // instead of allocating them (the entry point without allocation): a bump
-// pointer with 256-byte alignment, each array cleared on the caller's stream.
+// pointer with 256-byte alignment, the whole region cleared at the start.
+// What the set-up uploads is gathered in `image` (the region's first bytes:
+// descriptors, tables and lists come before the fields) and copied at once.
 struct Arena {
     char* base = nullptr;
     size_t size = 0, used = 0;
-    hipStream_t stream = nullptr;
+    std::vector<char> image;
 };
 thread_local Arena* g_arena = nullptr;
+
+// Copies set-up data to the device (finished when it returns, or, in an
+// arena, with the next h2d_flush).
+void h2d(void* dst, const void* src, size_t bytes) {
+    if (!g_arena) {
+        SF_HIP(hipMemcpy(dst, src, bytes, hipMemcpyHostToDevice));
+        return;
+    }
+    const size_t at = (size_t)(static_cast<char*>(dst) - g_arena->base);
+    if (g_arena->image.size() < at + bytes) g_arena->image.resize(at + bytes, 0);
+    std::memcpy(g_arena->image.data() + at, src, bytes);
+}
+template <typename X>
+void h2d(X* dst, const std::vector<X>& v) {
+    h2d((void*)dst, (const void*)v.data(), v.size() * sizeof(X));
+}
+// (before any kernel writes into the region's first bytes)
+void h2d_flush() {
+    if (!g_arena || g_arena->image.empty()) return;
+    SF_HIP(hipMemcpy(g_arena->base, g_arena->image.data(), g_arena->image.size(),
+                     hipMemcpyHostToDevice));
+    g_arena->image.clear();
+}
 
 struct ArenaScope {
     explicit ArenaScope(Arena* a) { g_arena = a; }
@@ -74,9 +99,6 @@ X* dalloc(size_t n, std::vector<void*>& owned) {
                                                  " MiB of the fixed device array"};
         p = g_arena->base + at;
         g_arena->used = at + bytes;
-        // cleared and finished before the set-up's synchronous copies write into it
-        SF_HIP(hipMemsetAsync(p, 0, bytes, g_arena->stream));
-        SF_HIP(hipStreamSynchronize(g_arena->stream));
         return static_cast<X*>(p);
     }
     hipError_t e = hipMalloc(&p, n * sizeof(X));
@@ -207,6 +229,7 @@ struct Base {
     // set up inside a caller's device array on the caller's stream: no
     // allocation, no stream, event, pinned buffer or graph of its own
     bool noalloc = false;
+    double t_start = 0.0;     // air-flow time the set-up gives the bubbles
     virtual ~Base() {
         if (stream) (void)hipStreamSynchronize(stream);
         for (auto& g : graphs) (void)hipGraphExecDestroy(g.second.exec);
@@ -1108,13 +1131,13 @@ void build_tables(Base& c, std::vector<void*>& owned) {
     }
     auto up64 = [&](const std::vector<double>& v) {
         double* d = dalloc<double>(v.size(), owned);
-        SF_HIP(hipMemcpy(d, v.data(), v.size() * sizeof(double), hipMemcpyHostToDevice));
+        h2d(d, v);
         return d;
     };
     auto up32 = [&](const std::vector<double>& v) {
         std::vector<float> f(v.begin(), v.end());
         float* d = dalloc<float>(f.size(), owned);
-        SF_HIP(hipMemcpy(d, f.data(), f.size() * sizeof(float), hipMemcpyHostToDevice));
+        h2d(d, f);
         return d;
     };
     Tables& t = c.tab;
@@ -1125,16 +1148,9 @@ void build_tables(Base& c, std::vector<void*>& owned) {
 }
 
 template <typename T, typename Ti>
-void upload_air_shapes(Impl<T, Ti>& c) {
-    for (int b = 0; b < c.nb; ++b) {
-        const BubbleDev& B = c.bub_h[b];
-        const size_t N = (size_t)B.nth * B.nph;
-        std::vector<double> su(N, 0.0), sv(N, 0.0);
-        sfh::air_shapes(B.nth, c.der[b].radius, c.der[b].U, su.data(), sv.data());
-        std::vector<T> tu(su.begin(), su.end()), tv(sv.begin(), sv.end());
-        SF_HIP(hipMemcpy(c.au + B.off, tu.data(), N * sizeof(T), hipMemcpyHostToDevice));
-        SF_HIP(hipMemcpy(c.av + B.off, tv.data(), N * sizeof(T), hipMemcpyHostToDevice));
-    }
+void form_air_shapes(Impl<T, Ti>& c) {
+    h2d_flush();
+    launch_air_shapes<T>(c.stream, c.geom, c.bub_d, c.au, c.av);
 }
 
 std::unique_ptr<Base> make_impl(int prec) {
@@ -1149,7 +1165,7 @@ std::unique_ptr<Base> make_impl(int prec) {
 template <typename T, typename Ti>
 void finish_setup(Impl<T, Ti>& c) {
     c.alloc_fields();
-    upload_air_shapes(c);
+    form_air_shapes(c);
     if (c.bimocq) c.alloc_bimocq();
     if (c.mg) c.alloc_mg();
 }
@@ -1184,7 +1200,7 @@ LaunchGeom pack_rows(Base& c, const std::vector<int>& ws, int C, size_t esz, siz
                                              " (use SF_PREC_MIXED for this size)"};
     items = xcd_order(items, make_int2(-1, 0), c.nxcd);
     int2* rows_d = dalloc<int2>(items.size(), c.owned);
-    SF_HIP(hipMemcpy(rows_d, items.data(), items.size() * sizeof(int2), hipMemcpyHostToDevice));
+    h2d(rows_d, items);
     LaunchGeom g = c.geom;
     g.rows = rows_d;
     g.nrows = (int)items.size();
@@ -1204,8 +1220,8 @@ void setup(Base& c, int prec) {
         SF_HIP(hipStreamCreateWithFlags(&c.stream, hipStreamNonBlocking));
         for (auto& e : c.ev) SF_HIP(hipEventCreate(&e));
     }
-    hipDeviceProp_t prop;
-    SF_HIP(hipGetDeviceProperties(&prop, c.device));
+    int lds_block = 0;
+    SF_HIP(hipDeviceGetAttribute(&lds_block, hipDeviceAttributeMaxSharedMemoryPerBlock, c.device));
 
     // bubble descriptors, offsets, row/column table bases
     long long off = 0;
@@ -1240,6 +1256,7 @@ void setup(Base& c, int prec) {
         B.re = c.der[b].re;
         B.invh32 = (float)B.invh;
         B.dt32 = (float)B.dt;
+        B.air_scale = c.der[b].radius / c.der[b].U;
         // every bubble starts on a 256-byte boundary (the row kernels load
         // C consecutive cells as one aligned vector)
         off += ((long long)B.nth * B.nph + 63) / 64 * 64;
@@ -1247,7 +1264,7 @@ void setup(Base& c, int prec) {
         ct += B.nph;
         pr += B.nth;
         nph_max = std::max(nph_max, B.nph);
-        c.time_h[b] = BubbleTime{0.0, d.dt * 1.0, c.opt.advance_time, 0, 0, 0, 0,
+        c.time_h[b] = BubbleTime{c.t_start, d.dt * 1.0, c.opt.advance_time, 0, 0, 0, 0,
                                  c.opt.halt_on_failure ? 1 : 0};
     }
     c.ncells = off;
@@ -1255,9 +1272,9 @@ void setup(Base& c, int prec) {
     c.stride = pr;
 
     c.bub_d = dalloc<BubbleDev>(nb, c.owned);
-    SF_HIP(hipMemcpy(c.bub_d, c.bub_h.data(), nb * sizeof(BubbleDev), hipMemcpyHostToDevice));
+    h2d(c.bub_d, c.bub_h);
     c.time_d = dalloc<BubbleTime>(nb, c.owned);
-    SF_HIP(hipMemcpy(c.time_d, c.time_h.data(), nb * sizeof(BubbleTime), hipMemcpyHostToDevice));
+    h2d(c.time_d, c.time_h);
     c.ctl_d = dalloc<SolveCtl>(nb, c.owned);
     c.hist_d = dalloc<SolveHist>(nb, c.owned);
     c.sstat_d = dalloc<SchedStat>(nb, c.owned);
@@ -1287,7 +1304,7 @@ void setup(Base& c, int prec) {
         }
         tiles = xcd_order(tiles, make_int4(-1, 0, 0, 1), nxcd);
         int4* tiles_d = dalloc<int4>(tiles.size(), c.owned);
-        SF_HIP(hipMemcpy(tiles_d, tiles.data(), tiles.size() * sizeof(int4), hipMemcpyHostToDevice));
+        h2d(tiles_d, tiles);
         return Base::TileSet{width, tiles_d, (int)tiles.size()};
     };
     c.tile_cands.clear();
@@ -1306,7 +1323,7 @@ void setup(Base& c, int prec) {
     // least 4 C cells for the reduced line system. Grouping the rows by
     // width keeps a narrow row from occupying a wide row's block.
     const size_t esz = c.fp64_inner() ? 8 : 4;
-    const size_t lds_limit = (size_t)prop.sharedMemPerBlock - 1024;
+    const size_t lds_limit = (size_t)lds_block - 1024;
     c.lds_limit = lds_limit;
     std::vector<int> widths;
     for (int b = 0; b < nb; ++b) widths.push_back(c.bub_h[b].nph);
@@ -1321,7 +1338,7 @@ void setup(Base& c, int prec) {
                 for (int j = 0; j < c.bub_h[b].nth; ++j) rows.push_back(make_int2(b, j));
         rows = xcd_order(rows, make_int2(-1, 0), nxcd);
         int2* rows_d = dalloc<int2>(rows.size(), c.owned);
-        SF_HIP(hipMemcpy(rows_d, rows.data(), rows.size() * sizeof(int2), hipMemcpyHostToDevice));
+        h2d(rows_d, rows);
         const int cpt = row_cpt(nph);
         if (cpt == 0)
             throw Status{SF_ERR_UNSUPPORTED, "rows of " + std::to_string(nph) + " cells are not supported"};
@@ -1402,7 +1419,7 @@ void setup(Base& c, int prec) {
             for (int j = 0; j < c.bub_h[b].nth; ++j) rows.push_back(make_int2(b, j));
         rows = xcd_order(rows, make_int2(-1, 0), nxcd);
         int2* rows_d = dalloc<int2>(rows.size(), c.owned);
-        SF_HIP(hipMemcpy(rows_d, rows.data(), rows.size() * sizeof(int2), hipMemcpyHostToDevice));
+        h2d(rows_d, rows);
         c.sgeo = c.geom;
         c.sgeo.rows = rows_d;
         c.sgeo.nrows = (int)rows.size();
@@ -1845,18 +1862,20 @@ int step_in_scratch(void* scratch, size_t bytes, const sf_options* opt,
         c.desc.assign(bubble, bubble + 1);
         c.noalloc = true;
         c.stream = stream;
+        c.t_start = t_seconds;
         {
             Arena a;
             a.base = static_cast<char*>(scratch);
             a.size = bytes;
-            a.stream = stream;
+            // cleared on the caller's stream and finished before the set-up's
+            // synchronous copies write into it
+            SF_HIP(hipMemsetAsync(scratch, 0, bytes, stream));
+            SF_HIP(hipStreamSynchronize(stream));
             ArenaScope scope(&a);
             setup(c, SF_PREC_MIXED);
         }
         const BubbleDev& B = c.bub_h[0];
         const size_t N = (size_t)B.nth * B.nph, Nt = N - B.nph;
-        c.time_h[0].t = t_seconds;
-        SF_HIP(hipMemcpy(c.time_d, c.time_h.data(), sizeof(BubbleTime), hipMemcpyHostToDevice));
         // the caller's state and air flow into the work arrays (the u_theta
         // array keeps its zero padding row)
         SF_HIP(hipMemcpyAsync(c.cur.uth, in[0], Nt * sizeof(float), hipMemcpyDeviceToDevice, stream));

@@ -22,6 +22,7 @@ struct BubbleDev {
     double M, Cr, gs, gamma_max, eva;
     double re;                   // Re^-1 of the VISCOUS path
     float invh32, dt32;          // 1/h and dt for the FP32 traces
+    double air_scale;            // radius / U: speed of the air corridor
     int gravity, evaporation, airflow, viscous;
 };
 

@@ -1,5 +1,5 @@
-// Host-only helpers: parameter derivation, air-flow corridor shape, seeded
-// synthetic initial fields and the OpenEXR thickness writer.
+// Host-only helpers: parameter derivation, seeded synthetic initial fields
+// and the OpenEXR thickness writer.
 #include "sf_host.h"
 
 #include <algorithm>
@@ -28,40 +28,6 @@ const double kNuA = 1.562e-5;
 const double kNu = 1.25e-4;   // soap solution kinematic viscosity, header.cuh:83
 const double kEvaporation = -0.00000003;  // header.cuh:95
 const double kPi = 3.14159265358979323846;
-const double kHalfPi = 1.57079632679489661923;
-
-struct V3 { double x, y, z; };
-V3 operator-(V3 a, V3 b) { return {a.x - b.x, a.y - b.y, a.z - b.z}; }
-V3 operator*(double s, V3 a) { return {a.x * s, a.y * s, a.z * s}; }
-V3 operator*(V3 a, double s) { return {a.x * s, a.y * s, a.z * s}; }
-double dot(V3 a, V3 b) { return a.x * b.x + a.y * b.y + a.z * b.z; }
-V3 cross(V3 a, V3 b) { return {a.y * b.z - a.z * b.y, a.z * b.x - a.x * b.z, a.x * b.y - a.y * b.x}; }
-V3 normalize(V3 v) { return v * (1.0 / std::sqrt(dot(v, v))); }
-
-// smoothstep of helper_math.h (float arithmetic)
-float smoothstepf(float a, float b, float x) {
-    float y = (x - a) / (b - a);
-    y = std::min(std::max(y, 0.0f), 1.0f);
-    return y * y * (3.0f - 2.0f * y);
-}
-
-// Corridor vector without its time factor: a great circle through the x
-// axis normal to the wind (0, cos(pi/2), sin(pi/2)), speed 0.5 sin(beta) r/U
-// faded out by smoothstep(0.2, 0.4, |beta - pi/2|).
-V3 corridor(double sinT, double cosT, double sinP, double cosP, double U, double radius) {
-    const double angle = kPi / 2.;
-    V3 wind = normalize(V3{0., std::cos(angle), std::sin(angle)});
-    V3 position{1., 0., 0.};
-    V3 normal = normalize(cross(position, wind));
-    V3 cur{sinT * cosP, sinT * sinP, cosT};
-    double c = std::max(-1.0, std::min(1.0, dot(normal, cur)));
-    double beta = std::acos(c);
-    V3 projected = normalize(cur - dot(normal, cur) * normal);
-    V3 pw = cross(normal, projected);
-    double ss = (double)smoothstepf(0.2f, 0.4f, (float)std::fabs(beta - kHalfPi));
-    V3 a = 0.5 * std::sin(beta) / U * radius * pw;
-    return a * (1. - ss);
-}
 
 // SplitMix64 (Steele, Lea, Flood 2014) seeding xoshiro256** (Blackman and
 // Vigna 2018).
@@ -165,31 +131,6 @@ void derive_params(const sf_bubble_desc& d, sf_derived& o) {
     o.eva = d.evaporation ? kEvaporation * d.radius / (d.H * 1.0) : 0.0;
     o.h = kPi / d.n_theta;
     o.re = kNu / (d.U * d.radius);   // re(nu / (U radius)) with the U argument
-}
-
-void air_shapes(int nth, double radius, double U, double* su, double* sv) {
-    const int nph = 2 * nth;
-    const double h = kPi / nth;
-    for (int j = 0; j < nth; ++j) {
-        const double th = ((double)j + 0.5) * h;
-        const double sT = std::sin(th), cT = std::cos(th);
-        for (int i = 0; i < nph; ++i) {
-            const double ph = ((double)i - 0.5) * h;
-            const double sP = std::sin(ph), cP = std::cos(ph);
-            V3 a = corridor(sT, cT, sP, cP, U, radius);
-            su[(size_t)j * nph + i] = dot(a, V3{-sP, cP, 0.});
-        }
-    }
-    for (int j = 0; j < nth - 1; ++j) {
-        const double th = ((double)j + 1.0) * h;
-        const double sT = std::sin(th), cT = std::cos(th);
-        for (int i = 0; i < nph; ++i) {
-            const double ph = (double)i * h;
-            const double sP = std::sin(ph), cP = std::cos(ph);
-            V3 a = corridor(sT, cT, sP, cP, U, radius);
-            sv[(size_t)j * nph + i] = dot(a, V3{cT * cP, cT * sP, -sT});
-        }
-    }
 }
 
 double real_ylm(int l, int m, double theta, double phi) {

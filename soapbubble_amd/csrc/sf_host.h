@@ -12,13 +12,6 @@ namespace sfh {
 // 2627-2638).
 void derive_params(const sf_bubble_desc& d, sf_derived& o);
 
-// Time-independent part of the air-flow corridor of airFlowU / airFlowV
-// (bubble.cu:2317-2335, 2358-2375) projected on e_phi at u_phi faces (su,
-// nth*nph) and on e_theta at u_theta faces (sv, rows 0..nth-2); the kernels
-// multiply it by 3 - |t - 3|. NaN marks points where the reference's
-// normalisation divides by zero.
-void air_shapes(int nth, double radius, double U, double* su, double* sv);
-
 // Real spherical harmonic, orthonormal on the unit sphere.
 double real_ylm(int l, int m, double theta, double phi);
 

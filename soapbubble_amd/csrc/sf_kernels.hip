@@ -158,8 +158,8 @@ __global__ __launch_bounds__(256) void k_advect(const int4* __restrict__ tiles,
 
 // ---------------------------------------------------------- air flow ----
 // u_air(t) = u_air_init + (3 - |t - 3|) * corridor, NaN -> 0 (airFlowU/V,
-// bubble.cu:2301-2380). The corridor shape is time-independent and is
-// precomputed on the host.
+// bubble.cu:2301-2380). The corridor shape is time-independent: formed once
+// per context (k_air_shapes).
 // FP32 fields (the mixed paths) evaluate it in FP32, as the reference's
 // float kernels do; FP64 fields in FP64.
 template <typename T>
@@ -180,6 +180,58 @@ __device__ __forceinline__ double air_at(const T* __restrict__ a0, const T* __re
 }
 
 
+
+// The corridor vector without its time factor at (theta, phi): a great circle
+// through the x axis normal to the wind (0, cos(pi/2), sin(pi/2)), speed 0.5
+// sin(beta) r/U faded out by smoothstep(0.2, 0.4, |beta - pi/2|) (helper_math.h's,
+// in float arithmetic), beta the angle from the circle's normal.
+__device__ __forceinline__ void corridor(double sT, double cT, double sP, double cP, double scale,
+                                         double& ax, double& ay, double& az) {
+    const double pi = 3.14159265358979323846;
+    // position (1, 0, 0) x wind, normalised (cos(pi/2) is not quite zero)
+    const double wy = 6.123233995736766e-17, wz = 1.0, wl = 1.0 / sqrt(wy * wy + wz * wz);
+    const double ny = -wz * wl, nz = wy * wl;
+    const double x = sT * cP, y = sT * sP, z = cT;
+    const double c = fmax(-1.0, fmin(1.0, ny * y + nz * z));
+    const double beta = acos(c);
+    double px = x, py = y - c * ny, pz = z - c * nz;
+    const double pl = 1.0 / sqrt(px * px + py * py + pz * pz);
+    px *= pl; py *= pl; pz *= pl;
+    float f = ((float)fabs(beta - pi / 2) - 0.2f) / (0.4f - 0.2f);
+    f = fminf(fmaxf(f, 0.0f), 1.0f);
+    const double s = 0.5 * sin(beta) * scale * (1.0 - (double)(f * f * (3.0f - 2.0f * f)));
+    // normal x projected
+    ax = s * (ny * pz - nz * py);
+    ay = s * (nz * px);
+    az = s * (-ny * px);
+}
+
+// Its e_phi component on the u_phi faces (au) and e_theta component on the
+// u_theta faces (av) of every bubble. On the host the same took 35 ns a value,
+// most of a context's set-up time.
+template <typename T>
+__global__ __launch_bounds__(256) void k_air_shapes(const int4* __restrict__ tiles,
+                                                    const BubbleDev* __restrict__ bub,
+                                                    T* __restrict__ au, T* __restrict__ av) {
+    const int4 tl = tiles[blockIdx.x];
+    if (tl.x < 0) return;
+    const BubbleDev B = bub[tl.x];
+    int j, i;
+    tile_cell(tl, j, i);
+    if (j >= B.nth || i >= B.nph) return;
+    const size_t c = (size_t)B.off + (size_t)j * B.nph + i;
+    double sT, cT, sP, cP, x, y, z;
+    sincos((j + 0.5) * B.h, &sT, &cT);
+    sincos((i - 0.5) * B.h, &sP, &cP);
+    corridor(sT, cT, sP, cP, B.air_scale, x, y, z);
+    au[c] = (T)(cP * y - sP * x);
+    if (j < B.nth - 1) {
+        sincos((j + 1.0) * B.h, &sT, &cT);
+        sincos(i * B.h, &sP, &cP);
+        corridor(sT, cT, sP, cP, B.air_scale, x, y, z);
+        av[c] = (T)(cT * cP * x + cT * sP * y - sT * z);
+    }
+}
 
 // ----------------------------------------------------------- VISCOUS ----
 // The VISCOUS stress path (header.cuh:99; off in the reference): div(u) at
@@ -2665,6 +2717,16 @@ void launch_cheb(hipStream_t s, const LaunchGeom& g, const BubbleDev* bub, Solve
 #undef SF_CALL
 #undef SF_CALL1
 }
+
+template <typename T>
+void launch_air_shapes(hipStream_t s, const LaunchGeom& g, const BubbleDev* bub,
+                       T* au, T* av) {
+    hipLaunchKernelGGL(k_air_shapes<T>, dim3(g.ntiles), dim3(256), 0, s, g.tiles, bub, au, av);
+}
+template void launch_air_shapes<float>(hipStream_t, const LaunchGeom&, const BubbleDev*,
+                                       float*, float*);
+template void launch_air_shapes<double>(hipStream_t, const LaunchGeom&, const BubbleDev*,
+                                        double*, double*);
 
 template <typename T>
 void launch_viscous(hipStream_t s, const LaunchGeom& g, const BubbleDev* bub, const Tables& tab,

@@ -162,6 +162,10 @@ template <typename Ti>
 void launch_cheb(hipStream_t s, const LaunchGeom& g, const BubbleDev* bub, SolveCtl* ctl,
                  SysPtrs<Ti> sys, const Ti* ek, const Ti* ekm1, Ti* enext, int it, int kr,
                  const SolveParams& sp, double* partB, long stride);
+// the air corridor's shapes (k_air_shapes)
+template <typename T>
+void launch_air_shapes(hipStream_t s, const LaunchGeom& g, const BubbleDev* bub,
+                       T* au, T* av);
 // VISCOUS: div(u) at the centres, then fu, fv (cell layout)
 template <typename T>
 void launch_viscous(hipStream_t s, const LaunchGeom& g, const BubbleDev* bub, const Tables& tab,
