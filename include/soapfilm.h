@@ -220,10 +220,12 @@ int sf_synchronize(sf_ctx* ctx);
  * (u_theta (nTheta-1) x nPhi, the others nTheta x nPhi; uair0 / vair0 the
  * air flow at t = 0, as SF_FIELD_UAIR0 / SF_FIELD_VAIR0); outputs may alias
  * the inputs. opt->precision must be SF_PREC_MIXED and scalar_advection 0;
- * the solve runs a fixed schedule of opt->max_outer refinements (0: 2) of
+ * the solve runs a schedule of opt->max_outer refinements (0: 2) of
  * opt->max_inner inner iterations (0: 16) plus one spare refinement, and a
- * bubble that has converged skips the rest; solves that miss the tolerance
- * are counted in stats->failed_solves (stats may be NULL). t_seconds is the
+ * bubble that has converged skips the rest (with both 0, after a first
+ * refinement as long as the step before suggests; the rest is launched only
+ * if that one misses the tolerance); solves that miss the tolerance are
+ * counted in stats->failed_solves (stats may be NULL). t_seconds is the
  * air-flow time at the first step. Work is queued on `stream` (a
  * hipStream_t; NULL: the default stream) after what the caller queued there;
  * the call returns when it has finished. The array is shared by every call

@@ -836,6 +836,39 @@ struct Impl : Base {
         return true;
     }
 
+    // Refinement k of the fixed Chebyshev schedule. A refinement of no inner
+    // iteration (only ever the last one) takes z = M^-1 r of the residual
+    // before as its correction; its residual launch forms that z itself (on
+    // its rows and one row either side), so the residual launch before it
+    // solves no line system: the spare refinement usually finds the tolerance
+    // met and returns at once.
+    void cheb_refinement(size_t k) {
+        for (int it = 1; it <= sched[k]; ++it) cheb(it, (int)k);
+        const bool zp = sched[k] == 0 && k > 0;
+        const bool zp_next = k + 2 == sched.size() && sched[k + 1] == 0;
+        resid((int)k + 1, zp ? nullptr : cheb_e(sched[k] + 1), sstat_d,
+              k + 1 == sched.size() || zp_next, zp);
+    }
+    // The residual norms of a one-bubble context before and after its first
+    // refinement (one copy: the slots are neighbours), as the tolerance
+    // takes them.
+    void first_refinement(double& before, double& after) {
+        const size_t w = (size_t)kAccVals * kAccSub;
+        slot_h.resize(2 * w);
+        SF_HIP(hipMemcpyAsync(slot_h.data(), acc, 2 * w * sizeof(double), hipMemcpyDeviceToHost,
+                              stream));
+        SF_HIP(hipStreamSynchronize(stream));
+        double v[3] = {0.0, 0.0, 0.0};
+        for (int q = 0; q < kAccSub; ++q) {
+            v[0] += slot_h[q];
+            v[1] += slot_h[w + q];
+            v[2] += slot_h[kAccSub + q];
+        }
+        const double bb = sp.absolute ? 1.0 : (v[2] > 0.0 ? std::sqrt(v[2]) : 1.0);
+        before = std::sqrt(v[0]) / bb;
+        after = std::sqrt(v[1]) / bb;
+    }
+
     // Refinement loop after the assembly. Host-driven: convergence flags are
     // read back after each residual and every four inner iterations (the
     // plain path, and the calibration steps of the graph schedule). Fixed:
@@ -900,19 +933,7 @@ struct Impl : Base {
                 }
 
             } else {
-                // a refinement of no inner iteration (only ever the last one)
-                // takes z = M^-1 r of the residual before as its correction;
-                // its residual launch forms that z itself (on its rows and
-                // one row either side), so the residual launch before it
-                // solves no line system: the spare refinement usually finds
-                // the tolerance met and returns at once
-                for (size_t k = 0; k < sched.size(); ++k) {
-                    for (int it = 1; it <= sched[k]; ++it) cheb(it, (int)k);
-                    const bool zp = sched[k] == 0 && k > 0;
-                    const bool zp_next = k + 2 == sched.size() && sched[k + 1] == 0;
-                    resid((int)k + 1, zp ? nullptr : cheb_e(sched[k] + 1), sstat_d,
-                          k + 1 == sched.size() || zp_next, zp);
-                }
+                for (size_t k = 0; k < sched.size(); ++k) cheb_refinement(k);
             }
         } else if (host_driven) {
             std::vector<SolveCtl> c(nb);
@@ -1885,18 +1906,40 @@ int step_in_scratch(void* scratch, size_t bytes, const sf_options* opt,
         SF_HIP(hipMemcpyAsync(c.ua0, uair0, N * sizeof(float), hipMemcpyDeviceToDevice, stream));
         SF_HIP(hipMemcpyAsync(c.va0, vair0, Nt * sizeof(float), hipMemcpyDeviceToDevice, stream));
         launch_nan_scan<float>(stream, c.geom, c.bub_d, c.time_d, c.cur);
-        // a fixed schedule (no host round trip inside the steps): max_outer
-        // refinements of max_inner inner iterations, then the spare
-        // refinement whose correction is the last line solve; a bubble that
-        // has converged skips the remaining kernels
+        // The schedule of a step: max_outer refinements of max_inner inner
+        // iterations, then the spare refinement whose correction is the last
+        // line solve. Launches cost the host more (7 us) than small kernels
+        // run, also the ones that find their bubble converged, so with the
+        // automatic schedule a first refinement of as many iterations as the
+        // residual's fall in the step before asks for comes in front, and
+        // the rest is launched only if its residual, read back (15 us),
+        // misses the tolerance: 8 launches a step instead of 36.
+        const bool automatic = opt->max_inner <= 0 && opt->max_outer <= 0 && c.method == 2;
         const int K = opt->max_inner > 0 ? opt->max_inner : 16;
         const int R = opt->max_outer > 0 ? std::min(opt->max_outer, kAccRefine - 1) : 2;
-        c.sched.assign((size_t)R, K);
-        c.sched.push_back(0);
+        std::vector<int> full((size_t)R, K);
+        full.push_back(0);
+        int first = std::min(6, K);
         for (int k = 0; k < nsteps; ++k) {
             c.advect();
             c.assemble();
-            c.solve(false, false);
+            c.sched = full;
+            if (!automatic) {
+                c.solve(false, false);
+            } else {
+                c.sched.insert(c.sched.begin(), first);
+                c.cheb_refinement(0);
+                double r0, r1;
+                c.first_refinement(r0, r1);
+                // (a hair inside the tolerance: the device sums in another order)
+                if (!(r1 <= c.sp.tol * (1.0 - 1e-9)))
+                    for (size_t q = 1; q < c.sched.size(); ++q) c.cheb_refinement(q);
+                // the next step's: a quarter of the tolerance at this step's
+                // fall per line solve, of which the assembly makes one
+                const double fall = std::log(r1 / r0) / (first + 1);
+                const double n = fall < 0.0 ? std::log(0.25 * c.sp.tol / r0) / fall : (double)K;
+                first = n >= 1.0 && n < (double)K ? std::max((int)std::ceil(n) - 1, 1) : n < 1.0 ? 1 : K;
+            }
             c.update(true);
         }
         c.steps_done = nsteps;
