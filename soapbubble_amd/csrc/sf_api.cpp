@@ -677,8 +677,8 @@ struct Impl : Base {
         double** arrays[] = {&bm.e_init,
                              &bm.e_initlast, &bm.e_delta, &bm.e_deltalast, &bm.g_init,
                              &bm.g_initlast, &bm.g_delta, &bm.g_deltalast, &bm.chg_e, &bm.chg_g,
-                             &bm.err_e, &bm.err_g, &bm.cpy_e, &bm.cpy_g};
-        for (double** a : arrays) *a = dalloc<double>(n, owned);
+                             &bm.err_e, &bm.err_g, &bm.cpy_e, &bm.cpy_g, &bm.e_last, &bm.e_mix};
+        for (double** a : arrays) *a = dalloc<double>(n + kFieldPad, owned);
         bm.tab = tab;
         bm.bt = time_d;
         bm.dist_bits = dalloc<unsigned>((size_t)nb, owned);

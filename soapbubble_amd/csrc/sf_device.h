@@ -786,7 +786,7 @@ struct P2d {
 // centre's index coordinates (j + 1/2, i) plus the angles turned from it,
 // each the asin of a sine that the (sin, cos) pair of the meridian half-plane
 // (a unit vector) or the equatorial plane (scale rho) gives, by its series
-// below 0.02 (truncation under 1e-22 rad); farther points take acos and
+// below 1/4; farther points take acos and
 // atan2. The same angles up to rounding, phi in the centre's period rather
 // than atan2's (-pi, pi] (the samplers wrap phi either way).
 struct CellRef {
@@ -796,19 +796,34 @@ __device__ __forceinline__ CellRef cell_ref(const Tables& tab, const BubbleDev& 
     return CellRef{j + 0.5, (double)i, tab.sinTc[B.rt0 + j], tab.cosTc[B.rt0 + j],
                    tab.sinPc[B.ct0 + i], tab.cosPc[B.ct0 + i]};
 }
+// asin(s) for |s| < kAsinWide by its odd series (truncated at 2e-18)
+constexpr double kAsinWide = 0.25;
+__device__ __forceinline__ double asin_wide(double s) {
+    const double y = s * s;
+    double p = 676039.0 / 104857600.0;
+    p = fma(p, y, 88179.0 / 12058624.0);
+    p = fma(p, y, 46189.0 / 5505024.0);
+    p = fma(p, y, 12155.0 / 1245184.0);
+    p = fma(p, y, 6435.0 / 557056.0);
+    p = fma(p, y, 143.0 / 10240.0);
+    p = fma(p, y, 231.0 / 13312.0);
+    p = fma(p, y, 63.0 / 2816.0);
+    p = fma(p, y, 35.0 / 1152.0);
+    p = fma(p, y, 5.0 / 112.0);
+    p = fma(p, y, 3.0 / 40.0);
+    p = fma(p, y, 1.0 / 6.0);
+    return s * fma(p, y, 1.0);
+}
 __device__ __forceinline__ P2d index_near(double invh, const U3& r, const CellRef& o) {
-    const double rho = sqrt(r.x * r.x + r.y * r.y);
+    const double r2 = r.x * r.x + r.y * r.y;
+    const double ir = inv_root(r2), rho = r2 * ir;
     const double nt = rho * o.cT - r.z * o.sT, ct = r.z * o.cT + rho * o.sT;
-    const double np = r.y * o.cP - r.x * o.sP, cp = r.x * o.cP + r.y * o.sP;
+    const double np = (r.y * o.cP - r.x * o.sP) * ir, cp = r.x * o.cP + r.y * o.sP;
     P2d q;
-    if (ct > 0.0 && fabs(nt) < 0.02) {
-        q.x = o.gx + asin_small(nt) * invh;
-    } else {
+    q.x = o.gx + asin_wide(nt) * invh;
+    q.y = o.gy + asin_wide(np) * invh;
+    if (!(ct > 0.0 && fabs(nt) < kAsinWide && cp > 0.0 && fabs(np) < kAsinWide)) {
         q.x = safe_acos_d(r.z) * invh;
-    }
-    if (cp > 0.0 && fabs(np) < 0.02 * rho) {
-        q.y = o.gy + asin_small(np * rcp64(rho)) * invh;
-    } else {
         q.y = atan2(r.y, r.x) * invh;
     }
     return q;
@@ -898,6 +913,121 @@ __device__ __forceinline__ U3 sample_map_u(const UMap& M, size_t off, int nth, i
         hl = at(tI + 1, pI); hr = at(tI + 1, pI + 1);
     }
     return slerp_u(slerp_u(ll, lr, aP), slerp_u(hl, hr, aP), aT);
+}
+
+// The same interpolations where every pair is near (|t - f|^2 below
+// kNearD2, grids of about 50 rows and more), for rows of any length; a row
+// past a pole is the first or last one at phi + pi. The coefficients of the end a fraction
+// beta away, sin(beta theta) / sin theta = beta (1 + u p1 + u^2 p2 + ...), u
+// = theta^2, are polynomials in beta^2: formed once for the two
+// interpolations along phi, and constants for the fixed sample points. One
+// more term of each series than slerp_u's (truncated below 1e-16 at kNearD2).
+constexpr double kNearD2 = 4e-3;
+struct SlerpEnd {
+    double k, p1, p2, p3, p4;
+};
+__device__ __forceinline__ constexpr SlerpEnd slerp_end(double beta) {
+    const double b = beta * beta, q = 1.0 - b;
+    return SlerpEnd{beta, q * (1.0 / 6), q * (7.0 / 360 - b * (1.0 / 120)),
+                    q * (31.0 / 15120 + b * (-1.0 / 840 + b * (1.0 / 5040))),
+                    q * (127.0 / 604800 + b * (-239.0 / 1814400 + b * (11.0 / 362880 - b / 362880)))};
+}
+__device__ __forceinline__ double slerp_weight(const SlerpEnd& e, double u) {
+    return e.k * fma(u, fma(u, fma(u, fma(u, e.p4, e.p3), e.p2), e.p1), 1.0);
+}
+// `near` stays set while the pairs are near.
+__device__ __forceinline__ U3 slerp_near(const U3& f, const U3& t, const SlerpEnd& ef,
+                                         const SlerpEnd& et, bool& near) {
+    const double dx = t.x - f.x, dy = t.y - f.y, dz = t.z - f.z;
+    const double d2 = fma(dx, dx, fma(dy, dy, dz * dz));
+    near = near && d2 < kNearD2;
+    const double u =
+        d2 * fma(d2, fma(d2, fma(d2, fma(d2, 1.0 / 3150, 1.0 / 560), 1.0 / 90), 1.0 / 12), 1.0);
+    const double a = slerp_weight(ef, u), b = slerp_weight(et, u);
+    return U3{fma(a, f.x, b * t.x), fma(a, f.y, b * t.y), fma(a, f.z, b * t.z)};
+}
+__device__ __forceinline__ U3 map_at(const UMap& M, size_t c) { return U3{M.x[c], M.y[c], M.z[c]}; }
+
+// Row r (-1 .. nth) of a map: its first cell, and the columns to add.
+__device__ __forceinline__ size_t map_row(const BubbleDev& B, size_t off, int r, int& shift) {
+    shift = r < 0 || r >= B.nth ? B.nth : 0;
+    return off + (size_t)min(max(r, 0), B.nth - 1) * B.nph;
+}
+// c in [0, 2 nph) wrapped into the row
+__device__ __forceinline__ int fold_col(const BubbleDev& B, int c) {
+    return c >= B.nph ? c - B.nph : c;
+}
+
+// sampleMapping at an index position (x, y); clears `near` where the general
+// form is needed (its value is then meaningless).
+__device__ __forceinline__ U3 sample_map_near(const UMap& M, size_t off, const BubbleDev& B, double rx,
+                                              double ry, bool& near) {
+    int tI, pI;
+    double aT, aP;
+    split_floor(rx - 0.5, tI, aT);
+    split_floor(ry, pI, aP);
+    near = near && tI >= -1 && tI < B.nth;
+    tI = min(max(tI, -1), B.nth - 1);
+    int sl, sh;
+    const size_t r0 = map_row(B, off, tI, sl), r1 = map_row(B, off, tI + 1, sh);
+    const int c = wrap_col(pI, B.nph, B.mask);
+    const SlerpEnd f = slerp_end(1.0 - aP), t = slerp_end(aP);
+    const U3 lo = slerp_near(map_at(M, r0 + fold_col(B, c + sl)),
+                             map_at(M, r0 + fold_col(B, fold_col(B, c + 1) + sl)), f, t, near);
+    const U3 hi = slerp_near(map_at(M, r1 + fold_col(B, c + sh)),
+                             map_at(M, r1 + fold_col(B, fold_col(B, c + 1) + sh)), f, t, near);
+    return slerp_near(lo, hi, slerp_end(1.0 - aT), slerp_end(aT), near);
+}
+
+// sampleMapping at the four quarter points around the centre of cell (j, i),
+// in kMsDx / kMsDy order, and the centre itself (the map's own value): six
+// interpolations along phi in three rows and four along theta, where five
+// separate lookups make fifteen.
+struct Around {
+    U3 nw, sw, ne, se, mid;
+};
+__device__ __forceinline__ void sample_map_around(const UMap& M, size_t off, const BubbleDev& B, int j,
+                                                  int i, Around& out, bool& near) {
+    const int iw = i == 0 ? B.nph - 1 : i - 1, ie = i + 1 == B.nph ? 0 : i + 1;
+    constexpr SlerpEnd q1 = slerp_end(0.25), q3 = slerp_end(0.75);
+    U3 w[3], e[3];
+#pragma unroll
+    for (int r = 0; r < 3; ++r) {
+        int sh;
+        const size_t row = map_row(B, off, j - 1 + r, sh);
+        const U3 c = map_at(M, row + fold_col(B, i + sh));
+        w[r] = slerp_near(map_at(M, row + fold_col(B, iw + sh)), c, q1, q3, near);
+        e[r] = slerp_near(c, map_at(M, row + fold_col(B, ie + sh)), q3, q1, near);
+        if (r == 1) out.mid = c;
+    }
+    out.nw = slerp_near(w[0], w[1], q1, q3, near);
+    out.sw = slerp_near(w[1], w[2], q3, q1, near);
+    out.ne = slerp_near(e[0], e[1], q1, q3, near);
+    out.se = slerp_near(e[1], e[2], q3, q1, near);
+}
+// the sample of kMsDx / kMsDy's number q (uniform)
+__device__ __forceinline__ U3 pick(const Around& v, int q) {
+    // (values, not references: the five stay in registers)
+    auto sel = [q](double a, double b, double c, double d, double e) {
+        return q == 0 ? +a : q == 1 ? +b : q == 2 ? +c : q == 3 ? +d : +e;
+    };
+    return U3{sel(v.nw.x, v.sw.x, v.ne.x, v.se.x, v.mid.x), sel(v.nw.y, v.sw.y, v.ne.y, v.se.y, v.mid.y),
+              sel(v.nw.z, v.sw.z, v.ne.z, v.se.z, v.mid.z)};
+}
+
+// sampleCentered of a field without NaNs at an index position of a map.
+__device__ __forceinline__ Corner<double> corner_of(const BubbleDev& B, const P2d& p) {
+    Corner<double> q;
+    split_floor(p.x - 0.5, q.t, q.aT);
+    split_floor(p.y, q.c, q.aP);
+    q.c = wrap_col(q.c, B.nph, B.mask);
+    return q;
+}
+__device__ __forceinline__ double sample_corner(const double* f, const BubbleDev& B,
+                                                const Corner<double>& q) {
+    const auto r = field_rsrc(f, B.nth * B.nph);
+    if (inside(q, B.nth)) return corner_bilerp(r, q, B.nph);
+    return pole_bilerp<1, false, double, false>(r, q, B.nth, B.nph, B.mask);
 }
 
 // MULTISAMPLE (header.cuh:98): five samples around a point with these

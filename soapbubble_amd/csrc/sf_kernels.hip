@@ -2260,7 +2260,12 @@ __global__ void k_row_stats(const int2* __restrict__ rows, const BubbleDev* __re
 // error-corrected reinitialisation when the maps drift apart
 // (bubble.cu:2509-2564). Gamma keeps the plain advection ("do not apply
 // bimocq on concentration for stability", bubble.cu:1195) but carries its
-// init/changes for the correction. One thread per cell, packed tiles.
+// init/changes for the correction. One thread per cell, packed tiles. Bound by
+// FP64 vector issue and, with it, by registers: the three kernels of every
+// step are held to three waves a SIMD (168 registers; two waves unbound, and
+// four spill: 275, 259 and 282 us a 512x1024 step). A step with them: 512x1024
+// 387 -> 259 us, 1024x2048 1351 -> 905 us, 1000x2000 1715 -> 955 us against
+// separate map lookups, 25 field samples and library arc functions per cell.
 
 // initMapping (solver.cu:12-22) and Init/InitLast = current, changes = 0
 __device__ __forceinline__ void set_identity(const UMap& M, size_t c, double h, int j, int i) {
@@ -2287,6 +2292,8 @@ __global__ __launch_bounds__(256) void k_bm_init(const int4* __restrict__ tiles,
     P.e_init[c] = P.e_initlast[c] = (double)cur.eta[c];
     P.g_init[c] = P.g_initlast[c] = (double)cur.gam[c];
     P.e_delta[c] = P.e_deltalast[c] = P.g_delta[c] = P.g_deltalast[c] = 0.0;
+    P.e_last[c] = P.e_init[c];
+    P.e_mix[c] = P.blend * P.e_init[c];
 }
 
 // traceGreatCircle from the cell centre (j + 1/2, i) over dt (either sign)
@@ -2319,7 +2326,10 @@ __device__ __forceinline__ void bm_maps_cell(const BubbleDev& B, const Tables& t
         double tx, ty;
         trace_centre<T, NANS>(uth, uph, tab, B, dir == 0 ? -TabSel<T>::dt(B) : TabSel<T>::dt(B),
                               j, i, tx, ty);
-        const U3 s = sample_map_u(dir == 0 ? P.fwd : P.bwd, o, B.nth, B.nph, tx, ty);
+        const UMap& from = dir == 0 ? P.fwd : P.bwd;
+        bool near = true;
+        U3 s = sample_map_near(from, o, B, tx, ty, near);
+        if (!near) s = sample_map_u(from, o, B.nth, B.nph, tx, ty);
         const UMap& out = dir == 0 ? P.nfwd : P.nbwd;
         out.x[c] = s.x;
         out.y[c] = s.y;
@@ -2328,7 +2338,7 @@ __device__ __forceinline__ void bm_maps_cell(const BubbleDev& B, const Tables& t
 }
 
 template <typename T>
-__global__ __launch_bounds__(256) void k_bm_maps(const int4* __restrict__ tiles,
+__global__ __launch_bounds__(256, 3) void k_bm_maps(const int4* __restrict__ tiles,
                                                  const BubbleDev* __restrict__ bub,
                                                  const BubbleTime* __restrict__ btime, Tables tab,
                                                  StatePtrs<T> cur, BimocqPtrs P) {
@@ -2346,7 +2356,7 @@ __global__ __launch_bounds__(256) void k_bm_maps(const int4* __restrict__ tiles,
 
 // advectionCenteredBimocq (bubble.cu:967-1013) through the new backward map
 // and the previous interval's backward map; overwrites the plain eta*.
-template <typename T, bool NANS>
+template <typename T>
 __device__ __forceinline__ void bm_eta_cell(const BubbleDev& B, StatePtrs<T> cur, StatePtrs<T> out,
                                             const BimocqPtrs& P, int j, int i) {
     const size_t o = (size_t)B.off, c = o + (size_t)j * B.nph + i;
@@ -2361,26 +2371,55 @@ __device__ __forceinline__ void bm_eta_cell(const BubbleDev& B, StatePtrs<T> cur
     const double bl = P.blend;
     const CellRef cr = cell_ref(P.tab, B, j, i);
     double a = 0.0;
+#pragma unroll 1
     for (int s = 0; s < ns; ++s) {
         const int q = ns == 5 ? s : 4;
         const double w = ns == 5 ? kMsW[q] : 1.0;
         const P2d ip = index_near(B.invh, sample_map_u(P.nbwd, o, B.nth, B.nph,
                                                         j + 0.5 + kMsDx[q], i + kMsDy[q]), cr);
         const P2d lp = index_near(B.invh, sample_map_u(P.prev, o, B.nth, B.nph, ip.x, ip.y), cr);
+        const double d = sample_centered<double, true>(fd, B.nth, ip.x, ip.y);
         a += (1.0 - bl) * w *
-             (sample_centered<double, NANS>(fil, B.nth, lp.x, lp.y) +
-              sample_centered<double, NANS>(fd, B.nth, ip.x, ip.y) +
-              sample_centered<double, NANS>(fdl, B.nth, lp.x, lp.y));
-        a += bl * w * (sample_centered<double, NANS>(fin, B.nth, ip.x, ip.y) +
-                       sample_centered<double, NANS>(fd, B.nth, ip.x, ip.y));
+             (sample_centered<double, true>(fil, B.nth, lp.x, lp.y) + d +
+              sample_centered<double, true>(fdl, B.nth, lp.x, lp.y));
+        a += bl * w * (sample_centered<double, true>(fin, B.nth, ip.x, ip.y) + d);
     }
     out.eta[c] = (T)fmax(kThresh, a);
+}
+
+// The same without NaNs and where the maps are smooth: the samples are of the two sums the formula above adds up, one each at ip
+// and lp (10 bilinear samples instead of 25). False: not the case here,
+// nothing written.
+template <typename T>
+__device__ __forceinline__ bool bm_eta_near(const BubbleDev& B, StatePtrs<T> cur, StatePtrs<T> out,
+                                            const BimocqPtrs& P, int j, int i) {
+    const size_t o = (size_t)B.off, c = o + (size_t)j * B.nph + i;
+    bool near = true;
+    double a = 0.0;
+    const CellRef cr = cell_ref(P.tab, B, j, i);
+    Around at{};
+    if (P.multisample) {
+        sample_map_around(P.nbwd, o, B, j, i, at, near);
+    } else {
+        at.mid = map_at(P.nbwd, c);
+    }
+#pragma unroll 1
+    for (int q = P.multisample ? 0 : 4; q < 5; ++q) {
+        const P2d ip = index_near(B.invh, pick(at, q), cr);
+        const P2d lp = index_near(B.invh, sample_map_near(P.prev, o, B, ip.x, ip.y, near), cr);
+        const double w = P.multisample ? (q == 4 ? 0.5 : 0.125) : 1.0;
+        a += w * ((1.0 - P.blend) * sample_corner(P.e_last + o, B, corner_of(B, lp)) +
+                  sample_corner(P.e_mix + o, B, corner_of(B, ip)));
+    }
+    if (!near) return false;
+    out.eta[c] = (double)cur.eta[c] == kThresh ? (T)kThresh : (T)fmax(kThresh, a);
+    return true;
 }
 
 // The NaN-skipping samplers only once a NaN exists in the bubble (its
 // sticky flag; the BIMOCQ fields derive from eta, which holds none before).
 template <typename T>
-__global__ __launch_bounds__(256) void k_bm_eta(const int4* __restrict__ tiles,
+__global__ __launch_bounds__(256, 3) void k_bm_eta(const int4* __restrict__ tiles,
                                                 const BubbleDev* __restrict__ bub,
                                                 StatePtrs<T> cur, StatePtrs<T> out, BimocqPtrs P) {
     const int4 tl = tiles[blockIdx.x];
@@ -2389,72 +2428,102 @@ __global__ __launch_bounds__(256) void k_bm_eta(const int4* __restrict__ tiles,
     int j, i;
     tile_cell(tl, j, i);
     if (j >= B.nth || i >= B.nph) return;
-    if (P.bt[tl.x].nans)
-        bm_eta_cell<T, true>(B, cur, out, P, j, i);
-    else
-        bm_eta_cell<T, false>(B, cur, out, P, j, i);
+    // the fast form; maps that vary too fast nearby take the general one
+    if (P.bt[tl.x].nans || !bm_eta_near<T>(B, cur, out, P, j, i)) bm_eta_cell<T>(B, cur, out, P, j, i);
 }
 
 // accumulateChangesCentered (bubble.cu:2081-2114) for eta and Gamma through
 // the new forward map, the new maps made current, and the distortion
 // (estimateDistortion, bubble.cu:1133-1168) of the new maps: its block
 // maximum goes to the bubble's running maximum.
-__global__ __launch_bounds__(256) void k_bm_accum(const int4* __restrict__ tiles,
+// The changes pulled back to one cell (de, dg) and the squared chords from
+// its centre to the two round trips of the maps: the general form, and the
+// one without NaNs, away from the poles and where the maps are smooth (false:
+// not the case here).
+__device__ __forceinline__ void bm_accum_cell(const BubbleDev& B, const BimocqPtrs& P, int j, int i,
+                                              const CellRef& cr, double& de, double& dg, U3& a, U3& e) {
+    const size_t o = (size_t)B.off, c = o + (size_t)j * B.nph + i;
+    const Field<double> ce{P.chg_e + o, B.nph, B.mask, B.nth - 1};
+    const Field<double> cg{P.chg_g + o, B.nph, B.mask, B.nth - 1};
+    const int ns = P.multisample ? 5 : 1;
+    de = dg = 0.0;
+#pragma unroll 1
+    for (int s = 0; s < ns; ++s) {
+        const int q = ns == 5 ? s : 4;
+        const double w = ns == 5 ? kMsW[q] : 1.0;
+        const P2d ip = index_near(B.invh, sample_map_u(P.nfwd, o, B.nth, B.nph,
+                                                        j + 0.5 + kMsDx[q], i + kMsDy[q]), cr);
+        de += w * sample_centered<double, true>(ce, B.nth, ip.x, ip.y);
+        dg += w * sample_centered<double, true>(cg, B.nth, ip.x, ip.y);
+    }
+    const P2d fi = index_near(B.invh, map_at(P.nfwd, c), cr);
+    const P2d bi = index_near(B.invh, map_at(P.nbwd, c), cr);
+    a = sample_map_u(P.nbwd, o, B.nth, B.nph, fi.x, fi.y);
+    e = sample_map_u(P.nfwd, o, B.nth, B.nph, bi.x, bi.y);
+}
+__device__ __forceinline__ bool bm_accum_near(const BubbleDev& B, const BimocqPtrs& P, int j, int i,
+                                              const CellRef& cr, double& de, double& dg, U3& a, U3& e) {
+    const size_t o = (size_t)B.off, c = o + (size_t)j * B.nph + i;
+    bool near = true;
+    Around at{};
+    if (P.multisample) sample_map_around(P.nfwd, o, B, j, i, at, near);
+    else at.mid = map_at(P.nfwd, c);
+    de = dg = 0.0;
+    P2d ip{};
+#pragma unroll 1
+    for (int q = P.multisample ? 0 : 4; q < 5; ++q) {
+        ip = index_near(B.invh, pick(at, q), cr);
+        const Corner<double> k = corner_of(B, ip);
+        const double w = P.multisample ? (q == 4 ? 0.5 : 0.125) : 1.0;
+        de += w * sample_corner(P.chg_e + o, B, k);
+        dg += w * sample_corner(P.chg_g + o, B, k);
+    }
+    // (the centre's sample came last: ip is the forward map's own position)
+    a = sample_map_near(P.nbwd, o, B, ip.x, ip.y, near);
+    const P2d bi = index_near(B.invh, map_at(P.nbwd, c), cr);
+    e = sample_map_near(P.nfwd, o, B, bi.x, bi.y, near);
+    return near;
+}
+
+__global__ __launch_bounds__(256, 3) void k_bm_accum(const int4* __restrict__ tiles,
                                                   const BubbleDev* __restrict__ bub,
                                                   BimocqPtrs P) {
-    __shared__ float red[8];
+    __shared__ double red[16];
     const int4 tl = tiles[blockIdx.x];
     if (tl.x < 0 || stopped(P.bt[tl.x])) return;
     const BubbleDev B = bub[tl.x];
     int j, i;
     tile_cell(tl, j, i);
-    float dmax = 0.0f;
+    double chord2 = 0.0;
     if (j < B.nth && i < B.nph) {
-        const size_t o = (size_t)B.off, c = o + (size_t)j * B.nph + i;
-        const Field<double> ce{P.chg_e + o, B.nph, B.mask, B.nth - 1};
-        const Field<double> cg{P.chg_g + o, B.nph, B.mask, B.nth - 1};
-        const int ns = P.multisample ? 5 : 1;
+        const size_t c = (size_t)B.off + (size_t)j * B.nph + i;
         const CellRef cr = cell_ref(P.tab, B, j, i);
+        double de, dg;
+        U3 a, e;
         // the changes derive from eta and Gamma: NaN-free while the bubble's
         // flag is clear (k_update sets it before this launch)
-        const bool nans = P.bt[tl.x].nans != 0;
-        double de = 0.0, dg = 0.0;
-        for (int s = 0; s < ns; ++s) {
-            const int q = ns == 5 ? s : 4;
-            const double w = ns == 5 ? kMsW[q] : 1.0;
-            const P2d ip = index_near(B.invh, sample_map_u(P.nfwd, o, B.nth, B.nph,
-                                                            j + 0.5 + kMsDx[q], i + kMsDy[q]), cr);
-            if (nans) {
-                de += w * sample_centered<double, true>(ce, B.nth, ip.x, ip.y);
-                dg += w * sample_centered<double, true>(cg, B.nth, ip.x, ip.y);
-            } else {
-                de += w * sample_centered<double, false>(ce, B.nth, ip.x, ip.y);
-                dg += w * sample_centered<double, false>(cg, B.nth, ip.x, ip.y);
-            }
-        }
+        if (P.bt[tl.x].nans || !bm_accum_near(B, P, j, i, cr, de, dg, a, e))
+            bm_accum_cell(B, P, j, i, cr, de, dg, a, e);
         P.e_delta[c] += de;
         P.g_delta[c] += dg;
-        const U3 f{P.nfwd.x[c], P.nfwd.y[c], P.nfwd.z[c]};
-        const U3 b{P.nbwd.x[c], P.nbwd.y[c], P.nbwd.z[c]};
-        const P2d fi = index_near(B.invh, f, cr), bi = index_near(B.invh, b, cr);
+        P.e_mix[c] = fma(P.blend, P.e_init[c], P.e_delta[c]);
         // the cell centre from the sin/cos tables
         const U3 x{cr.cP * cr.sT, cr.sP * cr.sT, cr.cT};
-        const U3 a = sample_map_u(P.nbwd, o, B.nth, B.nph, fi.x, fi.y);
-        const U3 e = sample_map_u(P.nfwd, o, B.nth, B.nph, bi.x, bi.y);
-        // dist (bubble.cu:60-79): great-circle distance in cells
-        const double da = B.invh * safe_acos_d(x.x * a.x + x.y * a.y + x.z * a.z);
-        const double dd = B.invh * safe_acos_d(x.x * e.x + x.y * e.y + x.z * e.z);
-        dmax = fmaxf((float)da, (float)dd);
+        auto chord = [&](const U3& q) {
+            const double dx = q.x - x.x, dy = q.y - x.y, dz = q.z - x.z;
+            return dx * dx + dy * dy + dz * dz;
+        };
+        chord2 = fmax(chord(a), chord(e));
+        const U3 f = map_at(P.nfwd, c), b = map_at(P.nbwd, c);
         P.fwd.x[c] = f.x; P.fwd.y[c] = f.y; P.fwd.z[c] = f.z;
         P.bwd.x[c] = b.x; P.bwd.y[c] = b.y; P.bwd.z[c] = b.z;
     }
-    dmax = wave_max(dmax);
-    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = dmax;
-    __syncthreads();
+    chord2 = block_max(chord2, red);
     if (threadIdx.x == 0) {
-        float m = 0.0f;
-        for (int w = 0; w < (int)(blockDim.x >> 6); ++w) m = fmaxf(m, red[w]);
-        // non-negative floats order as their bit patterns
+        // dist (bubble.cu:60-79), the great-circle distance in cells, of the
+        // block's largest: 2 asin(chord / 2) grows with the chord, so one
+        // thread forms it; non-negative floats order as their bit patterns
+        const float m = (float)(B.invh * 2.0 * asin(fmin(1.0, 0.5 * sqrt(chord2))));
         atomicMax(P.dist_bits + tl.x, __float_as_uint(m));
     }
 }
@@ -2574,9 +2643,11 @@ __global__ __launch_bounds__(256) void k_bm_finish(const int4* __restrict__ tile
     P.prev.x[c] = P.bwd.x[c];
     P.prev.y[c] = P.bwd.y[c];
     P.prev.z[c] = P.bwd.z[c];
+    P.e_last[c] = P.e_initlast[c] + P.e_deltalast[c];
     P.e_init[c] = (double)cur.eta[c];
     P.g_init[c] = (double)cur.gam[c];
     P.e_delta[c] = P.g_delta[c] = 0.0;
+    P.e_mix[c] = P.blend * P.e_init[c];
     set_identity(P.fwd, c, B.h, j, i);
     set_identity(P.bwd, c, B.h, j, i);
 }

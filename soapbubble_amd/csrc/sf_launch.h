@@ -14,6 +14,9 @@ struct BimocqPtrs {
     UMap fwd, bwd, prev, nfwd, nbwd;   // maps as unit vectors (x, y, z arrays)
     double *e_init, *e_initlast, *e_delta, *e_deltalast;
     double *g_init, *g_initlast, *g_delta, *g_deltalast;
+    // e_last = e_initlast + e_deltalast and e_mix = blend e_init + e_delta, the
+    // two sums that eta is sampled from while no field holds a NaN
+    double *e_last, *e_mix;
     double *chg_e, *chg_g, *err_e, *err_g, *cpy_e, *cpy_g;
     unsigned* dist_bits;   // per bubble: running max distortion (float bits)
     int* flag;             // per bubble: reinitialise at this step
