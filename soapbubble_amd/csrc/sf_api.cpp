@@ -271,6 +271,7 @@ struct Base {
     int host_hist = 0;
     std::vector<int> calib;   // max inner iterations per refinement seen while calibrating
     std::vector<int> sched;   // inner iterations per refinement of the fixed schedule
+    std::vector<int> last_used;   // inner PCG iterations per refinement of the last host-driven solve
     int method = 1;           // inner solver: 1 PCG, 2 Chebyshev
     bool mg = false;          // PCG preconditioned by the multigrid V-cycle
     bool spectral = false;    // PCG preconditioned by the row-mean operator
@@ -290,6 +291,7 @@ struct Base {
     // allocation, no stream, event, pinned buffer or graph of its own
     bool noalloc = false;
     double t_start = 0.0;     // air-flow time the set-up gives the bubbles
+    SolveCtl* ctl_h = nullptr;   // pinned copy of the control blocks
     void* stage_h = nullptr;  // pinned staging buffer of the downloads
     virtual ~Base() {
         if (stream) (void)hipStreamSynchronize(stream);
@@ -299,6 +301,7 @@ struct Base {
         for (auto& e : cev)
             if (e) (void)hipEventDestroy(e);
         if (sstat_h) (void)hipHostFree(sstat_h);
+        if (ctl_h) (void)hipHostFree(ctl_h);
         if (stage_h) (void)hipHostFree(stage_h);
         if (cstream) (void)hipStreamDestroy(cstream);
         for (void* p : owned) (void)hipFree(p);
@@ -889,8 +892,10 @@ struct Impl : Base {
     }
 
     bool all_flags(std::vector<SolveCtl>& c, bool inner_flag) {
-        SF_HIP(hipMemcpyAsync(c.data(), ctl_d, sizeof(SolveCtl) * nb, hipMemcpyDeviceToHost, stream));
+        SF_HIP(hipMemcpyAsync(ctl_h ? ctl_h : c.data(), ctl_d, sizeof(SolveCtl) * nb,
+                              hipMemcpyDeviceToHost, stream));
         SF_HIP(hipStreamSynchronize(stream));
+        if (ctl_h) std::copy(ctl_h, ctl_h + nb, c.begin());
         for (int b = 0; b < nb; ++b) {
             if (c[b].outer_done) continue;
             if (!inner_flag || !c[b].inner_done) return false;
@@ -1000,22 +1005,34 @@ struct Impl : Base {
         } else if (host_driven) {
             std::vector<SolveCtl> c(nb);
             std::vector<int> before(nb);
+            // The flags are read back where they are likely to be set: the
+            // inner ones first after as many iterations as the refinement took
+            // in the solve before (its launches past them return at once, so
+            // a late look costs little and an early one a wait for the
+            // device), then at growing intervals; the outer one not before
+            // the first refinement of a solve that never converges there.
             for (int k = 0; k < max_outer; ++k) {
                 for (const LaunchGeom& rg : pgeo)
                     launch_spmv<Ti>(stream, rg, bub_d, ctl_d, sys(x64[0]), p[1], p[0], 0, sp, partR,
                                     partB, partA, stride);
-                const bool done = all_flags(c, false);
-                if (trace_solve)
-                    std::fprintf(stderr, "[sf solve] outer %d residual %.3e (|b|^2 %.3e)%s\n", k,
-                                 c[0].rel_res, c[0].bb, done ? " converged" : "");
-                if (done) break;
-                for (int b = 0; b < nb; ++b) before[b] = c[b].iters;
-                cgstep(0);
-                for (int it = 1; it < max_inner; ++it) {
-                    inner(it);
-                    if ((mg || spectral || (it & 3) == 3) && all_flags(c, true)) break;
+                if (k > 0 || recording || last_used.empty() || trace_solve) {
+                    const bool done = all_flags(c, false);
+                    if (trace_solve)
+                        std::fprintf(stderr, "[sf solve] outer %d residual %.3e (|b|^2 %.3e)%s\n", k,
+                                     c[0].rel_res, c[0].bb, done ? " converged" : "");
+                    if (done) break;
                 }
-                all_flags(c, true);
+                for (int b = 0; b < nb; ++b) before[b] = k > 0 ? c[b].iters : 0;
+                cgstep(0);
+                int look = k < (int)last_used.size() ? std::max(last_used[k], 1) : mg || spectral ? 1 : 3;
+                bool seen = false;
+                for (int it = 1; it < max_inner && !seen; ++it) {
+                    inner(it);
+                    if (it < look) continue;
+                    seen = all_flags(c, true);
+                    look = it + std::max(1, it / 8);
+                }
+                if (!seen) all_flags(c, true);
                 int mx = 0;
                 for (int b = 0; b < nb; ++b) mx = std::max(mx, c[b].iters - before[b]);
                 used.push_back(mx);
@@ -1032,6 +1049,7 @@ struct Impl : Base {
                 resid((int)k + 1, e, spectral && end ? sstat_d : nullptr, end);
             }
         }
+        if (host_driven && method == 1) last_used = used;
         if (host_driven && recording) {
             if (calib.size() < used.size()) calib.resize(used.size(), 0);
             for (size_t k = 0; k < used.size(); ++k) calib[k] = std::max(calib[k], used[k]);
@@ -1370,6 +1388,7 @@ void setup(Base& c, int prec) {
     if (!c.noalloc) {
         SF_HIP(hipHostMalloc((void**)&c.sstat_h, 2 * nb * sizeof(SchedStat)));
         std::memset(c.sstat_h, 0, 2 * nb * sizeof(SchedStat));
+        SF_HIP(hipHostMalloc((void**)&c.ctl_h, nb * sizeof(SolveCtl)));
         for (auto& e : c.cev) SF_HIP(hipEventCreateWithFlags(&e, hipEventDisableTiming));
         SF_HIP(hipStreamCreateWithFlags(&c.cstream, hipStreamNonBlocking));
     }
