@@ -133,7 +133,7 @@ typedef struct {
                              the assembly's) on the context's own data, and
                              keep the fastest (sf_get_tuning reports them);
                              0: the fixed choices (256 columns; 8 cells a
-                             thread for rows of >= 2048 cells, else C)     */
+                             thread for rows of >= 768 cells, else C)      */
 } sf_options;
 
 typedef struct {

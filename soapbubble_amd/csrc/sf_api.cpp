@@ -1058,7 +1058,7 @@ struct Impl : Base {
     }
 
     void update(bool finalize) override {
-        launch_update<T>(stream, geom, bub_d, time_d, ctl_d, tab, nxt, air(), x64[0], x64[1], cur,
+        launch_update<T>(stream, geom, nb, bub_d, time_d, ctl_d, tab, nxt, air(), x64[0], x64[1], cur,
                          finalize ? 1 : 0, hist_d, sp, partR, stride,
                          bimocq ? bm.chg_e : nullptr, bimocq ? bm.chg_g : nullptr, gdel, gnext,
                          acc);
@@ -1477,7 +1477,9 @@ void setup(Base& c, int prec) {
     // narrower row takes its thread count rounded up to whole waves, as
     // many rows of one bubble to a block as fit (row_seg). The Chebyshev
     // launches take 8 cells a thread where the assembly takes 4 and the
-    // widest row has at least 2048 cells.
+    // widest row has at least 768 cells (a launch at 512x1024 7.26 -> 6.96 us,
+    // at 1000x2000 18.2 -> 15.7 with its loads issued first; at 256x512 no
+    // difference, and the 96-bubble batch of narrower rows loses: 27 -> 31).
     auto fits = [](int nph, int C) { return nph % C == 0 && nph / C >= 4 && nph / C <= kRowThreadsMax; };
     c.pgeo.clear();
     c.pgeo_inner.clear();
@@ -1510,7 +1512,7 @@ void setup(Base& c, int prec) {
         const int C = gcpt[gi];
         const int wmax = ws.back();
         int Ci = C;
-        if (!c.fp64_inner() && C == 4 && wmax / 8 >= 256) {
+        if (!c.fp64_inner() && C == 4 && wmax / 8 >= 96) {
             bool ok8 = true;
             for (int w : ws) ok8 = ok8 && fits(w, 8);
             if (ok8) Ci = 8;

@@ -1037,10 +1037,53 @@ __constant__ const double kMsDx[5] = {-0.25, 0.25, -0.25, 0.25, 0.0};
 __constant__ const double kMsDy[5] = {-0.25, -0.25, 0.25, 0.25, 0.0};
 
 // -------------------------------------------------------- reductions ----
+// Wave reductions by DPP (row shifts, then the last lanes of rows 0 and 2
+// into the rows after them, of row 1 into rows 2 and 3): lane 63 holds the
+// result, which every lane receives. Register moves a few cycles apart, where
+// shuffles through the LDS unit wait a hundred for each of six levels: 0.3-0.5
+// us a row kernel, which at the small sizes is one chain of latencies.
+template <int CTRL, int ROWS>
+__device__ __forceinline__ double dpp_or_zero(double v) {
+    u32x2 u = __builtin_bit_cast(u32x2, v);
+    const unsigned int x = u.x, y = u.y;
+    u.x = (unsigned int)__builtin_amdgcn_update_dpp(0, (int)x, CTRL, ROWS, 0xf, false);
+    u.y = (unsigned int)__builtin_amdgcn_update_dpp(0, (int)y, CTRL, ROWS, 0xf, false);
+    return __builtin_bit_cast(double, u);
+}
+template <int CTRL, int ROWS>
+__device__ __forceinline__ float dpp_or_zero(float v) {
+    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, ROWS, 0xf, false));
+}
+__device__ __forceinline__ double last_lane(double v) {
+    u32x2 u = __builtin_bit_cast(u32x2, v);
+    const unsigned int x = u.x, y = u.y;
+    u.x = (unsigned int)__builtin_amdgcn_readlane((int)x, 63);
+    u.y = (unsigned int)__builtin_amdgcn_readlane((int)y, 63);
+    return __builtin_bit_cast(double, u);
+}
+__device__ __forceinline__ float last_lane(float v) {
+    return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), 63));
+}
+// `op` combines two values; a lane without a source combines with zero
+template <typename T, typename Op>
+__device__ __forceinline__ T wave_reduce(T v, Op op) {
+    v = op(v, dpp_or_zero<0x111, 0xf>(v));   // row_shr:1
+    v = op(v, dpp_or_zero<0x112, 0xf>(v));   // row_shr:2
+    v = op(v, dpp_or_zero<0x114, 0xf>(v));   // row_shr:4
+    v = op(v, dpp_or_zero<0x118, 0xf>(v));   // row_shr:8
+    v = op(v, dpp_or_zero<0x142, 0xa>(v));   // row_bcast:15 into rows 1 and 3
+    v = op(v, dpp_or_zero<0x143, 0xc>(v));   // row_bcast:31 into rows 2 and 3
+    return last_lane(v);
+}
 __device__ __forceinline__ double wave_sum(double v) {
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) v += __shfl_down(v, o, 64);
-    return v;
+    return wave_reduce(v, [](double a, double b) { return a + b; });
+}
+// the maximum of non-negative values
+__device__ __forceinline__ double wave_max(double v) {
+    return wave_reduce(v, [](double a, double b) { return fmax(a, b); });
+}
+__device__ __forceinline__ float wave_max(float v) {
+    return wave_reduce(v, [](float a, float b) { return fmaxf(a, b); });
 }
 
 // Deterministic block sum of NV values; every thread receives the sums.
@@ -1069,8 +1112,7 @@ __device__ __forceinline__ void block_sum(double (&v)[NV], double* red) {
 // it. `red` must hold 16 doubles of LDS.
 __device__ __forceinline__ double block_max(double v, double* red) {
     const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6, nw = (blockDim.x + 63) >> 6;
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) v = fmax(v, __shfl_down(v, o, 64));
+    v = wave_max(v);
     __syncthreads();
     if (lane == 0) red[wid] = v;
     __syncthreads();
@@ -1137,8 +1179,7 @@ __device__ __forceinline__ void seg_sum(double (&v)[NV], double* red, const RowS
 // The segment's maximum of a non-negative value.
 __device__ __forceinline__ double seg_max(double v, double* red, const RowSeg& s) {
     const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) v = fmax(v, __shfl_down(v, o, 64));
+    v = wave_max(v);
     __syncthreads();
     if (lane == 0) red[wid] = v;
     __syncthreads();
@@ -1211,16 +1252,10 @@ __host__ __device__ inline size_t acc_index(int b, int slot, int v, int sub) {
 // The sum (maximum) of one value of a slot, in every lane of the calling
 // wave; the same in every wave (fixed reduction order).
 __device__ __forceinline__ double acc_sum(const double* __restrict__ acc, int b, int slot, int v) {
-    double x = acc[acc_index(b, slot, v, threadIdx.x & 63)];
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) x += __shfl_xor(x, o, 64);
-    return x;
+    return wave_sum(acc[acc_index(b, slot, v, threadIdx.x & 63)]);
 }
 __device__ __forceinline__ double acc_max(const double* __restrict__ acc, int b, int slot, int v) {
-    double x = acc[acc_index(b, slot, v, threadIdx.x & 63)];
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) x = fmax(x, __shfl_xor(x, o, 64));
-    return x;
+    return wave_max(acc[acc_index(b, slot, v, threadIdx.x & 63)]);
 }
 __device__ __forceinline__ void acc_add(double* acc, int b, int slot, int v, int sub, double x) {
     unsafeAtomicAdd(acc + acc_index(b, slot, v, sub & (kAccSub - 1)), x);
@@ -1264,12 +1299,6 @@ __device__ __forceinline__ double pre_rcp(double x) { return 1.0 / x; }
 template <typename Ti> struct PcrTol;
 template <> struct PcrTol<float> { static constexpr float v = 2e-9f; };
 template <> struct PcrTol<double> { static constexpr double v = 1e-18; };
-
-__device__ __forceinline__ float wave_max(float v) {
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) v = fmaxf(v, __shfl_down(v, o, 64));
-    return __shfl(v, 0, 64);
-}
 
 // Parallel cyclic reduction of one periodic tridiagonal row held in LDS,
 // normalised to unit diagonal: x_i + a_i x_{i-1} + c_i x_{i+1} = d_i, n a

@@ -1802,18 +1802,37 @@ __global__ void k_cheb(const int2* __restrict__ rows, const BubbleDev* __restric
     if (rw.x < 0) return;
     const int b = rw.x;
     SolveCtl* Cb = ctl + b;
-    const int od = flag_load(&Cb->outer_done);
-    const double* __restrict__ acc0 = sys.acc;
-    const double mu = acc_max(acc0, b, acc_slot_res(0), 4);
-    const bool converged =
-        it == 1 && residual_norm(acc_sum(acc0, b, acc_slot_res(kr), 0),
-                                 acc_sum(acc0, b, acc_slot_res(kr), 1), sp.absolute) <= sp.tol;
     const BubbleDev B = bub[b];
     const int nph = B.nph, m = B.mask, nth = B.nth;
     const RowSeg sg = row_seg<PK>(nph / C);
     const int j = rw.y + sg.seg;
     const bool valid = !PK || (sg.seg < sg.nseg && j < nth);
     const bool leader = (rw.y == 0 && threadIdx.x == 0);
+    const size_t row = (size_t)B.off + (size_t)j * nph;
+    const bool hasN = j > 0, hasS = j < nth - 1;
+    const bool act = valid && sg.lt < nph / C;
+    const int i0 = C * sg.lt;
+    // e_1 = z_0 and e_0 = 0, so d_0 = e_1 - e_0 = z_0
+    const Ti* __restrict__ e = it == 1 ? sys.z : ek;
+    // The row's loads are issued before the tests of the solve's state, whose
+    // own loads would otherwise come first in the chain (a launch that only
+    // has to return is rare here).
+    Ti ev[C], dvv[C], a[C], cc[C], d[C], eN[C], eS[C], rin[C], eW = Ti(0), eE = Ti(0);
+#pragma unroll
+    for (int q = 0; q < C; ++q) ev[q] = dvv[q] = a[q] = cc[q] = d[q] = rin[q] = eN[q] = eS[q] = Ti(0);
+    RowOp<Ti, C> op;
+    if (act) {
+        ld_stencil<Ti, C>(e, row, i0, m, nph, hasN, hasS, ev, eW, eE, eN, eS);
+        if (it > 1) ld_row<C>(ekm1 + row + i0, dvv);
+        ld_row<C>(sys.r + row + i0, rin);
+        op.load(sys, row, i0, m, nph, hasN, hasS);
+    }
+    const int od = flag_load(&Cb->outer_done);
+    const double* __restrict__ acc0 = sys.acc;
+    const double mu = acc_max(acc0, b, acc_slot_res(0), 4);
+    const bool converged =
+        it == 1 && residual_norm(acc_sum(acc0, b, acc_slot_res(kr), 0),
+                                 acc_sum(acc0, b, acc_slot_res(kr), 1), sp.absolute) <= sp.tol;
     if (od || converged) {
         if (leader && converged) flag_store(&Cb->outer_done, 1);
         return;
@@ -1841,33 +1860,11 @@ __global__ void k_cheb(const int2* __restrict__ rows, const BubbleDev* __restric
     const Ti cd = kk == 0 ? Ti(0) : (Ti)(rho * rho_prev),
              cz = kk == 0 ? Ti(1) : (Ti)(2.0 * rho / delta);
     const int steps = block_steps<PK>(sys.rsteps, B.pr0, rw.y, nth - rw.y, sg, red);
-    const size_t row = (size_t)B.off + (size_t)j * nph;
-    const bool hasN = j > 0, hasS = j < nth - 1;
-    const bool act = valid && sg.lt < nph / C;
-    const int i0 = C * sg.lt;
-    // e_1 = z_0 and e_0 = 0, so d_0 = e_1 - e_0 = z_0
-    const Ti* __restrict__ e = it == 1 ? sys.z : ek;
-    Ti ev[C], dvv[C], a[C], cc[C], d[C];
-#pragma unroll
-    for (int q = 0; q < C; ++q) ev[q] = dvv[q] = a[q] = cc[q] = d[q] = Ti(0);
     double acc = 0.0;
     if (act) {
-        Ti eN[C], eS[C], eW, eE;
-        ld_stencil<Ti, C>(e, row, i0, m, nph, hasN, hasS, ev, eW, eE, eN, eS);
-        if (it > 1) {
-            // d_{k-1} = e_k - e_{k-1}
-            Ti em[C];
-            ld_row<C>(ekm1 + row + i0, em);
+        // d_{k-1} = e_k - e_{k-1}
 #pragma unroll
-            for (int q = 0; q < C; ++q) dvv[q] = ev[q] - em[q];
-        } else {
-#pragma unroll
-            for (int q = 0; q < C; ++q) dvv[q] = ev[q];
-        }
-        Ti rin[C];
-        ld_row<C>(sys.r + row + i0, rin);
-        RowOp<Ti, C> op;
-        op.load(sys, row, i0, m, nph, hasN, hasS);
+        for (int q = 0; q < C; ++q) dvv[q] = it > 1 ? ev[q] - dvv[q] : ev[q];
         Ti ax[C], r[C];
         op.apply(ev, eW, eE, eN, eS, ax);
 #pragma unroll
@@ -2069,7 +2066,7 @@ __device__ __forceinline__ void st2(T* __restrict__ p, T a, T b) {
 }
 
 template <typename T>
-__global__ __launch_bounds__(128) void k_update(const int4* __restrict__ tiles,
+__global__ __launch_bounds__(128) void k_update(int nb, const int4* __restrict__ tiles,
                                                 const BubbleDev* __restrict__ bub,
                                                 BubbleTime* __restrict__ btime,
                                                 SolveCtl* __restrict__ ctl, Tables tab,
@@ -2083,20 +2080,23 @@ __global__ __launch_bounds__(128) void k_update(const int4* __restrict__ tiles,
                                                 T* __restrict__ gdel, T* __restrict__ gnext,
                                                 double* __restrict__ acc) {
     __shared__ double red[16 * 4];
-    const int4 tl = tiles[blockIdx.x];
+    if ((int)blockIdx.x < nb) {
+        // the launch's first blocks, one a bubble: solve verdict, and the time
+        // advance that the next step's advection applies (beside the tiles:
+        // as a part of the first tile it was the last of a small launch)
+        const int b = blockIdx.x;
+        if (stopped(btime[b])) return;
+        if (fin) finalize_block(bub[b], ctl + b, hist + b, sp, partR, stride, red);
+        if (fin && threadIdx.x == 0 && (btime[b].stop & 1) && !ctl[b].converged) btime[b].stop |= 2;
+        if (threadIdx.x == 0 && btime[b].advance) btime[b].pending = 1;
+        if (threadIdx.x == 0 && gdel) btime[b].gpend = 1;
+        // the next assembly adds its sums into a cleared slot
+        if (threadIdx.x < 64) acc_zero(acc, b, acc_slot_res(0));
+        return;
+    }
+    const int4 tl = tiles[blockIdx.x - nb];
     if (tl.x < 0 || stopped(btime[tl.x])) return;
     const BubbleDev B = bub[tl.x];
-    if (tl.y == 0 && tl.z == 0) {
-        // first tile of the bubble: solve verdict, and the time advance that
-        // the next step's advection applies
-        if (fin) finalize_block(B, ctl + tl.x, hist + tl.x, sp, partR, stride, red);
-        if (fin && threadIdx.x == 0 && (btime[tl.x].stop & 1) && !ctl[tl.x].converged)
-            btime[tl.x].stop |= 2;
-        if (threadIdx.x == 0 && btime[tl.x].advance) btime[tl.x].pending = 1;
-        if (threadIdx.x == 0 && gdel) btime[tl.x].gpend = 1;
-        // the next assembly adds its sums into a cleared slot
-        if (threadIdx.x < 64) acc_zero(acc, tl.x, acc_slot_res(0));
-    }
     const int sh = __builtin_ctz((unsigned)tl.w) - 1;   // tile width / 2 = 2^sh
     const int j = tl.y + ((int)threadIdx.x >> sh);
     const int i = tl.z + 2 * ((int)threadIdx.x & ((tl.w >> 1) - 1));
@@ -2878,12 +2878,12 @@ void launch_sched_stats(hipStream_t s, SchedStat* d, SchedStat* h, int nb) {
 }
 
 template <typename T>
-void launch_update(hipStream_t s, const LaunchGeom& g, const BubbleDev* bub, BubbleTime* bt,
+void launch_update(hipStream_t s, const LaunchGeom& g, int nb, const BubbleDev* bub, BubbleTime* bt,
                    SolveCtl* ctl, const Tables& tab, StatePtrs<T> st, AirPtrs<T> air,
                    const double* x0, const double* x1, StatePtrs<T> out, int fin, SolveHist* hist,
                    const SolveParams& sp, const double* partR, long stride, double* chg_e,
                    double* chg_g, T* gdel, T* gnext, double* acc) {
-    hipLaunchKernelGGL(k_update<T>, dim3(g.ntiles), dim3(128), 0, s, g.tiles, bub, bt, ctl, tab, st,
+    hipLaunchKernelGGL(k_update<T>, dim3(nb + g.ntiles), dim3(128), 0, s, nb, g.tiles, bub, bt, ctl, tab, st,
                        air, x0, x1, out, fin, hist, sp, partR, stride, chg_e, chg_g, gdel, gnext, acc);
 }
 
@@ -2945,12 +2945,12 @@ SF_INST_TI(double)
                                      const SolveParams&, const double*, double*, long);
 SF_INST_MG(float)
 SF_INST_MG(double)
-template void launch_update<float>(hipStream_t, const LaunchGeom&, const BubbleDev*, BubbleTime*,
+template void launch_update<float>(hipStream_t, const LaunchGeom&, int, const BubbleDev*, BubbleTime*,
                                    SolveCtl*, const Tables&, StatePtrs<float>, AirPtrs<float>,
                                    const double*, const double*, StatePtrs<float>, int,
                                    SolveHist*, const SolveParams&, const double*, long, double*,
                                    double*, float*, float*, double*);
-template void launch_update<double>(hipStream_t, const LaunchGeom&, const BubbleDev*, BubbleTime*,
+template void launch_update<double>(hipStream_t, const LaunchGeom&, int, const BubbleDev*, BubbleTime*,
                                     SolveCtl*, const Tables&, StatePtrs<double>, AirPtrs<double>,
                                     const double*, const double*, StatePtrs<double>, int,
                                     SolveHist*, const SolveParams&, const double*, long, double*,

@@ -203,7 +203,7 @@ void launch_finalize(hipStream_t s, int nb, const BubbleDev* bub, SolveCtl* ctl,
                      const SolveParams& sp, const double* partR, long stride);
 void launch_sched_stats(hipStream_t s, SchedStat* d, SchedStat* h, int nb);
 template <typename T>
-void launch_update(hipStream_t s, const LaunchGeom& g, const BubbleDev* bub, BubbleTime* bt,
+void launch_update(hipStream_t s, const LaunchGeom& g, int nb, const BubbleDev* bub, BubbleTime* bt,
                    SolveCtl* ctl, const Tables& tab, StatePtrs<T> st, AirPtrs<T> air,
                    const double* x0, const double* x1, StatePtrs<T> out, int fin, SolveHist* hist,
                    const SolveParams& sp, const double* partR, long stride, double* chg_e,
