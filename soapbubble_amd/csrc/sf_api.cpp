@@ -1320,6 +1320,16 @@ LaunchGeom pack_rows(Base& c, const std::vector<int>& ws, int C, size_t esz, siz
     return g;
 }
 
+// The step of one bubble and the products of its row systems that follow
+// from it.
+static void set_step(BubbleDev& B, double dt) {
+    B.dt = dt;
+    B.dt32 = (float)dt;
+    B.inv_dt = 1.0 / dt;
+    B.cr_dt = B.Cr * dt;
+    B.w_scale = (B.invh * B.invh) * (B.M * dt);
+}
+
 void setup(Base& c, int prec) {
     const int nb = c.nb;
     SF_HIP(hipSetDevice(c.device));
@@ -1350,7 +1360,6 @@ void setup(Base& c, int prec) {
         B.off = off;
         B.h = kPi / d.n_theta;
         B.invh = d.n_theta / kPi;
-        B.dt = c.der[b].dt;
         B.M = c.der[b].M;
         B.Cr = c.der[b].Cr;
         B.gs = c.der[b].gs;
@@ -1362,7 +1371,7 @@ void setup(Base& c, int prec) {
         B.viscous = c.opt.viscous ? 1 : 0;
         B.re = c.der[b].re;
         B.invh32 = (float)B.invh;
-        B.dt32 = (float)B.dt;
+        set_step(B, c.der[b].dt);
         B.air_scale = c.der[b].radius / c.der[b].U;
         // every bubble starts on a 256-byte boundary (the row kernels load
         // C consecutive cells as one aligned vector)
@@ -2143,8 +2152,7 @@ int sf_set_dt(sf_ctx* ctx, int32_t b, double dt_seconds) {
                 c.sp_short.clear();
                 drop_calibration(c);
             }
-            c.bub_h[k].dt = dtn;
-            c.bub_h[k].dt32 = (float)dtn;
+            set_step(c.bub_h[k], dtn);
             c.time_h[k].dt_s = dt_seconds;
         }
         SF_HIP(hipMemcpy(c.bub_d, c.bub_h.data(), c.nb * sizeof(BubbleDev), hipMemcpyHostToDevice));

@@ -21,6 +21,9 @@ struct BubbleDev {
     double h, invh, dt;          // grid spacing, 1/h, non-dimensional step
     double M, Cr, gs, gamma_max, eva;
     double re;                   // Re^-1 of the VISCOUS path
+    // products of the row systems that hold for a whole bubble, in scalar
+    // registers there: 1/dt, Cr dt, M dt / h^2
+    double inv_dt, cr_dt, w_scale;
     float invh32, dt32;          // 1/h and dt for the FP32 traces
     double air_scale;            // radius / U: speed of the air corridor
     int gravity, evaporation, airflow, viscous;
@@ -190,6 +193,10 @@ __device__ __forceinline__ float tfma(float a, float b, float c) { return fmaf(a
 __device__ __forceinline__ double tfma(double a, double b, double c) { return fma(a, b, c); }
 __device__ __forceinline__ float tabs(float x) { return fabsf(x); }
 __device__ __forceinline__ double tabs(double x) { return fabs(x); }
+__device__ __forceinline__ float tmax(float a, float b) { return fmaxf(a, b); }
+__device__ __forceinline__ double tmax(double a, double b) { return fmax(a, b); }
+__device__ __forceinline__ float tmin(float a, float b) { return fminf(a, b); }
+__device__ __forceinline__ double tmin(double a, double b) { return fmin(a, b); }
 
 // bubbleLerp (bubble.cu:153-160): NaN operands are skipped. With NANS =
 // false the fields are known to hold no NaN (a per-bubble flag that every

@@ -446,55 +446,141 @@ __device__ __forceinline__ void st_row(X* __restrict__ p, const X (&v)[C]) {
 // bl)), + for u_phi, - for u_theta. The mirror columns nph - i0 - k, k >= 1,
 // are the C-aligned block [nph - i0 - C, nph - i0) read backwards, so both
 // sides come as row vectors; column (nph - i0) mod nph is the one extra.
-// FP32 fields only; the blend in FP32 too (the reference's float
-// arithmetic), which keeps the 3 C + 1 results in single registers.
-template <int C, int N, bool MINUS, bool P2>
-__device__ __forceinline__ void air_blend(const float* __restrict__ a0,
-                                          const float* __restrict__ shape, size_t row, int i0,
-                                          int nph, int m, float kt, float bl, float (&out)[N]) {
-    float a[C], sh[C], am[C], sm[C];
+// In the precision of the fields (FP32: the reference's float arithmetic).
+// GUARD: a NaN of the corridor counts as no air.
+template <int C, int N, bool MINUS, bool P2, bool GUARD, typename T>
+__device__ __forceinline__ void air_blend(const T* __restrict__ a0, const T* __restrict__ shape,
+                                          size_t row, int i0, int nph, int m, T kt, T bl,
+                                          T (&out)[N]) {
+    T a[C], sh[C], am[C], sm[C];
     ld_row<C>(a0 + row + i0, a);
     ld_row<C>(shape + row + i0, sh);
     const size_t mb = row + (size_t)(nph - i0 - C), cm = row + wrap_t<P2>(nph - i0, nph, m);
     ld_row<C>(a0 + mb, am);
     ld_row<C>(shape + mb, sm);
-    auto val = [&](float x, float y) {
-        const float v = fmaf(y, kt, x);
-        return __builtin_isnan(v) ? 0.0f : v;
+    auto val = [&](T x, T y) {
+        const T v = tfma(y, kt, x);
+        return GUARD && __builtin_isnan(v) ? T(0) : v;
     };
     const size_t ce = row + wrap_t<P2>(i0 + C, nph, m);
+    const T ob = T(1) - bl;
 #pragma unroll
     for (int k = 0; k < N; ++k) {
-        const float own = k < C ? val(a[k], sh[k]) : val(a0[ce], shape[ce]);
-        const float mir = k == 0 ? val(a0[cm], shape[cm]) : val(am[C - k], sm[C - k]);
-        out[k] = MINUS ? 0.5f * (own * bl - mir * (1.0f - bl)) : 0.5f * (own * bl + mir * (1.0f - bl));
+        const T own = k < C ? val(a[k], sh[k]) : val(a0[ce], shape[ce]);
+        const T mir = k == 0 ? val(a0[cm], shape[cm]) : val(am[C - k], sm[C - k]);
+        out[k] = T(0.5) * tfma(own, bl, MINUS ? -(mir * ob) : mir * ob);
     }
 }
 
 // Operator (and optionally right-hand side) of the C consecutive cells
-// [i0, i0 + C) of row j, computed from row-vector loads. Every phi face is
-// evaluated once and shared by its two cells; each expression is the one of
-// concentrationLinearSystemKernel (bubble.cu:1330-1472), so a face weight
-// has the same value whichever cell computes it.
+// [i0, i0 + C) of a row.
 template <int C, typename T>
 struct RowSys {
     double wN[C], wS[C], wF[C + 1];   // effective weights; wF[k] is the face west of cell k
     double diag[C], rhs[C];
-    bool brk[C];
+    double r0[C];   // with the right-hand side: its residual at the initial iterate
     // the initial iterate on the cells and their neighbours: a value of the
-    // state precision, or gamma_max on a broken cell; kept as the state's
-    // value and the broken flags (an FP32 state then takes half the
-    // registers of FP64 copies)
+    // state precision, or gamma_max on a broken cell (to the state precision
+    // on a neighbour, whose weight is zero)
     T x0v[C], x0Nv[C], x0Sv[C], x0Wv, x0Ev;
-    bool bN[C], bS[C], bW, bE;
+    // C = 16 has 50 of them
+    std::conditional_t<(C > 8), unsigned long long, unsigned> brk;   // broken cells: own at bit k, north C + k, south 2 C + k, west 3 C, east 3 C + 1
     double gmax;
-    __device__ __forceinline__ double x0(int k) const { return brk[k] ? gmax : (double)x0v[k]; }
-    __device__ __forceinline__ double x0N(int k) const { return bN[k] ? gmax : (double)x0Nv[k]; }
-    __device__ __forceinline__ double x0S(int k) const { return bS[k] ? gmax : (double)x0Sv[k]; }
-    __device__ __forceinline__ double x0W() const { return bW ? gmax : (double)x0Wv; }
-    __device__ __forceinline__ double x0E() const { return bE ? gmax : (double)x0Ev; }
+    __device__ __forceinline__ double x0(int k) const { return brk >> k & 1 ? gmax : (double)x0v[k]; }
+    __device__ __forceinline__ double x0N(int k) const { return (double)x0Nv[k]; }
+    __device__ __forceinline__ double x0S(int k) const { return (double)x0Sv[k]; }
+    __device__ __forceinline__ double x0W() const { return (double)x0Wv; }
+    __device__ __forceinline__ double x0E() const { return (double)x0Ev; }
 };
 
+// The velocities and the blended air on the faces of C cells (state
+// precision), GUARD: NaN as zero. Without it the return value is the sum of
+// them all, not finite where one of them is not.
+template <int C, typename T>
+struct RowFlux {
+    T u[C + 1], vN[C], vS[C];
+    T ua[C + 1], vaN[C], vaS[C];
+};
+template <bool GUARD, bool P2, int C, typename T>
+__device__ __forceinline__ T flux_load(const BubbleDev& B, double t, const StatePtrs<T>& s,
+                                       const AirPtrs<T>& air, int j, int i0, RowFlux<C, T>& f) {
+    const int nph = B.nph, m = B.mask;
+    const size_t row = (size_t)B.off + (size_t)j * nph;
+    const bool hasN = j > 0, hasS = j < B.nth - 1;
+    T u[C];
+    ld_row<C>(s.uph + row + i0, u);
+#pragma unroll
+    for (int k = 0; k < C; ++k) {
+        f.u[k] = u[k];
+        f.ua[k] = f.vaN[k] = f.vaS[k] = T(0);
+    }
+    f.u[C] = s.uph[row + wrap_t<P2>(i0 + C, nph, m)];
+    f.ua[C] = T(0);
+    // the pole faces carry no flux: a row without the neighbour reads a row
+    // that exists, its zero face weight drops it (GUARD: whatever it holds)
+    const size_t rN = hasN ? row - nph : row, rS = hasS ? row : row - nph;
+    ld_row<C>(s.uth + rN + i0, f.vN);
+    ld_row<C>(s.uth + rS + i0, f.vS);
+    if (B.airflow) {
+        // per phi face, shared by the two cells of the face; v at the north
+        // and south faces of the cells
+        const T kt = (T)(3.0 - fabs(t - 3.0)), bl = (T)(t / 12.0);
+        // FP32 fields: row vectors; FP64 fields (twice the registers) per
+        // column
+        if constexpr (sizeof(T) == 4) {
+            air_blend<C, C + 1, false, P2, GUARD>(air.ua0, air.au, row, i0, nph, m, kt, bl, f.ua);
+            air_blend<C, C, true, P2, GUARD>(air.va0, air.av, rN, i0, nph, m, kt, bl, f.vaN);
+            air_blend<C, C, true, P2, GUARD>(air.va0, air.av, rS, i0, nph, m, kt, bl, f.vaS);
+        } else {
+#pragma unroll
+            for (int k = 0; k <= C; ++k) {
+                const int i = wrap_t<P2>(i0 + k, nph, m), opp = wrap_t<P2>(nph - i, nph, m);
+                auto blend = [&](const T* a0, const T* sh, size_t r, bool minus) {
+                    const T own = air_at(a0, sh, r + i, kt), mir = air_at(a0, sh, r + opp, kt) * (1 - bl);
+                    return 0.5 * fma(own, bl, minus ? -mir : mir);
+                };
+                f.ua[k] = blend(air.ua0, air.au, row, false);
+                if (k == C) continue;
+                f.vaN[k] = blend(air.va0, air.av, rN, true);
+                f.vaS[k] = blend(air.va0, air.av, rS, true);
+            }
+        }
+    }
+    T sum = T(0);
+    if constexpr (GUARD) {
+        auto zero = [](T& v) { v = __builtin_isnan(v) ? T(0) : v; };
+#pragma unroll
+        for (int k = 0; k < C; ++k) {
+            zero(f.u[k]), zero(f.vN[k]), zero(f.vS[k]);
+            if (!hasN) f.vN[k] = f.vaN[k] = T(0);
+            if (!hasS) f.vS[k] = f.vaS[k] = T(0);
+        }
+        zero(f.u[C]);
+    } else {
+        sum = f.u[C] + f.ua[C];
+#pragma unroll
+        for (int k = 0; k < C; ++k)
+            sum += ((f.u[k] + f.ua[k]) + (f.vN[k] + f.vaN[k])) + (f.vS[k] + f.vaS[k]);
+    }
+    return sum;
+}
+
+// The row system of this thread's cells from row-vector loads. Every phi
+// face is evaluated once and shared by its two cells; the terms are those of
+// concentrationLinearSystemKernel (bubble.cu:1330-1472), so a face weight has
+// the same value whichever cell computes it. The wave's cells are first taken
+// to be ordinary ones (straight-line code without flags, selects or divergent
+// branches); a wave that holds a broken cell in its stencils, a concentration
+// whose reciprocal is out of range, or a NaN among velocities and air takes
+// two detours that put them right, which change no bit of an ordinary cell.
+// Flags on every cell made four divergent branches a thread and joined their
+// registers at each, and every load of a face waited behind the branches of
+// the one before it. Without them a step takes 157.7 us at 1024 x 2048 (before
+// 161.6), 37.9 at 256 x 512 (39.4), 190 at 1000 x 2000 (195), 497 at 1024 x
+// 2048 in FP64 (522: 22 registers spilled instead of 56). The residual of the
+// initial iterate is formed beside the right-hand side because the iterate's
+// 14 values did not fit until the detour had passed (10 spilled in packed
+// rows, whose assembly then took 115 us instead of 104 on 96 bubbles).
 // With `guess` (assembly only) the initial iterate is Gamma* + guess instead
 // of Gamma* on cells that are not broken.
 template <typename T, int C, bool RHS, bool VISC, bool P2>
@@ -511,193 +597,193 @@ __device__ __forceinline__ void row_system(const BubbleDev& B, double t, const T
     const size_t rowN = hasN ? row - nph : row, rowS = hasS ? row + nph : row;
     const int iNS = hasN ? i0 : wrap_t<P2>(i0 + nth, nph, m);
     const int iSS = hasS ? i0 : wrap_t<P2>(i0 + nth, nph, m);
-    T ev[C], eNv[C], eSv[C], gv[C], gNv[C], gSv[C];
+    T ev[C], eNv[C], eSv[C], gv[C];
     ld_row<C>(s.eta + row + i0, ev);
     ld_row<C>(s.gam + row + i0, gv);
     ld_row_wrap<C, P2>(s.eta + rowN, iNS, nph, m, eNv);
-    ld_row_wrap<C, P2>(s.gam + rowN, iNS, nph, m, gNv);
+    ld_row_wrap<C, P2>(s.gam + rowN, iNS, nph, m, q.x0Nv);
     ld_row_wrap<C, P2>(s.eta + rowS, iSS, nph, m, eSv);
-    ld_row_wrap<C, P2>(s.gam + rowS, iSS, nph, m, gSv);
+    ld_row_wrap<C, P2>(s.gam + rowS, iSS, nph, m, q.x0Sv);
     const int iWc = wrap_t<P2>(i0 - 1, nph, m), iEc = wrap_t<P2>(i0 + C, nph, m);
-    const double eW = (double)s.eta[row + iWc], eE = (double)s.eta[row + iEc];
-    double gW = (double)s.gam[row + iWc], gE = (double)s.gam[row + iEc];
+    const T eW = s.eta[row + iWc], eE = s.eta[row + iEc];
+    q.x0Wv = s.gam[row + iWc];
+    q.x0Ev = s.gam[row + iEc];
 
-    const double dt = B.dt, invDt = 1.0 / dt, Cr = B.Cr;
-    const double CrDt = Cr * dt, MDt = B.M * dt, s2 = B.invh * B.invh;
-    const double sinN = tab.sinFace[B.rt0 + j], sinS = tab.sinFace[B.rt0 + j + 1];
-    const double sinTheta = tab.sinTc[B.rt0 + j], csc = tab.cscTc[B.rt0 + j];
-    const double cW = s2 * csc * MDt, cN = s2 * sinN * MDt, cS = s2 * sinS * MDt;
+    // FP32 fields: the velocities and the air are on their way before the
+    // wave's case is known, their NaNs found in their sum. FP64 fields, twice
+    // the registers: loaded after it, each value guarded.
+    constexpr bool kEarly = sizeof(T) == 4;
+    RowFlux<C, T> f;
+    T nsum = T(0);
+    if constexpr (RHS && kEarly) nsum = flux_load<false, P2>(B, t, s, air, j, i0, f);
 
-    bool bW = is_broken(gW, eW, gmax), bE = is_broken(gE, eE, gmax);
-    bool bN[C], bS[C];
-    double e[C], g[C];
+    static_assert(kThresh == 0.0, "the smallest |eta| stands for eta == kThresh");
+    T gm = tmax(q.x0Wv, q.x0Ev), em = tmin(tabs(eW), tabs(eE));
+    T lo = tabs(gv[0]), hi = lo;
 #pragma unroll
     for (int k = 0; k < C; ++k) {
-        e[k] = (double)ev[k];
-        g[k] = (double)gv[k];
-        q.brk[k] = is_broken(g[k], e[k], gmax);
-        bN[k] = hasN && is_broken((double)gNv[k], (double)eNv[k], gmax);
-        bS[k] = hasS && is_broken((double)gSv[k], (double)eSv[k], gmax);
+        gm = tmax(gm, tmax(gv[k], tmax(q.x0Nv[k], q.x0Sv[k])));
+        em = tmin(em, tmin(tabs(ev[k]), tmin(tabs(eNv[k]), tabs(eSv[k]))));
+        lo = tmin(lo, tabs(gv[k]));
+        hi = tmax(hi, tabs(gv[k]));
     }
+    const bool rare = __any((double)gm > gmax - kEps || em == T(0) || !((double)lo >= 1e-300) ||
+                            !((double)hi <= 1e300) || !__builtin_isfinite(nsum));
+    q.brk = 0;
+    q.gmax = gmax;
+    if (__builtin_expect(rare, 0)) {
+        decltype(q.brk) b = 0;
+#pragma unroll
+        for (int k = 0; k < C; ++k) {
+            b |= (decltype(q.brk))is_broken((double)gv[k], (double)ev[k], gmax) << k;
+            b |= (decltype(q.brk))(hasN && is_broken((double)q.x0Nv[k], (double)eNv[k], gmax)) << (C + k);
+            b |= (decltype(q.brk))(hasS && is_broken((double)q.x0Sv[k], (double)eSv[k], gmax)) << (2 * C + k);
+        }
+        b |= (decltype(q.brk))is_broken((double)q.x0Wv, (double)eW, gmax) << (3 * C);
+        b |= (decltype(q.brk))is_broken((double)q.x0Ev, (double)eE, gmax) << (3 * C + 1);
+        q.brk = b;
+        if constexpr (RHS && kEarly) {
+            int ig = i0;
+            asm volatile("" : "+v"(ig));   // loads of its own: none is kept in registers for it
+            flux_load<true, P2>(B, t, s, air, j, ig, f);
+        }
+    }
+    if constexpr (RHS && !kEarly) flux_load<true, P2>(B, t, s, air, j, i0, f);
+
     // the initial iterate: Gamma* plus the guess, rounded to the state
     // precision (its residual is evaluated exactly below, so the rounding
     // only perturbs the guess)
-    T gxv[C];
 #pragma unroll
-    for (int k = 0; k < C; ++k) gxv[k] = gv[k];
+    for (int k = 0; k < C; ++k) q.x0v[k] = gv[k];
     if (guess) {
         T gc[C];
         ld_row<C>(guess + row + i0, gc);
 #pragma unroll
-        for (int k = 0; k < C; ++k) gxv[k] = gv[k] + gc[k];
+        for (int k = 0; k < C; ++k) q.x0v[k] = gv[k] + gc[k];
         ld_row_wrap<C, P2>(guess + rowN, iNS, nph, m, gc);
 #pragma unroll
-        for (int k = 0; k < C; ++k) gNv[k] = gNv[k] + gc[k];
+        for (int k = 0; k < C; ++k) q.x0Nv[k] += gc[k];
         ld_row_wrap<C, P2>(guess + rowS, iSS, nph, m, gc);
 #pragma unroll
-        for (int k = 0; k < C; ++k) gSv[k] = gSv[k] + gc[k];
-        gW = (double)(T)(gW + (double)guess[row + iWc]);
-        gE = (double)(T)(gE + (double)guess[row + iEc]);
+        for (int k = 0; k < C; ++k) q.x0Sv[k] += gc[k];
+        q.x0Wv += guess[row + iWc];
+        q.x0Ev += guess[row + iEc];
     }
+    auto brk = [&](int bit) { return (q.brk >> bit & 1) != 0; };
+    if (__builtin_expect(rare, 0)) {
+#pragma unroll
+        for (int k = 0; k < C; ++k) {
+            if (brk(C + k)) q.x0Nv[k] = (T)gmax;
+            if (brk(2 * C + k)) q.x0Sv[k] = (T)gmax;
+            if (brk(k)) q.x0v[k] = (T)gmax;
+        }
+        if (brk(3 * C)) q.x0Wv = (T)gmax;
+        if (brk(3 * C + 1)) q.x0Ev = (T)gmax;
+    }
+
+    const double dt = B.dt, CrDt = B.cr_dt, s2M = B.w_scale;
+    const double sinN = tab.sinFace[B.rt0 + j], sinS = tab.sinFace[B.rt0 + j + 1];
+    const double sdt = tab.sinTc[B.rt0 + j] * B.inv_dt, cW = s2M * tab.cscTc[B.rt0 + j];
     // Every face term of concentrationLinearSystemKernel has the factor
-    // 1 / (eta_f + Cr dt): the weight s2 sin M dt / (eta_f + Cr dt), the
-    // film term u eta_f / (eta_f + Cr dt), the air term u_air / (eta_f / Cr
-    // / dt + 1) = u_air Cr dt / (eta_f + Cr dt) and the gravity term
-    // eta_f / (eta_f / dt + Cr) = eta_f dt / (eta_f + Cr dt). One reciprocal
-    // per face serves all of them (a few ulp from the reference's divisions).
+    // 1 / (eta_f + Cr dt): the weight s2 sin M dt / (eta_f + Cr dt), the film
+    // term u eta_f / (eta_f + Cr dt), the air term u_air / (eta_f / Cr / dt
+    // + 1) = u_air Cr dt / (eta_f + Cr dt) and the force term eta_f f /
+    // (eta_f / dt + Cr) = eta_f f dt / (eta_f + Cr dt). One reciprocal per
+    // face serves all of them, and the three fluxes are one product,
+    // (eta_f (u + f dt) + Cr dt u_air) / (eta_f + Cr dt) (a few ulp from the
+    // reference's divisions).
     // phi faces: face k lies between cells k-1 and k
-    double wFr[C + 1], etaF[C + 1], invF[C + 1];
+    double fF[C + 1];
 #pragma unroll
     for (int k = 0; k <= C; ++k) {
-        const double l = k == 0 ? eW : e[k - 1];
-        const double r = k == C ? eE : e[k];
-        etaF[k] = (l + r) / 2.0;
-        invF[k] = rcp64(etaF[k] + CrDt);
-        wFr[k] = cW * invF[k];
-        const bool bl = k == 0 ? bW : q.brk[k - 1];
-        const bool br = k == C ? bE : q.brk[k];
-        q.wF[k] = (bl || br) ? 0.0 : wFr[k];
-    }
-    T uv[C + 1], vNv[C], vSv[C];            // the film velocities (state precision)
-    T uAirF[C + 1], vAirNv[C], vAirSv[C];   // the blended air (state precision)
-#pragma unroll
-    for (int k = 0; k < C; ++k) vAirNv[k] = vAirSv[k] = T(0);
-    const double kt = 3.0 - fabs(t - 3.0);
-    const double bl = t / 12.0;
-    if (RHS) {
-        T u[C], vn[C], vs[C];
-        ld_row<C>(s.uph + row + i0, u);
-#pragma unroll
-        for (int k = 0; k < C; ++k) { uv[k] = u[k]; vNv[k] = vSv[k] = T(0); }
-        uv[C] = s.uph[row + iEc];
-        if (hasN) {
-            ld_row<C>(s.uth + row - nph + i0, vn);
-#pragma unroll
-            for (int k = 0; k < C; ++k) vNv[k] = vn[k];
-        }
-        if (hasS) {
-            ld_row<C>(s.uth + row + i0, vs);
-#pragma unroll
-            for (int k = 0; k < C; ++k) vSv[k] = vs[k];
-        }
-        if (B.airflow) {
-            // per phi face, shared by the two cells of the face; v at the
-            // north and south faces of the cells. FP32 fields: row vectors;
-            // FP64 fields (twice the registers) per column.
-            if constexpr (sizeof(T) == 4) {
-                const float ktf = (float)kt, blf = (float)bl;
-                air_blend<C, C + 1, false, P2>(air.ua0, air.au, row, i0, nph, m, ktf, blf, uAirF);
-                if (hasN)
-                    air_blend<C, C, true, P2>(air.va0, air.av, row - nph, i0, nph, m, ktf, blf, vAirNv);
-                if (hasS) air_blend<C, C, true, P2>(air.va0, air.av, row, i0, nph, m, ktf, blf, vAirSv);
-            } else {
-#pragma unroll
-                for (int k = 0; k <= C; ++k) {
-                    const int i = wrap_t<P2>(i0 + k, nph, m), opp = wrap_t<P2>(nph - i, nph, m);
-                    uAirF[k] = 0.5 * (air_at(air.ua0, air.au, row + i, kt) * bl +
-                                      air_at(air.ua0, air.au, row + opp, kt) * (1 - bl));
-                }
-            }
-        }
-    }
-#pragma unroll
-    for (int k = 0; k < C; ++k) {
-        const double eN = (double)eNv[k], eS = (double)eSv[k];
-        const double etaUp = (eN + e[k]) / 2.0, etaDown = (eS + e[k]) / 2.0;
-        const double etaLeft = etaF[k], etaRight = etaF[k + 1];
-        const double invU = rcp64(etaUp + CrDt), invD = rcp64(etaDown + CrDt);
-        const double invL = invF[k], invR = invF[k + 1];
-        const double wN = cN * invU;
-        const double wS = cS * invD;
-        const double wW = wFr[k], wE = wFr[k + 1];
-        const bool brk = q.brk[k];
-        q.wN[k] = (brk || bN[k]) ? 0.0 : wN;
-        q.wS[k] = (brk || bS[k]) ? 0.0 : wS;
-        q.x0v[k] = gxv[k];
-        q.x0Nv[k] = gNv[k];
-        q.x0Sv[k] = gSv[k];
-        q.bN[k] = bN[k];
-        q.bS[k] = bS[k];
-        q.rhs[k] = 0.0;
-        if (brk) {
-            q.diag[k] = 1.0;
-            q.rhs[k] = gmax;
-            continue;
-        }
-        q.diag[k] = qdiv(sinTheta * invDt, g[k]) - (((-wN) + (-wW)) + (-wE) + (-wS));
-        if (!RHS) continue;
-        const int i = i0 + k;
-        double uW = (double)uv[k], uE = (double)uv[k + 1], vN = (double)vNv[k], vS = (double)vSv[k];
-        if (__builtin_isnan(vN)) vN = 0.0;
-        if (__builtin_isnan(vS)) vS = 0.0;
-        if (__builtin_isnan(uW)) uW = 0.0;
-        if (__builtin_isnan(uE)) uE = 0.0;
-        double div = B.invh * (uE * etaRight * invR - uW * etaLeft * invL +
-                               (vS * sinS * etaDown * invD - vN * sinN * etaUp * invU));
-        if (B.airflow) {
-            double vAirN = (double)vAirNv[k], vAirS = (double)vAirSv[k];
-            if constexpr (sizeof(T) != 4) {
-                const int opp = wrap_t<P2>(nph - i, nph, m);
-                if (hasN) {
-                    const size_t rn = row - nph;
-                    vAirN = 0.5 * (air_at(air.va0, air.av, rn + i, kt) * bl -
-                                   air_at(air.va0, air.av, rn + opp, kt) * (1 - bl));
-                }
-                if (hasS) {
-                    vAirS = 0.5 * (air_at(air.va0, air.av, row + i, kt) * bl -
-                                   air_at(air.va0, air.av, row + opp, kt) * (1 - bl));
-                }
-            }
-            div += B.invh * CrDt *
-                   ((double)uAirF[k + 1] * invR - (double)uAirF[k] * invL + vAirS * sinS * invD -
-                    vAirN * sinN * invU);
-        }
-        if (VISC && B.gravity) {
+        const double sum = (double)(k == 0 ? eW : ev[k - 1]) + (double)(k == C ? eE : ev[k]);
+        const double inv = rcp64(fma(sum, 0.5, CrDt));
+        q.wF[k] = cW * inv;
+        if constexpr (RHS) {
+            double u = (double)f.u[k];
             // `gravity` with `VISCOUS` (bubble.cu:1458-1464): the viscous
             // forces in place of the gravity term
-            const size_t cc = row + i;
-            const double fuW = air.fu[cc], fuE = air.fu[row + wrap_t<P2>(i + 1, nph, m)];
-            const double fvN = hasN ? air.fv[cc - nph] : 0.0;
-            const double fvS = hasS ? air.fv[cc] : 0.0;
-            div += B.invh * dt *
-                   (sinS * fvS * etaDown * invD - sinN * fvN * etaUp * invU +
-                    fuE * etaRight * invR - fuW * etaLeft * invL);
-        } else if (B.gravity) {
-            div += B.gs * B.invh * dt *
-                   (sinS * sinS * etaDown * invD - sinN * sinN * etaUp * invU);
+            if (VISC && B.gravity) u = fma(dt, (double)air.fu[row + wrap_t<P2>(i0 + k, nph, m)], u);
+            fF[k] = inv * fma(0.5 * sum, u, CrDt * (double)f.ua[k]);
         }
-        double rr = sinTheta * invDt - div;
-        if (bN[k]) rr += wN * gmax;
-        if (bS[k]) rr += wS * gmax;
-        if (k == 0 ? bW : q.brk[k - 1]) rr += wW * gmax;
-        if (k == C - 1 ? bE : q.brk[k + 1]) rr += wE * gmax;
-        q.rhs[k] = rr;
     }
-    q.x0Wv = (T)gW;
-    q.x0Ev = (T)gE;
-    q.bW = bW;
-    q.bE = bE;
-    q.gmax = gmax;
+    const double gN = !VISC && B.gravity ? B.gs * dt * sinN : 0.0;
+    const double gS = !VISC && B.gravity ? B.gs * dt * sinS : 0.0;
+#pragma unroll
+    for (int k = 0; k < C; ++k) {
+        const double e = (double)ev[k];
+        const double sumN = (double)eNv[k] + e, sumS = (double)eSv[k] + e;
+        const double pN = sinN * rcp64(fma(sumN, 0.5, CrDt)), pS = sinS * rcp64(fma(sumS, 0.5, CrDt));
+        q.wN[k] = s2M * pN;
+        q.wS[k] = s2M * pS;
+        q.diag[k] = fma(sdt, rcp64((double)gv[k]), (q.wN[k] + q.wS[k]) + (q.wF[k] + q.wF[k + 1]));
+        q.rhs[k] = 0.0;
+        if constexpr (RHS) {
+            double vN = (double)f.vN[k] + gN, vS = (double)f.vS[k] + gS;
+            if (VISC && B.gravity) {
+                const size_t cc = row + i0 + k;
+                if (hasN) vN = fma(dt, (double)air.fv[cc - nph], vN);
+                if (hasS) vS = fma(dt, (double)air.fv[cc], vS);
+            }
+            const double fN = pN * fma(0.5 * sumN, vN, CrDt * (double)f.vaN[k]);
+            const double fS = pS * fma(0.5 * sumS, vS, CrDt * (double)f.vaS[k]);
+            q.rhs[k] = fma(-B.invh, (fF[k + 1] - fF[k]) + (fS - fN), sdt);
+            // formed here, where the iterate's registers end
+            const double xl = k == 0 ? q.x0W() : (double)q.x0v[k - 1];
+            const double xr = k == C - 1 ? q.x0E() : (double)q.x0v[k + 1];
+            double r0 = fma(-q.diag[k], (double)q.x0v[k], q.rhs[k]);
+            r0 = fma(q.wN[k], q.x0N(k), r0);
+            r0 = fma(q.wS[k], q.x0S(k), r0);
+            r0 = fma(q.wF[k], xl, r0);
+            q.r0[k] = fma(q.wF[k + 1], xr, r0);
+        }
+    }
+    if (__builtin_expect(rare, 0)) {
+        // a concentration out of the reciprocal's range; a broken cell: an
+        // identity row with rhs gamma_max, its coupling to the cells beside
+        // it moved to their right-hand sides
+        int ig = i0;
+        asm volatile("" : "+v"(ig));
+        const double gT = (double)(T)gmax;   // the iterate on a broken cell, as above
+        double w0 = q.wF[0];
+        if (brk(3 * C) || brk(0)) q.wF[0] = 0.0;
+#pragma unroll
+        for (int k = 0; k < C; ++k) {
+            const double g = (double)s.gam[row + ig + k], ag = fabs(g), w1 = q.wF[k + 1];
+            const int bl = k == 0 ? 3 * C : k - 1, br = k == C - 1 ? 3 * C + 1 : k + 1;
+            if (!(ag >= 1e-300 && ag <= 1e300)) {
+                q.diag[k] = sdt / g + ((q.wN[k] + q.wS[k]) + (w0 + w1));
+                if constexpr (RHS) {
+                    auto x = [&](size_t c) { return (double)(guess ? s.gam[c] + guess[c] : s.gam[c]); };
+                    double r0 = fma(-q.diag[k], x(row + ig + k), q.rhs[k]);
+                    r0 = fma(q.wN[k], brk(C + k) ? gT : x(rowN + wrap_t<P2>(iNS + k, nph, m)), r0);
+                    r0 = fma(q.wS[k], brk(2 * C + k) ? gT : x(rowS + wrap_t<P2>(iSS + k, nph, m)), r0);
+                    r0 = fma(w0, brk(bl) ? gT : x(row + wrap_t<P2>(ig + k - 1, nph, m)), r0);
+                    q.r0[k] = fma(w1, brk(br) ? gT : x(row + wrap_t<P2>(ig + k + 1, nph, m)), r0);
+                }
+            }
+            if constexpr (RHS) {
+                auto move = [&](int bit, double w) {
+                    if (!brk(bit)) return;
+                    q.rhs[k] = fma(w, gmax, q.rhs[k]);
+                    q.r0[k] = fma(w, gmax - gT, q.r0[k]);
+                };
+                move(C + k, q.wN[k]);
+                move(2 * C + k, q.wS[k]);
+                move(bl, w0);
+                move(br, w1);
+                if (brk(k)) q.r0[k] = 0.0;
+            }
+            if (brk(k)) {
+                q.diag[k] = 1.0;
+                q.rhs[k] = gmax;
+            }
+            if (brk(k) || brk(C + k)) q.wN[k] = 0.0;
+            if (brk(k) || brk(2 * C + k)) q.wS[k] = 0.0;
+            if (brk(k) || brk(br)) q.wF[k + 1] = 0.0;
+            w0 = w1;
+        }
+    }
 }
 
 // Periodic phi-line solve of one row, normalised to unit diagonal
@@ -841,26 +927,22 @@ __global__ void k_assemble(const int2* __restrict__ rows, const BubbleDev* __res
 #pragma unroll
     for (int k = 0; k < C; ++k) a[k] = cc[k] = d[k] = rin[k] = Ti(0);
     if (act) {
-        RowSys<C, T> q;
         // the extrapolated correction once a previous solve stored one
+        RowSys<C, T> q;
         row_system<T, C, true, VISC, P2>(B, t, tab, s, air, j, i0, q,
-                                     btime[rw.x].ghist > 0 ? guess : nullptr);
+                                         btime[rw.x].ghist > 0 ? guess : nullptr);
         Ti wn[C], ww[C], dg[C];
 #pragma unroll
         for (int k = 0; k < C; ++k) {
             const double wW = q.wF[k], wE = q.wF[k + 1];
-            const double xl = k == 0 ? q.x0W() : q.x0(k - 1);
-            const double xr = k == C - 1 ? q.x0E() : q.x0(k + 1);
-            const double ax = q.diag[k] * q.x0(k) - q.wN[k] * q.x0N(k) - q.wS[k] * q.x0S(k) -
-                              wW * xl - wE * xr;
-            const double r0 = q.rhs[k] - ax;
+            const double r0 = q.r0[k];
             // x^T N x <= sum (wN + wS) x_i^2 and x^T M x >= sum (diag - wW - wE)
             // x_i^2 for the theta couplings N and the phi-line blocks M, so
             // the eigenvalues of M^-1 A lie in [1 - mu, 1 + mu] with mu the
             // largest ratio below
-            // (a bound with a 2 % margin downstream: FP32 is ample)
-            if (!q.brk[k])
-                muf = fmaxf(muf, (float)(q.wN[k] + q.wS[k]) *
+            // (a bound with a 2 % margin downstream: FP32 is ample; zero on a
+            // broken cell, whose weights are)
+            muf = fmaxf(muf, (float)(q.wN[k] + q.wS[k]) *
                                      __builtin_amdgcn_rcpf((float)(q.diag[k] - wW - wE)));
             rin[k] = (Ti)r0;
             wn[k] = (Ti)q.wN[k];
@@ -870,9 +952,9 @@ __global__ void k_assemble(const int2* __restrict__ rows, const BubbleDev* __res
             a[k] = -ww[k] * inv;
             cc[k] = -(Ti)wE * inv;
             d[k] = rin[k] * inv;
-            acc[0] += r0 * r0;
-            acc[1] += q.rhs[k] * q.rhs[k];
-            acc[3] += (double)rin[k] * (double)rin[k];
+            acc[0] = fma(r0, r0, acc[0]);
+            acc[1] = fma(q.rhs[k], q.rhs[k], acc[1]);
+            acc[3] = fma((double)rin[k], (double)rin[k], acc[3]);
         }
         st_row<C>(sys.b64 + row + i0, q.rhs);
         st_row<C>(sys.wN + row + i0, wn);
@@ -1096,10 +1178,10 @@ __global__ void k_resid(const int2* __restrict__ rows, const BubbleDev* __restri
     for (int q = 0; q < C; ++q) a[q] = cc[q] = d[q] = rin[q] = Ti(0);
     if (act) {
         double xc[C], xN[C], xS[C], xW, xE;
+        const T* __restrict__ gs = FIRST && btime[rw.x].ghist > 0 ? guess : nullptr;
         RowSys<C, T> w;
+        row_system<T, C, false, false, P2>(B, 0.0, tab, s, AirPtrs<T>{}, j, i0, w, gs);
         if constexpr (FIRST) {
-            row_system<T, C, false, false, P2>(B, 0.0, tab, s, AirPtrs<T>{}, j, i0, w,
-                                    btime[rw.x].ghist > 0 ? guess : nullptr);
 #pragma unroll
             for (int q = 0; q < C; ++q) {
                 xc[q] = w.x0(q);
@@ -1110,7 +1192,6 @@ __global__ void k_resid(const int2* __restrict__ rows, const BubbleDev* __restri
             xE = w.x0E();
         } else {
             ld_stencil<double, C>(xo, row, i0, m, nph, hasN, hasS, xc, xW, xE, xN, xS);
-            row_system<T, C, false, false, P2>(B, 0.0, tab, s, AirPtrs<T>{}, j, i0, w);
         }
         if constexpr (!ZP) ld_stencil<Ti, C>(ecorr, row, i0, m, nph, hasN, hasS, ec, eW, eE, eN, eS);
         double bv[C];
@@ -1123,14 +1204,15 @@ __global__ void k_resid(const int2* __restrict__ rows, const BubbleDev* __restri
         for (int q = 0; q < C; ++q) {
             const double l = q == 0 ? xWn : xnew[q - 1];
             const double r = q == C - 1 ? xEn : xnew[q + 1];
-            double ax = w.diag[q] * xnew[q] - w.wF[q] * l - w.wF[q + 1] * r;
-            if (hasN) ax -= w.wN[q] * (xN[q] + (double)eN[q]);
-            if (hasS) ax -= w.wS[q] * (xS[q] + (double)eS[q]);
-            const double res = bv[q] - ax;
+            double res = fma(-w.diag[q], xnew[q], bv[q]);
+            res = fma(w.wF[q], l, res);
+            res = fma(w.wF[q + 1], r, res);
+            if (hasN) res = fma(w.wN[q], xN[q] + (double)eN[q], res);
+            if (hasS) res = fma(w.wS[q], xS[q] + (double)eS[q], res);
             rin[q] = (Ti)res;
-            acc[0] += res * res;
-            acc[1] += bv[q] * bv[q];
-            acc[3] += (double)rin[q] * (double)rin[q];
+            acc[0] = fma(res, res, acc[0]);
+            acc[1] = fma(bv[q], bv[q], acc[1]);
+            acc[3] = fma((double)rin[q], (double)rin[q], acc[3]);
         }
         st_row<C>(xn + row + i0, xnew);
         if constexpr (!ZP) st_row<C>(sys.r + row + i0, rin);
