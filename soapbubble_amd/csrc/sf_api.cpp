@@ -202,6 +202,9 @@ struct Base {
     long stride = 0;          // partial-sum stride (rows)
     hipStream_t stream = nullptr;
     std::vector<void*> owned;
+    std::vector<void*> sp_owned;   // the spectral preconditioner's, given back when multigrid takes over
+    // test hook: parts of the solver whose lazy allocation fails
+    std::string fail_alloc = std::getenv("SF_FAIL_ALLOC") ? std::getenv("SF_FAIL_ALLOC") : "";
     BubbleDev* bub_d = nullptr;
     BubbleTime* time_d = nullptr;
     SolveCtl* ctl_d = nullptr;
@@ -305,7 +308,26 @@ struct Base {
         if (stage_h) (void)hipHostFree(stage_h);
         if (cstream) (void)hipStreamDestroy(cstream);
         for (void* p : owned) (void)hipFree(p);
+        for (void* p : sp_owned) (void)hipFree(p);
         if (stream && !noalloc) (void)hipStreamDestroy(stream);
+    }
+    // Lazily allocated arrays of one part of the solver, all of them or none:
+    // `build` collects what it allocates, which goes to `keep` when it
+    // returns and is freed when it throws.
+    template <typename F>
+    void all_or_none(const char* part, std::vector<void*>& keep, F&& build) {
+        std::vector<void*> got;
+        try {
+            build(got);
+            if (fail_alloc.find(part) != std::string::npos)
+                throw Status{SF_ERR_NOMEM, std::string("no memory for ") + part};
+            keep.insert(keep.end(), got.begin(), got.end());
+        } catch (...) {
+            (void)hipStreamSynchronize(stream);
+            for (void* p : got) (void)hipFree(p);
+            (void)hipGetLastError();
+            throw;
+        }
     }
     virtual void advect() = 0;
     // applies what uploads left pending (BIMOCQ's maps and initial fields
@@ -385,7 +407,7 @@ struct Impl : Base {
     }
     bool fp64_inner() const override { return sizeof(Ti) == 8; }
     void enable_mg() override {
-        if (mgp.empty()) alloc_mg();
+        need_mg();
         mg = true;
         spectral = false;
         method = 1;
@@ -399,18 +421,18 @@ struct Impl : Base {
         int nfwd = 0, nline = 0, threads = 0;
         size_t lds = 0;
     };
-    std::vector<SpLaunch> spl;
-    SpPtrs spp{};
-    void alloc_spectral() {
+    std::vector<SpLaunch> spl;   // empty until the bases are there
+    SpPtrs spp{};                // null until allocated
+    void alloc_spectral(std::vector<void*>& own, std::vector<SpLaunch>& launches, SpPtrs& ptrs) {
         std::vector<SpDev> dev(nb);
         long long tot = 0;
-        spl.assign(rgeo.size(), SpLaunch{});
+        launches.assign(rgeo.size(), SpLaunch{});
         for (size_t w = 0; w < rgeo.size(); ++w) {
             const int nph = rgeo_nph[w], n = nph / 2;
             int R = 4;
             while (R * kSpCells < n) R *= 2;
             const int npad = R * kSpCells, wv = (R + 63) / 64 * 64;
-            SpLaunch& L = spl[w];
+            SpLaunch& L = launches[w];
             // at least two modes a block, so the blocks of a bubble are at
             // most its rows (the r.z slots)
             L.threads = std::max(256, 2 * wv);
@@ -423,12 +445,12 @@ struct Impl : Base {
                 const double q = std::sin(kPi * ((m + 1) / 2) / nph);
                 lam[m] = (float)(4.0 * q * q);
             }
-            double* cs_d = dalloc<double>(cs.size(), owned);
+            double* cs_d = dalloc<double>(cs.size(), own);
             SF_HIP(hipMemcpy(cs_d, cs.data(), cs.size() * sizeof(double), hipMemcpyHostToDevice));
-            float* lam_d = dalloc<float>(lam.size(), owned);
+            float* lam_d = dalloc<float>(lam.size(), own);
             SF_HIP(hipMemcpy(lam_d, lam.data(), lam.size() * sizeof(float), hipMemcpyHostToDevice));
-            float* Qt = dalloc<float>((size_t)nph * nph, owned);
-            float* Q = dalloc<float>((size_t)nph * nph, owned);
+            float* Qt = dalloc<float>((size_t)nph * nph, own);
+            float* Q = dalloc<float>((size_t)nph * nph, own);
             launch_sp_basis(stream, nph, cs_d, Qt, Q);
             std::vector<int4> fwd, line;
             for (int b = 0; b < nb; ++b) {
@@ -441,17 +463,23 @@ struct Impl : Base {
             }
             auto up = [&](const std::vector<int4>& v, int4*& p, int& k) {
                 k = (int)v.size();
-                p = dalloc<int4>(v.size(), owned);
+                p = dalloc<int4>(v.size(), own);
                 SF_HIP(hipMemcpy(p, v.data(), v.size() * sizeof(int4), hipMemcpyHostToDevice));
             };
             up(fwd, L.fwd, L.nfwd);
             up(line, L.line, L.nline);
         }
-        SpDev* d = dalloc<SpDev>(nb, owned);
+        SpDev* d = dalloc<SpDev>(nb, own);
         SF_HIP(hipMemcpy(d, dev.data(), nb * sizeof(SpDev), hipMemcpyHostToDevice));
-        spp.d = d;
-        spp.Y = dalloc<float>((size_t)tot, owned);
-        spp.coef = dalloc<float>(5 * (size_t)stride, owned);
+        ptrs.d = d;
+        ptrs.Y = dalloc<float>((size_t)tot, own);
+    }
+    void free_spectral() {
+        SF_HIP(hipStreamSynchronize(stream));
+        for (void* p : sp_owned) (void)hipFree(p);
+        sp_owned.clear();
+        spl.clear();
+        spp = SpPtrs{};
     }
     // The row-constant operator of the assembled system.
     void sp_coef() {
@@ -496,9 +524,38 @@ struct Impl : Base {
         if (sizeof(Ti) != 4) return false;
         for (int b = 0; b < nb; ++b)
             if (bub_h[b].nth > kSpMaxTheta) return false;
-        if (spl.empty()) alloc_spectral();
-        sp_coef();
-        if (!(sp_condition() <= kSpMaxCondition)) return false;
+        // first the row-constant operator alone, which tells whether the
+        // preconditioner serves; its bases (two n_phi x n_phi matrices per row
+        // width, 134 MB at 4096 columns) only then. Without memory for them
+        // multigrid, which needs less at that size, takes over.
+        try {
+            if (!spp.coef) {
+                float* coef = nullptr;
+                all_or_none("coefficients", sp_owned, [&](std::vector<void*>& own) {
+                    coef = dalloc<float>(5 * (size_t)stride, own);
+                });
+                spp.coef = coef;
+            }
+            sp_coef();
+            if (sp_condition() <= kSpMaxCondition) {
+                if (spl.empty()) {
+                    std::vector<SpLaunch> launches;
+                    SpPtrs ptrs = spp;
+                    all_or_none("spectral", sp_owned, [&](std::vector<void*>& own) {
+                        alloc_spectral(own, launches, ptrs);
+                    });
+                    spl.swap(launches);
+                    spp = ptrs;
+                }
+            } else {
+                free_spectral();
+                return false;
+            }
+        } catch (const Status& s) {
+            if (s.code != SF_ERR_NOMEM) throw;
+            free_spectral();
+            return false;
+        }
         spectral = true;
         mg = false;
         method = 1;
@@ -547,7 +604,20 @@ struct Impl : Base {
         }
     }
 
-    void alloc_mg() {
+    void need_mg() {
+        if (!mgp.empty()) return;
+        int levels = 0;
+        std::vector<MgPtrs<Ti>> ptrs;
+        std::vector<std::vector<MgLaunch>> launches;
+        all_or_none("multigrid", owned, [&](std::vector<void*>& own) {
+            alloc_mg(own, levels, ptrs, launches);
+        });
+        mg_levels = levels;
+        mgp.swap(ptrs);
+        mgl.swap(launches);
+    }
+    void alloc_mg(std::vector<void*>& own, int& levels, std::vector<MgPtrs<Ti>>& ptrs,
+                  std::vector<std::vector<MgLaunch>>& launches) {
         // rows per level of each bubble: halved while the count is even
         std::vector<std::vector<int>> nl(nb);
         for (int b = 0; b < nb; ++b) {
@@ -557,11 +627,11 @@ struct Impl : Base {
                 n /= 2;
                 nl[b].push_back(n);
             }
-            mg_levels = std::max(mg_levels, (int)nl[b].size());
+            levels = std::max(levels, (int)nl[b].size());
         }
-        mgp.assign(mg_levels, MgPtrs<Ti>{});
-        mgl.assign(mg_levels, std::vector<MgLaunch>(rgeo.size()));
-        for (int l = 0; l < mg_levels; ++l) {
+        ptrs.assign(levels, MgPtrs<Ti>{});
+        launches.assign(levels, std::vector<MgLaunch>(rgeo.size()));
+        for (int l = 0; l < levels; ++l) {
             std::vector<MgLevelDev> lv(nb, MgLevelDev{0, 0, 0});
             long long tot = 0;
             for (int b = 0; b < nb; ++b) {
@@ -570,20 +640,20 @@ struct Impl : Base {
                 lv[b].off = l == 0 ? bub_h[b].off : tot;
                 tot += ((long long)nl[b][l] * bub_h[b].nph + 63) / 64 * 64;
             }
-            MgLevelDev* lv_d = dalloc<MgLevelDev>(nb, owned);
+            MgLevelDev* lv_d = dalloc<MgLevelDev>(nb, own);
             SF_HIP(hipMemcpy(lv_d, lv.data(), nb * sizeof(MgLevelDev), hipMemcpyHostToDevice));
-            MgPtrs<Ti>& P = mgp[l];
+            MgPtrs<Ti>& P = ptrs[l];
             P.lv = lv_d;
             if (l == 0) {
                 P.wN = wN; P.wW = wW; P.dg = dg; P.x = z;
             } else {
                 const size_t n = (size_t)tot;
-                P.wN = dalloc<Ti>(n, owned);
-                P.wW = dalloc<Ti>(n, owned);
-                P.dg = dalloc<Ti>(n, owned);
-                P.x = dalloc<Ti>(n, owned);
-                P.U = dalloc<Ti>(n, owned);
-                P.D = dalloc<Ti>(n, owned);
+                P.wN = dalloc<Ti>(n, own);
+                P.wW = dalloc<Ti>(n, own);
+                P.dg = dalloc<Ti>(n, own);
+                P.x = dalloc<Ti>(n, own);
+                P.U = dalloc<Ti>(n, own);
+                P.D = dalloc<Ti>(n, own);
             }
             for (size_t w = 0; w < rgeo.size(); ++w) {
                 std::vector<int2> lists[5];
@@ -595,15 +665,15 @@ struct Impl : Base {
                         lists[4].push_back(make_int2(b, j));
                     }
                 }
-                LaunchGeom* gs[5] = {&mgl[l][w].even, &mgl[l][w].odd, &mgl[l][w].ceven,
-                                     &mgl[l][w].codd, &mgl[l][w].all};
+                MgLaunch& L = launches[l][w];
+                LaunchGeom* gs[5] = {&L.even, &L.odd, &L.ceven, &L.codd, &L.all};
                 for (int k = 0; k < 5; ++k) {
                     *gs[k] = rgeo[w];
                     gs[k]->nrows = 0;
                     gs[k]->rows = nullptr;
                     if (lists[k].empty() || (k == 4 && l == 0)) continue;
                     std::vector<int2> rows = xcd_order(lists[k], make_int2(-1, 0), nxcd);
-                    int2* rows_d = dalloc<int2>(rows.size(), owned);
+                    int2* rows_d = dalloc<int2>(rows.size(), own);
                     SF_HIP(hipMemcpy(rows_d, rows.data(), rows.size() * sizeof(int2),
                                      hipMemcpyHostToDevice));
                     gs[k]->rows = rows_d;
@@ -962,6 +1032,8 @@ struct Impl : Base {
             method_changed = true;
             if (trace_solve) std::fprintf(stderr, "[sf solve] uneven film: multigrid from here on\n");
             enable_mg();
+            // (no executable that was captured with them is launched again)
+            free_spectral();
             mg_coarsen();
             mg_vcycle(true, partR + 2 * stride);
         }
@@ -1274,7 +1346,7 @@ void finish_setup(Impl<T, Ti>& c) {
     c.alloc_fields();
     form_air_shapes(c);
     if (c.bimocq) c.alloc_bimocq();
-    if (c.mg) c.alloc_mg();
+    if (c.mg) c.need_mg();
 }
 
 // The row blocks of one launch over the rows of the widths `ws` (C cells a
