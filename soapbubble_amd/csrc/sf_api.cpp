@@ -279,11 +279,17 @@ struct Base {
     bool mg = false;          // PCG preconditioned by the multigrid V-cycle
     bool spectral = false;    // PCG preconditioned by the row-mean operator
     bool method_changed = false;   // ... since the executable graphs were captured
-    // captured spectral steps watch for a schedule that has become too short,
-    // until a calibration gives the same one again
-    bool sp_watch = true;
+    // captured steps of the automatic method's PCG stand behind a gate
+    // (StepGate): the schedule that let a solve miss its tolerance, the
+    // iterations that the spectral schedules made since have on top of the
+    // calibrated ones, and the chunks for which a miss closes the gate no more
+    // (the host's own solve missed it too)
+    StepGate* gate_d = nullptr;
+    StepGate* gate_h = nullptr;    // pinned copies, by chunk parity
     bool sp_recal = false;         // a state was uploaded: its film sets the rate
     std::vector<int> sp_short;
+    int sp_margin = 1, sp_accept = 0;
+    bool sp_uneven = false;        // the gate closed on an uneven film
     bool trace_solve = std::getenv("SF_SOLVE_TRACE") != nullptr;
     int steps_done = 0;
     int stage = 0;            // 0 idle, 1 advected, 2 assembled, 3 solved
@@ -304,6 +310,7 @@ struct Base {
         for (auto& e : cev)
             if (e) (void)hipEventDestroy(e);
         if (sstat_h) (void)hipHostFree(sstat_h);
+        if (gate_h) (void)hipHostFree(gate_h);
         if (ctl_h) (void)hipHostFree(ctl_h);
         if (stage_h) (void)hipHostFree(stage_h);
         if (cstream) (void)hipStreamDestroy(cstream);
@@ -342,6 +349,15 @@ struct Base {
     // the frame output's binary16 gray plane of bubble b (eta H 2e5)
     virtual void thickness_half(int b, uint16_t* h) = 0;
     virtual void row_stats() = 0;
+    // the gate of captured steps: its hand-off to pinned slot `slot`, its
+    // opening; the automatic method's PCG takes one
+    bool gated() const { return gate_d && auto_method() && method == 1; }
+    void need_gate() {
+        if (!gate_h) SF_HIP(hipHostMalloc((void**)&gate_h, 2 * sizeof(StepGate)));
+        if (!gate_d) gate_d = dalloc<StepGate>(1, owned);
+    }
+    void gate_read(int slot) { launch_gate_read(stream, gate_d, gate_h + slot); }
+    void gate_open() { launch_gate_open(stream, nb, time_d, gate_d, acc, sp_accept > 0 ? 1 : 0); }
     // one inner Chebyshev launch (iteration `it` of refinement `kr`)
     virtual void inner_launch(int it, int kr) = 0;
     // average time of n launches of the advection / of inner iteration 2 of
@@ -1018,6 +1034,7 @@ struct Impl : Base {
             // its operator and first application for this solve, then the
             // PCG branch below
             method_changed = true;
+            need_gate();
             if (try_spectral()) {
                 if (trace_solve) std::fprintf(stderr, "[sf solve] stiff operator: spectral preconditioner\n");
                 sp_apply(true, partR + 2 * stride);
@@ -1027,9 +1044,10 @@ struct Impl : Base {
                 mg_coarsen();
                 mg_vcycle(true, partR + 2 * stride);
             }
-        } else if (host_driven && spectral && !(sp_condition() <= kSpMaxCondition)) {
+        } else if (host_driven && spectral && (sp_uneven || !(sp_condition() <= kSpMaxCondition))) {
             // the film has become too uneven since
             method_changed = true;
+            sp_uneven = false;
             if (trace_solve) std::fprintf(stderr, "[sf solve] uneven film: multigrid from here on\n");
             enable_mg();
             // (no executable that was captured with them is launched again)
@@ -1115,11 +1133,11 @@ struct Impl : Base {
         } else {
             for (size_t k = 0; k < sched.size(); ++k) {
                 for (int it = 0; it < sched[k]; ++it) inner(it, it + 1 == sched[k]);
-                // (statistics of the spare refinement alone, for a schedule
-                // that has become too short)
-                const bool end = k + 1 == sched.size();
-                resid((int)k + 1, e, spectral && end ? sstat_d : nullptr, end);
+                resid((int)k + 1, e, nullptr, k + 1 == sched.size());
             }
+            if (gated())
+                launch_gate(stream, nb, bub_d, time_d, gate_d, spectral ? spp.coef : nullptr, sp, partR,
+                            stride, kSpMaxCondition);
         }
         if (host_driven && method == 1) last_used = used;
         if (host_driven && recording) {
@@ -1847,7 +1865,8 @@ hipGraphExec_t step_graph(Base& c, int nsteps, int slot) {
             c.solve(false, false);
             c.update(true);
         }
-        if (slot >= 0) launch_sched_stats(c.stream, c.sstat_d, c.sstat_h + slot * c.nb, c.nb);
+        if (slot >= 0 && c.gated()) c.gate_read(slot);
+        else if (slot >= 0) launch_sched_stats(c.stream, c.sstat_d, c.sstat_h + slot * c.nb, c.nb);
         e = hipStreamEndCapture(c.stream, &g);
     }
     std::swap(c.stream, c.cstream);
@@ -1873,6 +1892,11 @@ constexpr int kGraphSteps = 4;
 // The cap on a captured schedule (kCaptureMaxInner); the next sf_step after
 // a longer one calibrates again.
 constexpr int kGraphMaxInner = kCaptureMaxInner;
+// The most iterations of margin a refinement of a spectral schedule takes, and
+// the chunks of gated replays that apply solves which miss a tolerance that
+// the host's solve missed too (an unreachable one then costs a host-driven
+// step in 64).
+constexpr int kMaxMargin = 4, kAcceptChunks = 16;
 
 void drop_calibration(Base& c) {
     c.calibrated = false;
@@ -1915,12 +1939,33 @@ bool drop_stale_graphs(Base& c) {
     return true;
 }
 
-// Whether a step of the chunk needed its spare refinement (PCG schedules,
-// which do not adapt: the next steps calibrate again).
-bool spare_ran(const Base& c, const SchedStat* st) {
+// A new film or step size: the gated steps' schedules start afresh.
+void reset_gate(Base& c) {
+    c.sp_short.clear();
+    c.sp_margin = 1;
+    c.sp_accept = 0;
+    c.sp_uneven = false;
+    drop_calibration(c);
+}
+
+// Whether the last step left a solve short of its tolerance, of the bubbles
+// that go on.
+bool solve_missed(Base& c) {
+    std::vector<SolveCtl> v;
+    c.ctl_to_host(v);
+    std::vector<BubbleTime> t((size_t)c.nb);
+    SF_HIP(hipMemcpy(t.data(), c.time_d, t.size() * sizeof(BubbleTime), hipMemcpyDeviceToHost));
     for (int b = 0; b < c.nb; ++b)
-        if (st[b].extra > 0) return true;
+        if (!v[b].converged && (t[b].stop & 3) != 3) return true;
     return false;
+}
+
+// Whether schedule `a` is nowhere longer than `b`.
+bool not_longer(const std::vector<int>& a, const std::vector<int>& b) {
+    if (a.size() > b.size()) return false;
+    for (size_t k = 0; k < a.size(); ++k)
+        if (a[k] > b[k]) return false;
+    return true;
 }
 
 void check_index(sf_ctx* ctx, int b) {
@@ -2220,9 +2265,7 @@ int sf_set_dt(sf_ctx* ctx, int32_t b, double dt_seconds) {
                 // to the old step
                 c.time_h[k].ghist = c.time_h[k].gpend = 0;
                 c.host_hist = 0;
-                c.sp_watch = true;
-                c.sp_short.clear();
-                drop_calibration(c);
+                reset_gate(c);
             }
             set_step(c.bub_h[k], dtn);
             c.time_h[k].dt_s = dt_seconds;
@@ -2255,12 +2298,10 @@ int sf_step(sf_ctx* ctx, int32_t nsteps) {
         }
         if (c.sp_recal) {
             c.sp_recal = false;
-            c.sp_watch = true;
-            c.sp_short.clear();
-            drop_calibration(c);
+            reset_gate(c);
         }
-        // calibration, then replays; once more where the spectral
-        // preconditioner's schedule has become too short on the way
+        // calibration, then replays; once more where the gate of a gated step
+        // closed on the way
         for (bool again = true; again && k < nsteps;) {
             again = false;
             for (int pass = 0; pass < 2 && want_graph && !c.calibrated; ++pass) {
@@ -2274,6 +2315,12 @@ int sf_step(sf_ctx* ctx, int32_t nsteps) {
                     c.recording = false;
                 }
                 (void)drop_stale_graphs(c);
+                // the host's own solve of a step that had missed its tolerance:
+                // where it misses too, the schedule is not at fault
+                if (!c.sp_short.empty() && c.calib_steps == 1 && solve_missed(c)) {
+                    c.sp_accept = kAcceptChunks;
+                    c.sp_short.clear();
+                }
                 if (c.calib_steps == 1) {
                     // schedule: per refinement one inner iteration fewer than the
                     // host-driven step ran (it stopped at the first n whose
@@ -2291,9 +2338,17 @@ int sf_step(sf_ctx* ctx, int32_t nsteps) {
                     // halt_on_failure is set: one more refinement of margin
                     if (c.opt.halt_on_failure) c.sched.push_back(1);
                     // (the spectral preconditioner's rate follows the film: one more
-                    // iteration of margin in each refinement)
-                    if (c.spectral && c.opt.max_inner <= 0)
-                        for (int& n : c.sched) n += 1;
+                    // iteration of margin in each refinement, and another where
+                    // a schedule as long has been too short)
+                    if (c.spectral && c.opt.max_inner <= 0) {
+                        for (int& n : c.sched) n += c.sp_margin;
+                        if (!c.sp_short.empty() && c.sp_margin < kMaxMargin &&
+                            not_longer(c.sched, c.sp_short)) {
+                            c.sp_margin += 1;
+                            for (int& n : c.sched) n += 1;
+                        }
+                    }
+                    c.sp_short.clear();
                     c.sched.push_back(1);
                     if (c.opt.max_outer > 0) c.sched.resize((size_t)c.opt.max_outer, 1);
                     if (c.sched.size() > (size_t)kAccRefine) c.sched.resize(kAccRefine);
@@ -2304,7 +2359,6 @@ int sf_step(sf_ctx* ctx, int32_t nsteps) {
                     // residual launch): one skipped launch per step fewer
                     if (c.method == 2 && c.sched.size() >= 2) c.sched.back() = 0;
                     c.calibrated = true;
-                    if (c.sched == c.sp_short) c.sp_watch = false;
                     if (c.sched[0] > kGraphMaxInner) {
                         drop_calibration(c);
                         // the calibration step switched to multigrid: calibrate
@@ -2318,7 +2372,7 @@ int sf_step(sf_ctx* ctx, int32_t nsteps) {
                     }
                     if (c.calibrated) {
                         const bool adapt = c.method == 2 && c.opt.max_inner <= 0;
-                        (void)step_graph(c, kGraphSteps, -1);
+                        (void)step_graph(c, kGraphSteps, c.gated() ? 0 : -1);
                         if (adapt) {
                             // the graphs of the calibrated schedule and of one
                             // inner iteration fewer (where the schedule usually
@@ -2348,11 +2402,15 @@ int sf_step(sf_ctx* ctx, int32_t nsteps) {
                 // its statistics to the host, which reads them one chunk later,
                 // so the device never waits for the host
                 const bool adapt = c.method == 2 && c.opt.max_inner <= 0;
-                const bool watch = adapt || (c.spectral && c.sp_watch && c.opt.max_inner <= 0);
+                const bool gated = c.gated(), watch = adapt || gated;
                 if (k < nsteps) {
+                    const int k0 = k;
+                    if (gated) c.gate_open();
                     SF_HIP(hipEventRecord(c.ev[0], c.stream));
                     int chunk = 0;
-                    while (k < nsteps && c.sched[0] <= kGraphMaxInner && !again) {
+                    // chunks until misses close the gate again
+                    const int most = gated && c.sp_accept > 0 ? c.sp_accept : nsteps;
+                    while (k < nsteps && c.sched[0] <= kGraphMaxInner && !again && chunk < most) {
                         const int n = std::min(nsteps - k, kAdaptChunk);
                         const int p = chunk & 1;
                         // kGraphSteps steps per launch, the chunk's last launch
@@ -2364,31 +2422,46 @@ int sf_step(sf_ctx* ctx, int32_t nsteps) {
                         }
                         k += n;
                         c.host_hist += n;
+                        ++chunk;
                         if (!watch) continue;
                         SF_HIP(hipEventRecord(c.cev[p], c.stream));
                         c.chunk_sched[p] = c.sched[0];
-                        if (chunk > 0) {
+                        if (chunk > 1) {
                             SF_HIP(hipEventSynchronize(c.cev[p ^ 1]));
-                            const SchedStat* st = c.sstat_h + (p ^ 1) * c.nb;
-                            if (adapt) adapt_schedule(c, st, c.chunk_sched[p ^ 1]);
-                            else again = spare_ran(c, st);
+                            if (adapt) adapt_schedule(c, c.sstat_h + (p ^ 1) * c.nb, c.chunk_sched[p ^ 1]);
+                            else again = c.gate_h[p ^ 1].why != 0;
                         }
-                        ++chunk;
                     }
                     SF_HIP(hipEventRecord(c.ev[5], c.stream));
                     SF_HIP(hipEventSynchronize(c.ev[5]));
-                    if (watch && chunk > 0) {
-                        const int p = (chunk - 1) & 1;
-                        const SchedStat* st = c.sstat_h + p * c.nb;
-                        if (adapt) adapt_schedule(c, st, c.chunk_sched[p]);
-                        else again = again || spare_ran(c, st);
+                    const int p = (chunk - 1) & 1;
+                    if (adapt && chunk > 0) adapt_schedule(c, c.sstat_h + p * c.nb, c.chunk_sched[p]);
+                    if (gated && chunk > 0) {
+                        const StepGate g = c.gate_h[p];
+                        again = g.why != 0;
+                        c.sp_accept = std::max(0, c.sp_accept - chunk);
+                        if (again) {
+                            // the step that closed the gate is the host's
+                            // (a miss) or multigrid's (an uneven film)
+                            c.host_hist -= k - k0 - g.done;
+                            k = k0 + g.done;
+                            c.gate_open();
+                            if (g.why & kGateUneven) c.sp_uneven = true;
+                            else c.sp_short = c.sched;
+                            drop_calibration(c);
+                            if (c.trace_solve)
+                                std::fprintf(stderr, "[sf solve] gate closed after %d steps:%s%s\n",
+                                             g.done, g.why & kGateMissed ? " missed" : "",
+                                             g.why & kGateUneven ? " uneven" : "");
+                        } else {
+                            again = k < nsteps;   // on with the gate as it is from here
+                        }
                     }
                     float ms = 0.f;
                     SF_HIP(hipEventElapsedTime(&ms, c.ev[0], c.ev[5]));
                     c.timing.step_ms += ms;
                 }
-                if (again) c.sp_short = c.sched;
-                if (c.sched[0] > kGraphMaxInner || again) drop_calibration(c);
+                if (c.sched[0] > kGraphMaxInner) drop_calibration(c);
             }
         }
         for (; k < nsteps; ++k) eager_step(c, true);

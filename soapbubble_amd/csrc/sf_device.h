@@ -50,12 +50,17 @@ struct BubbleTime {
     // bit 1 set by the update kernel when this bubble's solve missed its
     // tolerance, bit 2 set by the next step's assembly. Kernels before the
     // assembly skip a bubble with bits 0 and 1, those after it one with bit
-    // 2, so each launch reads a bit that an earlier launch wrote.
+    // 2, so each launch reads a bit that an earlier launch wrote. Bit 3: the
+    // captured steps wait for the host (StepGate); every kernel skips the bubble
+    // until the host has taken the bit back.
     int stop;
 };
+constexpr int kPaused = 8;
 
-__device__ __forceinline__ bool stopped_early(const BubbleTime& t) { return (t.stop & 3) == 3; }
-__device__ __forceinline__ bool stopped(const BubbleTime& t) { return (t.stop & 4) != 0; }
+__device__ __forceinline__ bool stopped_early(const BubbleTime& t) {
+    return (t.stop & 3) == 3 || (t.stop & kPaused);
+}
+__device__ __forceinline__ bool stopped(const BubbleTime& t) { return (t.stop & (4 | kPaused)) != 0; }
 
 // Per-bubble control block of the iterative solve. Every field is written by
 // one kernel (the block of a row launch that arrives last, see arrive_last)
@@ -89,6 +94,19 @@ struct SchedStat {
     int extra;
     int pad_;
 };
+
+// The gate of captured steps in the stiff regime, where the iterations a solve
+// needs rest on the film: before the update of a step, k_gate looks at every
+// bubble's residual and, with the spectral preconditioner, at its condition
+// bound. A step that missed its tolerance or whose film is too uneven is not
+// applied and no later one runs, until the host has taken that step itself.
+struct StepGate {
+    int done;     // steps applied since the host last opened the gate
+    int why;      // kGateMissed, kGateUneven: what closed it (0: open)
+    int accept;   // solves that miss their tolerance are applied
+    int pad_;
+};
+constexpr int kGateMissed = 1, kGateUneven = 2;
 
 struct Tables {
     // per-row, FP64: centres (j+1/2)h, faces j h (advection positions),

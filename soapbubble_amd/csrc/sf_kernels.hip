@@ -903,10 +903,10 @@ __global__ void k_assemble(const int2* __restrict__ rows, const BubbleDev* __res
     if (rw.x < 0) return;
     if (stopped_early(btime[rw.x])) {
         // a bubble stopped by a failed solve: its solve kernels return at
-        // once, its verdict stays the failed one
+        // once, its verdict stays the failed one (or a paused one)
         if (rw.y == 0 && threadIdx.x == 0) {
             flag_store(&ctl[rw.x].outer_done, 1);
-            btime[rw.x].stop |= 4;
+            if ((btime[rw.x].stop & 3) == 3) btime[rw.x].stop |= 4;
         }
         return;
     }
@@ -1854,6 +1854,64 @@ __global__ void k_sp_line(const int4* __restrict__ items, const BubbleDev* __res
     const int blocks = (B.nph + sg.nseg - 1) / sg.nseg;
     for (int k = it.y + (int)threadIdx.x * blocks; k < n; k += (int)blockDim.x * blocks)
         rz_out[B.pr0 + k] = k == it.y ? acc[0] : 0.0;
+}
+
+// The gate of a captured step (StepGate), one block, a wave a bubble; the
+// condition bound (of `coef`, null without one) as the host forms it. A bubble
+// stopped by a failed solve has no say. A launch of its own: the update's
+// blocks need the verdict on all bubbles before the first of them writes.
+__global__ __launch_bounds__(1024) void k_gate(int nb, const BubbleDev* __restrict__ bub,
+                                               BubbleTime* __restrict__ bt,
+                                               StepGate* __restrict__ g,
+                                               const float* __restrict__ coef, SolveParams sp,
+                                               const double* __restrict__ partR, long stride,
+                                               double max_condition) {
+    __shared__ int bad[16];
+    const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6, nw = blockDim.x >> 6;
+    if (g->why) return;
+    const int accept = g->accept;
+    int why = 0;
+    for (int b = wid; b < nb; b += nw) {
+        if ((bt[b].stop & 3) == 3) continue;
+        const long long r0 = bub[b].pr0;
+        double rr = 0.0, bb = 0.0;
+        float hi = 0.0f, lo = 0.0f;
+        for (int j = lane; j < bub[b].nth; j += 64) {
+            rr += partR[r0 + j];
+            bb += partR[stride + r0 + j];
+            if (!coef) continue;
+            hi = fmaxf(hi, coef[3 * stride + r0 + j]);
+            lo = fmaxf(lo, coef[4 * stride + r0 + j]);
+        }
+        rr = wave_sum(rr);
+        bb = wave_sum(bb);
+        hi = wave_max(hi);
+        lo = wave_max(lo);
+        if (!accept && !(residual_norm(rr, bb, sp.absolute) <= sp.tol)) why |= kGateMissed;
+        if (!((double)hi * (double)lo <= max_condition)) why |= kGateUneven;
+    }
+    if (lane == 0) bad[wid] = why;
+    __syncthreads();
+    why = 0;
+    for (int w = 0; w < nw; ++w) why |= bad[w];
+    if (why)
+        for (int b = threadIdx.x; b < nb; b += blockDim.x) bt[b].stop |= kPaused;
+    if (threadIdx.x == 0) {
+        if (why) g->why = why;
+        else g->done += 1;
+    }
+}
+__global__ __launch_bounds__(64) void k_gate_read(const StepGate* __restrict__ d,
+                                                  StepGate* __restrict__ h) {
+    if (threadIdx.x == 0) *h = *d;
+}
+__global__ __launch_bounds__(64) void k_gate_open(BubbleTime* __restrict__ bt,
+                                                  StepGate* __restrict__ g,
+                                                  double* __restrict__ acc, int accept) {
+    const int b = blockIdx.x;
+    acc_zero(acc, b, acc_slot_res(0));
+    if (threadIdx.x == 0) bt[b].stop &= ~kPaused;
+    if (b == 0 && threadIdx.x == 0) *g = StepGate{0, 0, accept, 0};
 }
 
 // ------------------------------------------- inner Chebyshev iteration ----
@@ -2935,6 +2993,18 @@ void launch_sp_line(hipStream_t s, const int4* items, int nitems, int threads, s
                     double* rz_out, long stride) {
     hipLaunchKernelGGL(k_sp_line, dim3(nitems), dim3(threads), lds, s, items, bub, ctl, P, flags,
                        rz_out, stride);
+}
+void launch_gate(hipStream_t s, int nb, const BubbleDev* bub, BubbleTime* bt, StepGate* g,
+                 const float* coef, const SolveParams& sp, const double* partR, long stride,
+                 double max_condition) {
+    hipLaunchKernelGGL(k_gate, dim3(1), dim3(1024), 0, s, nb, bub, bt, g, coef, sp, partR, stride,
+                       max_condition);
+}
+void launch_gate_read(hipStream_t s, const StepGate* d, StepGate* h) {
+    hipLaunchKernelGGL(k_gate_read, dim3(1), dim3(64), 0, s, d, h);
+}
+void launch_gate_open(hipStream_t s, int nb, BubbleTime* bt, StepGate* g, double* acc, int accept) {
+    hipLaunchKernelGGL(k_gate_open, dim3(nb), dim3(64), 0, s, bt, g, acc, accept);
 }
 void launch_sp_basis(hipStream_t s, int nph, const double* cosines, float* Qt, float* Q) {
     hipLaunchKernelGGL(k_sp_basis, dim3(nph), dim3(256), 0, s, nph, cosines, Qt, Q);

@@ -197,6 +197,14 @@ void launch_sp_gemm(hipStream_t s, const int4* items, int nitems, const BubbleDe
 void launch_sp_line(hipStream_t s, const int4* items, int nitems, int threads, size_t lds,
                     const BubbleDev* bub, SolveCtl* ctl, const SpPtrs& P, int flags,
                     double* rz_out, long stride);
+// the gate of a captured step before its update, the hand-off of its state to
+// the host's pinned copy, and the host's opening of it (which also clears the
+// sums that a step not applied left in the assembly's slot)
+void launch_gate(hipStream_t s, int nb, const BubbleDev* bub, BubbleTime* bt, StepGate* g,
+                 const float* coef, const SolveParams& sp, const double* partR, long stride,
+                 double max_condition);
+void launch_gate_read(hipStream_t s, const StepGate* d, StepGate* h);
+void launch_gate_open(hipStream_t s, int nb, BubbleTime* bt, StepGate* g, double* acc, int accept);
 // the basis of rows of nph columns from the cosines cos(2 pi t / nph)
 void launch_sp_basis(hipStream_t s, int nph, const double* cosines, float* Qt, float* Q);
 void launch_finalize(hipStream_t s, int nb, const BubbleDev* bub, SolveCtl* ctl, SolveHist* hist,

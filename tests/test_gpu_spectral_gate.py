@@ -1,0 +1,133 @@
+"""Captured steps of the spectral preconditioner on films that change while they
+are replayed (needs an MI355X): a film that evaporates until it tears, within one
+sf_step call, must be solved as well as by host-driven steps and go to multigrid
+when it is too uneven, whichever parts of the schedule the caller fixes; which
+preconditioner serves which film; and a new film's first chunk, which knows
+nothing of the steps before it."""
+import numpy as np
+import pytest
+
+import soapbubble_amd as sb
+from cases import copy_state, load, make_case
+from conftest import rel_l2
+
+pytestmark = pytest.mark.gpu
+
+# (the velocity of a broken cell may be NaN, which the samplers skip)
+FIELDS = ("eta", "gamma")
+N, DT, RADIUS = 64, 0.02, 0.05
+
+# Replayed and host-driven steps solve to the same tolerance and round FP32
+# fields apart (6e-8); a film that tears multiplies such differences, and cells
+# that break a step earlier or later differ by a step's evaporation (1.5e-3 of
+# 0.3). A solve that misses its tolerance on the torn film leaves tens of percent.
+TOL = 5e-2
+
+
+def thinning_film():
+    """Even but for a dip that evaporation opens after some hundred steps."""
+    st, ua, va = make_case(N, 8, u_scale=0.1)
+    th = (np.arange(N) + 0.5) * np.pi / N
+    ph = np.arange(2 * N) * np.pi / N
+    x = np.sin(th)[:, None] * np.cos(ph)[None]
+    st["eta"] = (0.5 - 0.45 * np.exp(-(1 - x) / 0.05)).ravel()
+    return st, ua, va
+
+
+def thinning_bubble(**kw):
+    return sb.bubble(N, DT, radius=RADIUS, H=4e-7, evaporation=True, **kw)
+
+
+def run(bubbles, cases, steps, graph, **kw):
+    with sb.SoapFilm(bubbles, "mixed", use_graph=graph, **kw) as ctx:
+        for b, c in enumerate(cases):
+            load(ctx, b, *c)
+        ctx.step(steps)
+        return ([ctx.state(b) for b in range(len(cases))],
+                [ctx.stats(b) for b in range(len(cases))])
+
+
+@pytest.mark.parametrize("fixed", [{}, {"max_inner": 20, "max_outer": 3}, {"halt_on_failure": True},
+                                   {"scalar_advection": "bimocq"}])
+def test_a_tearing_film(fixed, monkeypatch, capfd):
+    monkeypatch.setenv("SF_SOLVE_TRACE", "1")
+    film = thinning_film()
+    want, ws = run(thinning_bubble(), [film], 320, False, **fixed)
+    assert ws[0]["failed_solves"] == 0, ws
+    assert "uneven film: multigrid" in capfd.readouterr().err
+    got, gs = run(thinning_bubble(), [film], 320, True, **fixed)
+    err = capfd.readouterr().err
+    assert "spectral preconditioner" in err and "uneven film: multigrid" in err
+    assert gs[0]["failed_solves"] == 0, gs
+    assert gs[0]["steps"] == 320 and abs(gs[0]["time"] - ws[0]["time"]) < 1e-9
+    for k in FIELDS:
+        assert rel_l2(got[0][k], want[0][k]) < TOL, (k, rel_l2(got[0][k], want[0][k]))
+
+
+@pytest.mark.parametrize("fixed", [{"max_outer": 2}, {"tol": 1e-15}])
+def test_a_tearing_film_whose_solves_may_not_converge(fixed, monkeypatch, capfd):
+    """Too few refinements, or a tolerance below the rounding: host-driven solves
+    miss it too, and replayed ones may not be worse off on the torn film."""
+    monkeypatch.setenv("SF_SOLVE_TRACE", "1")
+    film = thinning_film()
+    want, ws = run(thinning_bubble(), [film], 320, False, **fixed)
+    capfd.readouterr()
+    got, gs = run(thinning_bubble(), [film], 320, True, **fixed)
+    assert "uneven film: multigrid" in capfd.readouterr().err
+    assert gs[0]["max_residual"] < 1e-6, gs
+    for k in FIELDS:
+        assert rel_l2(got[0][k], want[0][k]) < TOL, (k, rel_l2(got[0][k], want[0][k]))
+
+
+def test_one_of_several_films_tears():
+    """The films of a context wait together: the even one is as far as the other."""
+    even, torn = make_case(48, 5, u_scale=0.1), thinning_film()
+    bubbles = [sb.bubble(48, 0.025, radius=RADIUS), thinning_bubble()]
+    want, ws = run(bubbles, [even, torn], 320, False)
+    got, gs = run(bubbles, [even, torn], 320, True)
+    for b in range(2):
+        assert gs[b]["failed_solves"] == 0 and ws[b]["failed_solves"] == 0
+        assert abs(gs[b]["time"] - ws[b]["time"]) < 1e-9
+        for k in FIELDS:
+            assert rel_l2(got[b][k], want[b][k]) < TOL, (b, k)
+
+
+@pytest.mark.parametrize("thick,method", [(4.0, "spectral"), (30.0, "multigrid")])
+@pytest.mark.parametrize("graph", [True, False])
+def test_which_preconditioner(graph, thick, method, monkeypatch, capfd):
+    """Either side of the line, from the start and uploaded into a running context."""
+    monkeypatch.setenv("SF_SOLVE_TRACE", "1")
+    even, ua, va = make_case(N, 8, u_scale=0.1)
+    thin = copy_state(even)
+    th = (np.arange(N) + 0.5) * np.pi / N
+    ph = np.arange(2 * N) * np.pi / N
+    w = 0.5 + 0.5 * np.sin(th)[:, None] * np.cos(ph)[None]
+    thin["eta"] = (0.01 + thick * w ** 4).ravel()
+    run(sb.bubble(N, DT, radius=RADIUS), [(thin, ua, va)], 4, graph)
+    err = capfd.readouterr().err
+    assert ("spectral preconditioner" in err) == (method == "spectral")
+    assert ("multigrid" in err) == (method == "multigrid")
+    with sb.SoapFilm(sb.bubble(N, DT, radius=RADIUS), "mixed", use_graph=graph) as ctx:
+        load(ctx, 0, even, ua, va)
+        ctx.step(12)
+        err = capfd.readouterr().err
+        assert "spectral preconditioner" in err and "multigrid" not in err
+        load(ctx, 0, thin, ua, va)
+        ctx.step(9)
+        assert ("uneven film: multigrid" in capfd.readouterr().err) == (method == "multigrid")
+
+
+def test_a_new_film_starts_afresh(monkeypatch, capfd):
+    """A context that runs with fewer refinements than its solves could take, then a
+    new film: one calibration, and no verdict on it from the steps before."""
+    monkeypatch.setenv("SF_SOLVE_TRACE", "1")
+    even, ua, va = make_case(N, 8, u_scale=0.1)
+    with sb.SoapFilm(sb.bubble(N, DT, radius=RADIUS), "mixed", use_graph=True, max_outer=2) as ctx:
+        load(ctx, 0, even, ua, va)
+        ctx.step(40)
+        capfd.readouterr()
+        load(ctx, 0, even, ua, va)
+        ctx.step(10)
+        ctx.step(10)
+        err = capfd.readouterr().err
+    assert err.count("graph schedule:") == 1, err
