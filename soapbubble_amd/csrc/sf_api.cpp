@@ -711,8 +711,9 @@ struct Impl : Base {
     // the start of a refinement (its first launch ends a solve whose FP64
     // residual already meets the tolerance); else inside the inner PCG
     // (launches return once the inner solve is done). The r.z partials of
-    // level 0 go to rz_out.
-    void mg_vcycle(bool start, double* rz_out) {
+    // level 0 go to rz_out. `cold`: z holds no line solve of r (it was another
+    // preconditioner's), the cycle makes its first half-sweep itself.
+    void mg_vcycle(bool start, double* rz_out, bool cold = false) {
         const int nw = (int)rgeo.size();
         std::vector<char> first((size_t)nw, 1);
         auto line = [&](int l, int w, const LaunchGeom& g, int flags) {
@@ -728,12 +729,12 @@ struct Impl : Base {
             for (int w = 0; w < nw; ++w) {
                 const MgLaunch& q = mgl[l][w];
                 const int rz = l == 0 ? kMgRz : 0;
-                if (l > 0) line(l, w, q.even, kMgZeroNb);
+                if (l > 0 || cold) line(l, w, q.even, kMgZeroNb);
                 line(l, w, q.odd, kMgRestrict);
                 // the coarsest level of some bubbles: one row is solved
                 // exactly; more rows take symmetric zebra passes (even, odd,
                 // even, odd, even) from zero
-                if (l > 0) line(l, w, q.ceven, kMgZeroNb | (q.codd.nrows ? 0 : rz));
+                if (l > 0 || cold) line(l, w, q.ceven, kMgZeroNb | (q.codd.nrows ? 0 : rz));
                 if (q.codd.nrows) {
                     line(l, w, q.codd, 0);
                     line(l, w, q.ceven, 0);
@@ -1053,7 +1054,7 @@ struct Impl : Base {
             // (no executable that was captured with them is launched again)
             free_spectral();
             mg_coarsen();
-            mg_vcycle(true, partR + 2 * stride);
+            mg_vcycle(true, partR + 2 * stride, true);
         }
         std::vector<int> used;
         if (method == 2) {

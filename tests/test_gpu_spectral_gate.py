@@ -131,3 +131,29 @@ def test_a_new_film_starts_afresh(monkeypatch, capfd):
         ctx.step(10)
         err = capfd.readouterr().err
     assert err.count("graph schedule:") == 1, err
+
+
+@pytest.mark.parametrize("n", [64, 33])
+def test_the_step_that_hands_over(n, monkeypatch, capfd):
+    """Multigrid's first solve of a film that the spectral preconditioner had taken
+    up to then is as quick as its next ones (rows that halve, and an odd number)."""
+    monkeypatch.setenv("SF_SOLVE_TRACE", "1")
+    even, ua, va = make_case(n, 8, u_scale=0.1)
+    thin = copy_state(even)
+    th = (np.arange(n) + 0.5) * np.pi / n
+    ph = np.arange(2 * n) * np.pi / n
+    w = 0.5 + 0.5 * np.sin(th)[:, None] * np.cos(ph)[None]
+    thin["eta"] = (0.01 + 30.0 * w ** 4).ravel()
+    with sb.SoapFilm(sb.bubble(n, 0.005 * 256 / n, radius=RADIUS), "mixed") as ctx:
+        load(ctx, 0, even, ua, va)
+        ctx.step(3)
+        load(ctx, 0, thin, ua, va)
+        capfd.readouterr()
+        ctx.step(1)
+        first = capfd.readouterr().err
+        ctx.step(1)
+        later = capfd.readouterr().err
+    counts = lambda err: [int(x.split()[-1]) for x in err.splitlines() if "inner iterations" in x]
+    print(f"  n={n}: {counts(first)}, then {counts(later)}", flush=True)
+    assert "uneven film: multigrid" in first
+    assert counts(first)[0] <= 1.5 * counts(later)[0] + 1, (counts(first), counts(later))
