@@ -15,6 +15,7 @@
 #include <cstring>
 #include <map>
 #include <memory>
+#include <mutex>
 #include <string>
 #include <vector>
 
@@ -114,7 +115,49 @@ X* dalloc(size_t n, std::vector<void*>& owned) {
     return static_cast<X*>(p);
 }
 
-constexpr size_t kStageBytes = (size_t)8 << 20;
+// Pinned staging buffers of the downloads, lent for the length of a call, so
+// that calls on one context or on several do not meet in one. Up to kIdle of
+// them wait here for the next call (16 MiB; the rest is freed at once): the
+// first use of a buffer's pages costs the host more than the copies through
+// it (1.7 us a page, 0.5 ms a MiB), which each new context's first download
+// paid when it had a buffer of its own: 512x1024 1.0 ms for that call, 0.14 the
+// next. Never destroyed: at the process's end HIP may have gone first.
+class StagePool {
+    static constexpr size_t kIdle = 2;
+    std::mutex m;
+    std::vector<void*> idle;
+
+public:
+    static constexpr size_t kBytes = (size_t)8 << 20;
+    StagePool() { idle.reserve(kIdle); }
+    void* take() {
+        {
+            std::lock_guard<std::mutex> lock(m);
+            if (!idle.empty()) {
+                void* p = idle.back();
+                idle.pop_back();
+                return p;
+            }
+        }
+        void* p = nullptr;
+        SF_HIP(hipHostMalloc(&p, kBytes, hipHostMallocPortable));
+        return p;
+    }
+    void give(void* p) {
+        {
+            std::lock_guard<std::mutex> lock(m);
+            if (idle.size() < kIdle) {
+                idle.push_back(p);
+                return;
+            }
+        }
+        (void)hipHostFree(p);
+    }
+};
+StagePool& stage_pool() {
+    static StagePool* pool = new StagePool;
+    return *pool;
+}
 
 // The XCD-aware order of the work items of a launch (defined below).
 template <typename X>
@@ -244,7 +287,6 @@ struct Base {
     bool noalloc = false;
     double t_start = 0.0;     // air-flow time the set-up gives the bubbles
     SolveCtl* ctl_h = nullptr;   // pinned copy of the control blocks
-    void* stage_h = nullptr;  // pinned staging buffer of the downloads
     virtual ~Base() {
         if (stream) (void)hipStreamSynchronize(stream);
         for (auto& g : graphs) (void)hipGraphExecDestroy(g.second.exec);
@@ -255,7 +297,6 @@ struct Base {
         if (sstat_h) (void)hipHostFree(sstat_h);
         if (gate_h) (void)hipHostFree(gate_h);
         if (ctl_h) (void)hipHostFree(ctl_h);
-        if (stage_h) (void)hipHostFree(stage_h);
         if (cstream) (void)hipStreamDestroy(cstream);
         for (void* p : owned) (void)hipFree(p);
         for (void* p : sp_owned) (void)hipFree(p);
@@ -1142,16 +1183,19 @@ struct Impl : Base {
         SF_HIP(hipStreamSynchronize(stream));
     }
 
-    // A field to the caller's FP64 array, by way of the context's pinned
-    // staging buffer (kStageBytes a round).
+    // A field to the caller's FP64 array, by way of a pinned staging buffer
+    // (StagePool::kBytes a round).
     template <typename X>
     void fetch(const X* src, size_t off, size_t n, double* h) {
-        if (!stage_h) SF_HIP(hipHostMalloc(&stage_h, kStageBytes));
-        const X* s = static_cast<const X*>(stage_h);
-        const size_t most = kStageBytes / sizeof(X);
+        struct Lent {
+            void* p = stage_pool().take();
+            ~Lent() { stage_pool().give(p); }
+        } stage;
+        const X* s = static_cast<const X*>(stage.p);
+        const size_t most = StagePool::kBytes / sizeof(X);
         for (size_t o = 0; o < n; o += most) {
             const size_t m = std::min(most, n - o);
-            SF_HIP(hipMemcpyAsync(stage_h, src + off + o, m * sizeof(X), hipMemcpyDeviceToHost, stream));
+            SF_HIP(hipMemcpyAsync(stage.p, src + off + o, m * sizeof(X), hipMemcpyDeviceToHost, stream));
             sfh::widen(s, m, h + o, [this] { SF_HIP(hipStreamSynchronize(stream)); });
         }
     }
