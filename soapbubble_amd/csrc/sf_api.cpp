@@ -987,19 +987,19 @@ struct Impl : Base {
         resid((int)k + 1, zp ? nullptr : cheb_e(sched[k] + 1), sstat_d,
               k + 1 == sched.size() || zp_next, zp);
     }
-    // The residual norms of a one-bubble context before and after its first
-    // refinement (one copy: the slots are neighbours), as the tolerance
+    // The residual norms of a one-bubble context before its first and after its
+    // k-th refinement (one copy: the slots are neighbours), as the tolerance
     // takes them.
-    void first_refinement(double& before, double& after) {
+    void refinement_norms(int k, double& before, double& after) {
         const size_t w = (size_t)kAccVals * kAccSub;
-        slot_h.resize(2 * w);
-        SF_HIP(hipMemcpyAsync(slot_h.data(), acc, 2 * w * sizeof(double), hipMemcpyDeviceToHost,
-                              stream));
+        slot_h.resize((size_t)(k + 1) * w);
+        SF_HIP(hipMemcpyAsync(slot_h.data(), acc, slot_h.size() * sizeof(double),
+                              hipMemcpyDeviceToHost, stream));
         SF_HIP(hipStreamSynchronize(stream));
         double v[3] = {0.0, 0.0, 0.0};
         for (int q = 0; q < kAccSub; ++q) {
             v[0] += slot_h[q];
-            v[1] += slot_h[w + q];
+            v[1] += slot_h[k * w + q];
             v[2] += slot_h[kAccSub + q];
         }
         const double bb = sp.absolute ? 1.0 : (v[2] > 0.0 ? std::sqrt(v[2]) : 1.0);
@@ -2116,13 +2116,18 @@ int step_in_scratch(void* scratch, size_t bytes, const sf_options* opt,
         // automatic schedule a first refinement of as many iterations as the
         // residual's fall in the step before asks for comes in front, and
         // the rest is launched only if its residual, read back (15 us),
-        // misses the tolerance: 8 launches a step instead of 36.
+        // misses the tolerance: 8 launches a step instead of 36. Where one as
+        // long as the schedule's refinements misses it, a second look tells
+        // whether two of them serve with some margin or three are needed, and
+        // the next steps run so without a look: a look drains the queue (45 us
+        // of a step's 200 on 64x128 cells, 0.1 s a step, where two serve; a
+        // third one launched for nothing costs 75).
         const bool automatic = opt->max_inner <= 0 && opt->max_outer <= 0 && c.method == 2;
         const int K = opt->max_inner > 0 ? opt->max_inner : 16;
         const int R = opt->max_outer > 0 ? std::min(opt->max_outer, kAccRefine - 1) : 2;
         std::vector<int> full((size_t)R, K);
         full.push_back(0);
-        int first = std::min(6, K);
+        int first = std::min(6, K), unseen = 0, need = 3;
         for (int k = 0; k < nsteps; ++k) {
             c.advect();
             c.assemble();
@@ -2130,18 +2135,33 @@ int step_in_scratch(void* scratch, size_t bytes, const sf_options* opt,
             if (!automatic) {
                 c.solve(false, false);
             } else {
-                c.sched.insert(c.sched.begin(), first);
-                c.cheb_refinement(0);
-                double r0, r1;
-                c.first_refinement(r0, r1);
-                // (a hair inside the tolerance: the device sums in another order)
-                if (!(r1 <= c.sp.tol * (1.0 - 1e-9)))
-                    for (size_t q = 1; q < c.sched.size(); ++q) c.cheb_refinement(q);
-                // the next step's: a quarter of the tolerance at this step's
-                // fall per line solve, of which the assembly makes one
-                const double fall = std::log(r1 / r0) / (first + 1);
-                const double n = fall < 0.0 ? std::log(0.25 * c.sp.tol / r0) / fall : (double)K;
-                first = n >= 1.0 && n < (double)K ? std::max((int)std::ceil(n) - 1, 1) : n < 1.0 ? 1 : K;
+                if (unseen == 0 || need == 3) c.sched.insert(c.sched.begin(), unseen > 0 ? K : first);
+                size_t q = 0;
+                bool done = false;
+                if (unseen > 0) {
+                    --unseen;
+                } else {
+                    double r0, r1;
+                    // (a hair inside the tolerance: the device sums in another order)
+                    const double tol = c.sp.tol * (1.0 - 1e-9);
+                    c.cheb_refinement(q++);
+                    c.refinement_norms(1, r0, r1);
+                    done = r1 <= tol;
+                    // the next step's: a quarter of the tolerance at this step's
+                    // fall per line solve, of which the assembly makes one
+                    const int ran = first;
+                    const double fall = std::log(r1 / r0) / (ran + 1);
+                    const double n = fall < 0.0 ? std::log(0.25 * c.sp.tol / r0) / fall : (double)K;
+                    first = n >= 1.0 && n < (double)K ? std::max((int)std::ceil(n) - 1, 1) : n < 1.0 ? 1 : K;
+                    if (!done && ran == K) {
+                        c.cheb_refinement(q++);
+                        c.refinement_norms(2, r0, r1);
+                        done = r1 <= tol;
+                        need = r1 <= 0.5 * tol ? 2 : 3;
+                        if (first == K) unseen = 7;
+                    }
+                }
+                for (; !done && q < c.sched.size(); ++q) c.cheb_refinement(q);
             }
             c.update(true);
         }

@@ -1,0 +1,64 @@
+"""sf_step_noalloc on systems coupled so strongly that a first refinement of 16
+iterations does not meet the tolerance (needs an MI355X): a step solves at least
+as well as when the caller fixes the schedule of two refinements, and takes as
+long where that schedule serves."""
+import time
+
+import numpy as np
+import pytest
+
+import soapbubble_amd as sb
+from cases import make_case
+from test_zz_no_alloc import FIELDS, _Hip
+
+pytestmark = pytest.mark.gpu
+
+
+def _film(hip, n):
+    st, ua, va = make_case(n, 3, u_scale=0.5)
+    ins = [hip.put(st[k]) for k in FIELDS]
+    air = [hip.put(ua), hip.put(va)]
+    outs = [hip.put(np.full(sz, np.nan)) for _, sz in ins]
+
+    def run(dt, steps, **kw):
+        return sb.step_noalloc(sb.bubble(n, dt), sb.options("mixed", **kw), 0.0, steps,
+                               [p for p, _ in ins], [p for p, _ in air], [p for p, _ in outs])
+    return run
+
+
+@pytest.mark.parametrize("n,dt", [(64, 0.04), (64, 0.1), (128, 0.04), (128, 0.1), (256, 0.03),
+                                  (256, 0.04)])
+def test_solves_as_well(n, dt):
+    hip = _Hip()
+    run = _film(hip, n)
+    for steps in (1, 2, 3, 12, 25):
+        s, fixed = run(dt, steps), run(dt, steps, max_outer=2, max_inner=16)
+        print(f"  n={n} dt={dt} {steps} steps: {s['iterations']} iterations, residual "
+              f"{s['residual']:.1e}; fixed {fixed['iterations']}, {fixed['residual']:.1e}", flush=True)
+        assert s["residual"] <= max(1.1 * fixed["residual"], 1e-10), (s, fixed)
+        assert s["failed_solves"] <= fixed["failed_solves"], (s, fixed)
+    hip.free()
+
+
+def test_takes_no_longer_than_the_schedule():
+    """Two refinements serve here: a look now and then costs less than the
+    launches of another one (by which a step would take half as long again)."""
+    hip = _Hip()
+    run = _film(hip, 64)
+
+    def a_step(**kw):
+        def best(steps):
+            out = []
+            for _ in range(7):
+                t0 = time.perf_counter()
+                s = run(0.1, steps, **kw)
+                out.append(time.perf_counter() - t0)
+            assert s["failed_solves"] == 0 and s["iterations"] == 32, s
+            return min(out)
+        return (best(60) - best(10)) / 50
+
+    a_step()
+    auto, fixed = a_step(), a_step(max_outer=2, max_inner=16)
+    print(f"  a step: {1e6 * auto:.0f} us, with the schedule fixed {1e6 * fixed:.0f}", flush=True)
+    assert auto < 1.2 * fixed, (auto, fixed)
+    hip.free()
