@@ -754,6 +754,10 @@ struct Impl : Base {
                              &bm.err_e, &bm.err_g, &bm.cpy_e, &bm.cpy_g, &bm.e_last, &bm.e_mix};
         for (double** a : arrays) *a = dalloc<double>(n + kFieldPad, owned);
         bm.tab = tab;
+        bm.films = 0;
+        for (const BubbleDev& B : bub_h) bm.films |= B.nth < kCoarseRows ? 2 : 1;
+        bm.far = dalloc<int>((size_t)nb, owned);
+        bm.far_next = dalloc<int>((size_t)nb, owned);
         bm.bt = time_d;
         bm.dist_bits = dalloc<unsigned>((size_t)nb, owned);
         bm.flag = dalloc<int>((size_t)nb, owned);

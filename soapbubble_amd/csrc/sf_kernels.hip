@@ -2406,6 +2406,17 @@ __global__ void k_row_stats(const int2* __restrict__ rows, const BubbleDev* __re
 // four spill: 275, 259 and 282 us a 512x1024 step). A step with them: 512x1024
 // 387 -> 259 us, 1024x2048 1351 -> 905 us, 1000x2000 1715 -> 955 us against
 // separate map lookups, 25 field samples and library arc functions per cell.
+// Where a film's maps have come too far apart for the fast forms somewhere, a
+// wave that holds such a cell computes both forms. On a coarse film
+// (kCoarseRows), whose launches last as long as their longest wave, that costs
+// more than the general form everywhere: its kernels note it, and until the maps
+// restart take the general form at once, without the NaN-skipping samplers. In
+// a flow of 0.8 cells a step 64x128 178 -> 143 us a step, 128x256 178 -> 144;
+// fine films do not have that form, whose registers cost them 8 % (1024x2048).
+
+// The films a launch of those three kernels takes: fine ones, in a context that
+// has no others; coarse ones; the fine ones of a context that has both.
+constexpr int kFineFilms = 0, kCoarseFilms = 1, kFineAmongCoarse = 2;
 
 // initMapping (solver.cu:12-22) and Init/InitLast = current, changes = 0
 __device__ __forceinline__ void set_identity(const UMap& M, size_t c, double h, int j, int i) {
@@ -2434,6 +2445,7 @@ __global__ __launch_bounds__(256) void k_bm_init(const int4* __restrict__ tiles,
     P.e_delta[c] = P.e_deltalast[c] = P.g_delta[c] = P.g_deltalast[c] = 0.0;
     P.e_last[c] = P.e_init[c];
     P.e_mix[c] = P.blend * P.e_init[c];
+    if (j == 0 && i == 0) P.far[tl.x] = P.far_next[tl.x] = 0;
 }
 
 // traceGreatCircle from the cell centre (j + 1/2, i) over dt (either sign)
@@ -2458,7 +2470,7 @@ __device__ __forceinline__ void trace_centre(const Field<T>& uth, const Field<T>
 template <typename T, bool NANS>
 __device__ __forceinline__ void bm_maps_cell(const BubbleDev& B, const Tables& tab,
                                              const StatePtrs<T>& cur, const BimocqPtrs& P, int j,
-                                             int i) {
+                                             int i, bool direct, int* far_next) {
     const Field<T> uth{cur.uth + B.off, B.nph, B.mask, B.nth - 2};
     const Field<T> uph{cur.uph + B.off, B.nph, B.mask, B.nth - 1};
     const size_t o = (size_t)B.off, c = o + (size_t)j * B.nph + i;
@@ -2467,9 +2479,13 @@ __device__ __forceinline__ void bm_maps_cell(const BubbleDev& B, const Tables& t
         trace_centre<T, NANS>(uth, uph, tab, B, dir == 0 ? -TabSel<T>::dt(B) : TabSel<T>::dt(B),
                               j, i, tx, ty);
         const UMap& from = dir == 0 ? P.fwd : P.bwd;
-        bool near = true;
-        U3 s = sample_map_near(from, o, B, tx, ty, near);
-        if (!near) s = sample_map_u(from, o, B.nth, B.nph, tx, ty);
+        bool near = !direct;
+        U3 s{};
+        if (near) s = sample_map_near(from, o, B, tx, ty, near);
+        if (!near) {
+            if (far_next && !direct) *far_next = 1;
+            s = sample_map_u(from, o, B.nth, B.nph, tx, ty);
+        }
         const UMap& out = dir == 0 ? P.nfwd : P.nbwd;
         out.x[c] = s.x;
         out.y[c] = s.y;
@@ -2477,7 +2493,7 @@ __device__ __forceinline__ void bm_maps_cell(const BubbleDev& B, const Tables& t
     }
 }
 
-template <typename T>
+template <typename T, int FILMS>
 __global__ __launch_bounds__(256, 3) void k_bm_maps(const int4* __restrict__ tiles,
                                                  const BubbleDev* __restrict__ bub,
                                                  const BubbleTime* __restrict__ btime, Tables tab,
@@ -2485,18 +2501,22 @@ __global__ __launch_bounds__(256, 3) void k_bm_maps(const int4* __restrict__ til
     const int4 tl = tiles[blockIdx.x];
     if (tl.x < 0 || stopped_early(btime[tl.x])) return;
     const BubbleDev B = bub[tl.x];
+    constexpr bool COARSE = FILMS == kCoarseFilms;
+    if (FILMS != kFineFilms && (B.nth < kCoarseRows) != COARSE) return;
     int j, i;
     tile_cell(tl, j, i);
     if (j >= B.nth || i >= B.nph) return;
+    const bool direct = COARSE && P.far[tl.x] != 0;
+    int* far_next = COARSE ? P.far_next + tl.x : nullptr;
     if (btime[tl.x].nans)
-        bm_maps_cell<T, true>(B, tab, cur, P, j, i);
+        bm_maps_cell<T, true>(B, tab, cur, P, j, i, direct, far_next);
     else
-        bm_maps_cell<T, false>(B, tab, cur, P, j, i);
+        bm_maps_cell<T, false>(B, tab, cur, P, j, i, direct, far_next);
 }
 
 // advectionCenteredBimocq (bubble.cu:967-1013) through the new backward map
 // and the previous interval's backward map; overwrites the plain eta*.
-template <typename T>
+template <typename T, bool NANS>
 __device__ __forceinline__ void bm_eta_cell(const BubbleDev& B, StatePtrs<T> cur, StatePtrs<T> out,
                                             const BimocqPtrs& P, int j, int i) {
     const size_t o = (size_t)B.off, c = o + (size_t)j * B.nph + i;
@@ -2518,18 +2538,18 @@ __device__ __forceinline__ void bm_eta_cell(const BubbleDev& B, StatePtrs<T> cur
         const P2d ip = index_near(B.invh, sample_map_u(P.nbwd, o, B.nth, B.nph,
                                                         j + 0.5 + kMsDx[q], i + kMsDy[q]), cr);
         const P2d lp = index_near(B.invh, sample_map_u(P.prev, o, B.nth, B.nph, ip.x, ip.y), cr);
-        const double d = sample_centered<double, true>(fd, B.nth, ip.x, ip.y);
+        const double d = sample_centered<double, NANS>(fd, B.nth, ip.x, ip.y);
         a += (1.0 - bl) * w *
-             (sample_centered<double, true>(fil, B.nth, lp.x, lp.y) + d +
-              sample_centered<double, true>(fdl, B.nth, lp.x, lp.y));
-        a += bl * w * (sample_centered<double, true>(fin, B.nth, ip.x, ip.y) + d);
+             (sample_centered<double, NANS>(fil, B.nth, lp.x, lp.y) + d +
+              sample_centered<double, NANS>(fdl, B.nth, lp.x, lp.y));
+        a += bl * w * (sample_centered<double, NANS>(fin, B.nth, ip.x, ip.y) + d);
     }
     out.eta[c] = (T)fmax(kThresh, a);
 }
 
-// The same without NaNs and where the maps are smooth: the samples are of the two sums the formula above adds up, one each at ip
-// and lp (10 bilinear samples instead of 25). False: not the case here,
-// nothing written.
+// The same without NaNs and where the maps are smooth: the samples are of the
+// two sums the formula above adds up, one each at ip and lp (10 bilinear
+// samples instead of 25). False: not the case here, nothing written.
 template <typename T>
 __device__ __forceinline__ bool bm_eta_near(const BubbleDev& B, StatePtrs<T> cur, StatePtrs<T> out,
                                             const BimocqPtrs& P, int j, int i) {
@@ -2557,29 +2577,36 @@ __device__ __forceinline__ bool bm_eta_near(const BubbleDev& B, StatePtrs<T> cur
 }
 
 // The NaN-skipping samplers only once a NaN exists in the bubble (its
-// sticky flag; the BIMOCQ fields derive from eta, which holds none before).
-template <typename T>
+// sticky flag; the BIMOCQ fields derive from eta, which holds none before) and,
+// on fine films, where the maps vary too fast for the fast form.
+template <typename T, int FILMS>
 __global__ __launch_bounds__(256, 3) void k_bm_eta(const int4* __restrict__ tiles,
                                                 const BubbleDev* __restrict__ bub,
                                                 StatePtrs<T> cur, StatePtrs<T> out, BimocqPtrs P) {
     const int4 tl = tiles[blockIdx.x];
     if (tl.x < 0) return;
     const BubbleDev B = bub[tl.x];
+    constexpr bool COARSE = FILMS == kCoarseFilms;
+    if (FILMS != kFineFilms && (B.nth < kCoarseRows) != COARSE) return;
     int j, i;
     tile_cell(tl, j, i);
     if (j >= B.nth || i >= B.nph) return;
-    // the fast form; maps that vary too fast nearby take the general one
-    if (P.bt[tl.x].nans || !bm_eta_near<T>(B, cur, out, P, j, i)) bm_eta_cell<T>(B, cur, out, P, j, i);
+    const bool nans = P.bt[tl.x].nans != 0, direct = COARSE && P.far[tl.x] != 0;
+    if (!nans && !direct && bm_eta_near<T>(B, cur, out, P, j, i)) return;
+    if (COARSE && !nans) {
+        if (!direct) P.far_next[tl.x] = 1;
+        bm_eta_cell<T, false>(B, cur, out, P, j, i);
+    } else {
+        bm_eta_cell<T, true>(B, cur, out, P, j, i);
+    }
 }
 
-// accumulateChangesCentered (bubble.cu:2081-2114) for eta and Gamma through
-// the new forward map, the new maps made current, and the distortion
-// (estimateDistortion, bubble.cu:1133-1168) of the new maps: its block
-// maximum goes to the bubble's running maximum.
-// The changes pulled back to one cell (de, dg) and the squared chords from
-// its centre to the two round trips of the maps: the general form, and the
-// one without NaNs, away from the poles and where the maps are smooth (false:
-// not the case here).
+// accumulateChangesCentered (bubble.cu:2081-2114) for eta and Gamma and the two
+// round trips of estimateDistortion (bubble.cu:1133-1168) of one cell: the
+// changes pulled back through the new forward map (de, dg), the cell's centre
+// mapped forth and back (a) and back and forth (e). The general form, and the
+// one without NaNs where the maps are smooth (false: not the case here).
+template <bool NANS>
 __device__ __forceinline__ void bm_accum_cell(const BubbleDev& B, const BimocqPtrs& P, int j, int i,
                                               const CellRef& cr, double& de, double& dg, U3& a, U3& e) {
     const size_t o = (size_t)B.off, c = o + (size_t)j * B.nph + i;
@@ -2593,8 +2620,8 @@ __device__ __forceinline__ void bm_accum_cell(const BubbleDev& B, const BimocqPt
         const double w = ns == 5 ? kMsW[q] : 1.0;
         const P2d ip = index_near(B.invh, sample_map_u(P.nfwd, o, B.nth, B.nph,
                                                         j + 0.5 + kMsDx[q], i + kMsDy[q]), cr);
-        de += w * sample_centered<double, true>(ce, B.nth, ip.x, ip.y);
-        dg += w * sample_centered<double, true>(cg, B.nth, ip.x, ip.y);
+        de += w * sample_centered<double, NANS>(ce, B.nth, ip.x, ip.y);
+        dg += w * sample_centered<double, NANS>(cg, B.nth, ip.x, ip.y);
     }
     const P2d fi = index_near(B.invh, map_at(P.nfwd, c), cr);
     const P2d bi = index_near(B.invh, map_at(P.nbwd, c), cr);
@@ -2625,6 +2652,9 @@ __device__ __forceinline__ bool bm_accum_near(const BubbleDev& B, const BimocqPt
     return near;
 }
 
+// The changes added up, the new maps made current, and the block's largest
+// distortion to the bubble's running maximum.
+template <int FILMS>
 __global__ __launch_bounds__(256, 3) void k_bm_accum(const int4* __restrict__ tiles,
                                                   const BubbleDev* __restrict__ bub,
                                                   BimocqPtrs P) {
@@ -2632,6 +2662,8 @@ __global__ __launch_bounds__(256, 3) void k_bm_accum(const int4* __restrict__ ti
     const int4 tl = tiles[blockIdx.x];
     if (tl.x < 0 || stopped(P.bt[tl.x])) return;
     const BubbleDev B = bub[tl.x];
+    constexpr bool COARSE = FILMS == kCoarseFilms;
+    if (FILMS != kFineFilms && (B.nth < kCoarseRows) != COARSE) return;
     int j, i;
     tile_cell(tl, j, i);
     double chord2 = 0.0;
@@ -2642,8 +2674,15 @@ __global__ __launch_bounds__(256, 3) void k_bm_accum(const int4* __restrict__ ti
         U3 a, e;
         // the changes derive from eta and Gamma: NaN-free while the bubble's
         // flag is clear (k_update sets it before this launch)
-        if (P.bt[tl.x].nans || !bm_accum_near(B, P, j, i, cr, de, dg, a, e))
-            bm_accum_cell(B, P, j, i, cr, de, dg, a, e);
+        const bool nans = P.bt[tl.x].nans != 0, direct = COARSE && P.far[tl.x] != 0;
+        if (nans || direct || !bm_accum_near(B, P, j, i, cr, de, dg, a, e)) {
+            if (COARSE && !nans) {
+                if (!direct) P.far_next[tl.x] = 1;
+                bm_accum_cell<false>(B, P, j, i, cr, de, dg, a, e);
+            } else {
+                bm_accum_cell<true>(B, P, j, i, cr, de, dg, a, e);
+            }
+        }
         P.e_delta[c] += de;
         P.g_delta[c] += dg;
         P.e_mix[c] = fma(P.blend, P.e_init[c], P.e_delta[c]);
@@ -2682,6 +2721,8 @@ __global__ void k_bm_decide(int nb, BimocqPtrs P) {
     const int f = (double)d > P.threshold ? 1 : 0;
     P.flag[b] = f;
     P.reinits[b] += f;
+    P.far[b] = f ? 0 : P.far[b] | P.far_next[b];
+    P.far_next[b] = 0;
 }
 
 // correctCentered1 (bubble.cu:2180-2220): the error of the forward-mapped
@@ -3125,21 +3166,39 @@ void launch_bimocq_init(hipStream_t s, const LaunchGeom& g, const BubbleDev* bub
                         StatePtrs<T> cur, const BimocqPtrs& P) {
     hipLaunchKernelGGL(k_bm_init<T>, dim3(g.ntiles), dim3(256), 0, s, g.tiles, bub, cur, P);
 }
+// fine films and coarse ones by kernels of their own
+#define SF_BM_FILMS(LAUNCH)                              \
+    do {                                                 \
+        if (P.films == 1) LAUNCH(kFineFilms);            \
+        if (P.films & 2) LAUNCH(kCoarseFilms);           \
+        if (P.films == 3) LAUNCH(kFineAmongCoarse);      \
+    } while (0)
 template <typename T>
 void launch_bimocq_maps(hipStream_t s, const LaunchGeom& g, const BubbleDev* bub,
                         BubbleTime* bt, const Tables& tab, StatePtrs<T> cur, const BimocqPtrs& P) {
-    hipLaunchKernelGGL(k_bm_maps<T>, dim3(g.ntiles), dim3(256), 0, s, g.tiles, bub, bt, tab, cur, P);
+#define SF_LAUNCH(F)                                                                              \
+    hipLaunchKernelGGL((k_bm_maps<T, F>), dim3(g.ntiles), dim3(256), 0, s, g.tiles, bub, bt, tab, \
+                       cur, P)
+    SF_BM_FILMS(SF_LAUNCH);
+#undef SF_LAUNCH
 }
 template <typename T>
 void launch_bimocq_eta(hipStream_t s, const LaunchGeom& g, const BubbleDev* bub,
                        StatePtrs<T> cur, StatePtrs<T> out, const BimocqPtrs& P) {
-    hipLaunchKernelGGL(k_bm_eta<T>, dim3(g.ntiles), dim3(256), 0, s, g.tiles, bub, cur, out, P);
+#define SF_LAUNCH(F)                                                                              \
+    hipLaunchKernelGGL((k_bm_eta<T, F>), dim3(g.ntiles), dim3(256), 0, s, g.tiles, bub, cur, out, P)
+    SF_BM_FILMS(SF_LAUNCH);
+#undef SF_LAUNCH
 }
 void launch_bimocq_accumulate(hipStream_t s, const LaunchGeom& g, const BubbleDev* bub, int nb,
                               const BimocqPtrs& P) {
-    hipLaunchKernelGGL(k_bm_accum, dim3(g.ntiles), dim3(256), 0, s, g.tiles, bub, P);
+#define SF_LAUNCH(F)                                                                              \
+    hipLaunchKernelGGL(k_bm_accum<F>, dim3(g.ntiles), dim3(256), 0, s, g.tiles, bub, P)
+    SF_BM_FILMS(SF_LAUNCH);
+#undef SF_LAUNCH
     hipLaunchKernelGGL(k_bm_decide, dim3((nb + 63) / 64), dim3(64), 0, s, nb, P);
 }
+#undef SF_BM_FILMS
 template <typename T>
 void launch_bimocq_reinit(hipStream_t s, const LaunchGeom& g, const BubbleDev* bub,
                           StatePtrs<T> cur, const BimocqPtrs& P) {

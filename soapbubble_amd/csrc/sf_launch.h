@@ -24,9 +24,17 @@ struct BimocqPtrs {
     int* reinits;          // per bubble: reinitialisations so far
     double blend, threshold;
     int multisample;
+    int films;             // films of the context: 1 fine ones, 2 coarse ones (kCoarseRows)
+    int *far, *far_next;   // per coarse film: maps too far apart for the fast forms, and
+                           // whether this step found them so
     Tables tab;            // the grid's sin/cos tables (cell-relative map positions)
     const BubbleTime* bt;  // per bubble: the NaN flag selects the NaN-skipping samplers
 };
+// A film of fewer rows is coarse: it leaves the chip room, and a launch lasts as
+// long as its longest wave. With and without the note of maps stretched beyond
+// the fast forms, in a flow of 0.8 cells a step: 128x256 178, 144 us a step;
+// 160x320 199, 201 (260, 214 in the slowest stretches); 200x400 169, 198.
+constexpr int kCoarseRows = 192;
 
 template <typename T>
 struct StatePtrs {
