@@ -1090,6 +1090,8 @@ struct Impl : Base {
             // a late look costs little and an early one a wait for the
             // device), then at growing intervals; the outer one not before
             // the first refinement of a solve that never converges there.
+            // Without a solve before (of this film, at this step) every four
+            // iterations, or every one of a preconditioner of many launches.
             for (int k = 0; k < max_outer; ++k) {
                 for (const LaunchGeom& rg : pgeo)
                     launch_spmv<Ti>(stream, rg, bub_d, ctl_d, sys(x64[0]), p[1], p[0], 0, sp, partR,
@@ -1103,13 +1105,14 @@ struct Impl : Base {
                 }
                 for (int b = 0; b < nb; ++b) before[b] = k > 0 ? c[b].iters : 0;
                 cgstep(0);
-                int look = k < (int)last_used.size() ? std::max(last_used[k], 1) : mg || spectral ? 1 : 3;
+                const bool seen_before = k < (int)last_used.size();
+                int look = seen_before ? std::max(last_used[k], 1) : mg || spectral ? 1 : 3;
                 bool seen = false;
                 for (int it = 1; it < max_inner && !seen; ++it) {
                     inner(it);
                     if (it < look) continue;
                     seen = all_flags(c, true);
-                    look = it + std::max(1, it / 8);
+                    look = it + (seen_before || mg || spectral ? std::max(1, it / 8) : 4);
                 }
                 if (!seen) all_flags(c, true);
                 int mx = 0;
@@ -1173,6 +1176,7 @@ struct Impl : Base {
         SF_HIP(hipMemcpyAsync(dst + B.off, tmp.data(), N * sizeof(T), hipMemcpyHostToDevice, stream));
         if (field == SF_FIELD_ETA || field == SF_FIELD_GAMMA) bimocq_dirty = true;
         if (field <= SF_FIELD_GAMMA) reset_guess(b);
+        if (field <= SF_FIELD_GAMMA) last_used.clear();
         if (field <= SF_FIELD_GAMMA && spectral) sp_recal = true;
         if (field <= SF_FIELD_GAMMA) {
             // a new state steps again after a failed solve; the advection
@@ -2277,6 +2281,7 @@ int sf_set_dt(sf_ctx* ctx, int32_t b, double dt_seconds) {
                 // to the old step
                 c.time_h[k].ghist = c.time_h[k].gpend = 0;
                 c.host_hist = 0;
+                c.last_used.clear();
                 reset_gate(c);
             }
             set_step(c.bub_h[k], dtn);
