@@ -224,8 +224,9 @@ int sf_synchronize(sf_ctx* ctx);
  * opt->max_inner inner iterations (0: 16) plus one spare refinement, and a
  * bubble that has converged skips the rest (with both 0, after a first
  * refinement as long as the step before suggests; the rest is launched only
- * if that one misses the tolerance); solves that miss the tolerance are
- * counted in stats->failed_solves (stats may be NULL). t_seconds is the
+ * if that one misses the tolerance or, on strongly coupled systems, as the
+ * steps before needed it); solves that miss the tolerance are counted in
+ * stats->failed_solves (stats may be NULL). t_seconds is the
  * air-flow time at the first step. Work is queued on `stream` (a
  * hipStream_t; NULL: the default stream) after what the caller queued there;
  * the call returns when it has finished. The array is shared by every call

@@ -1011,11 +1011,11 @@ struct Impl : Base {
         after = std::sqrt(v[1]) / bb;
     }
 
-    // Refinement loop after the assembly. Host-driven: convergence flags are
-    // read back after each residual and every four inner iterations (the
-    // plain path, and the calibration steps of the graph schedule). Fixed:
-    // the calibrated schedule, every kernel launched, converged bubbles
-    // skip the work (graph capture).
+    // Refinement loop after the assembly. Host-driven (the plain path, and the
+    // calibration steps of the graph schedule): the convergence flags are read
+    // back where the solve before says they are likely to be set. Fixed: the
+    // calibrated schedule, every kernel launched, converged bubbles skip the
+    // work (graph capture), and a gate behind it in the stiff regime.
     void solve(bool host_driven, bool finalize) override {
         if (host_driven && method == 2 && auto_method() && stiff_for_chebyshev()) {
             // the automatic inner method continues with PCG, preconditioned

@@ -202,8 +202,6 @@ __device__ __forceinline__ double qdiv(double a, double y) {
     if (ay >= 1e-300 && ay <= 1e300) return a * rcp64(y);
     return a / y;
 }
-__device__ __forceinline__ float trcp(float x) { return __builtin_amdgcn_rcpf(x); }
-__device__ __forceinline__ double trcp(double x) { return rcp64(x); }
 
 __device__ __forceinline__ void tsincos(float x, float* s, float* c) { sincosf(x, s, c); }
 __device__ __forceinline__ void tsincos(double x, double* s, double* c) { sincos(x, s, c); }
@@ -1233,14 +1231,6 @@ __device__ __forceinline__ int block_steps(const int* __restrict__ rsteps, int b
     const int r = (int)red[0];
     __syncthreads();
     return r;
-}
-
-// Maximum of the per-row values [base, base+n) of one slot.
-__device__ __forceinline__ double max_partials(const double* __restrict__ part, int base, int n,
-                                               double* red) {
-    double m = 0.0;
-    for (int r = threadIdx.x; r < n; r += blockDim.x) m = fmax(m, part[base + r]);
-    return block_max(m, red);
 }
 
 // Sum the per-row partials [base, base+n) of NV interleaved slots
