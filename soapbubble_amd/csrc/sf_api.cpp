@@ -276,6 +276,8 @@ struct Base {
     std::vector<int> sp_short;
     int sp_margin = 1, sp_accept = 0;
     bool sp_uneven = false;        // the gate closed on an uneven film
+    int gate_mode = -1;            // how the gate stands open (accept), -1: unknown
+    int gate_done = 0;             // its count of applied steps when last read
     bool trace_solve = std::getenv("SF_SOLVE_TRACE") != nullptr;
     int steps_done = 0;
     int stage = 0;            // 0 idle, 1 advected, 2 assembled, 3 solved
@@ -341,7 +343,11 @@ struct Base {
         if (!gate_d) gate_d = dalloc<StepGate>(1, owned);
     }
     void gate_read(int slot) { launch_gate_read(stream, gate_d, gate_h + slot); }
-    void gate_open() { launch_gate_open(stream, nb, time_d, gate_d, acc, sp_accept > 0 ? 1 : 0); }
+    void gate_open() {
+        gate_mode = sp_accept > 0 ? 1 : 0;
+        gate_done = 0;
+        launch_gate_open(stream, nb, time_d, gate_d, acc, gate_mode);
+    }
     // one inner Chebyshev launch (iteration `it` of refinement `kr`)
     virtual void inner_launch(int it, int kr) = 0;
     // average time of n launches of the advection / of inner iteration 2 of
@@ -2422,7 +2428,9 @@ int sf_step(sf_ctx* ctx, int32_t nsteps) {
                 const bool gated = c.gated(), watch = adapt || gated;
                 if (k < nsteps) {
                     const int k0 = k;
-                    if (gated) c.gate_open();
+                    const int mode = c.sp_accept > 0 ? 1 : 0;
+                    if (gated && c.gate_mode != mode) c.gate_open();
+                    c.gate_mode = -1;   // until its state has been read
                     SF_HIP(hipEventRecord(c.ev[0], c.stream));
                     int chunk = 0;
                     // chunks until misses close the gate again
@@ -2460,17 +2468,20 @@ int sf_step(sf_ctx* ctx, int32_t nsteps) {
                         if (again) {
                             // the step that closed the gate is the host's
                             // (a miss) or multigrid's (an uneven film)
-                            c.host_hist -= k - k0 - g.done;
-                            k = k0 + g.done;
+                            const int done = (int)((unsigned)g.done - (unsigned)c.gate_done);
+                            c.host_hist -= k - k0 - done;
+                            k = k0 + done;
                             c.gate_open();
                             if (g.why & kGateUneven) c.sp_uneven = true;
                             else c.sp_short = c.sched;
                             drop_calibration(c);
                             if (c.trace_solve)
                                 std::fprintf(stderr, "[sf solve] gate closed after %d steps:%s%s\n",
-                                             g.done, g.why & kGateMissed ? " missed" : "",
+                                             done, g.why & kGateMissed ? " missed" : "",
                                              g.why & kGateUneven ? " uneven" : "");
                         } else {
+                            c.gate_mode = mode;
+                            c.gate_done = g.done;
                             again = k < nsteps;   // on with the gate as it is from here
                         }
                     }

@@ -21,6 +21,7 @@
 #include "sf_device.h"
 #include "sf_launch.h"
 
+#include <algorithm>
 #include <type_traits>
 
 namespace sfk {
@@ -1868,15 +1869,13 @@ __global__ __launch_bounds__(1024) void k_gate(int nb, const BubbleDev* __restri
                                                double max_condition) {
     __shared__ int bad[16];
     const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6, nw = blockDim.x >> 6;
-    if (g->why) return;
-    const int accept = g->accept;
+    const int closed = g->why, accept = g->accept;
     int why = 0;
     for (int b = wid; b < nb; b += nw) {
-        if ((bt[b].stop & 3) == 3) continue;
-        const long long r0 = bub[b].pr0;
+        const int r0 = bub[b].pr0, nth = bub[b].nth, stop = bt[b].stop;
         double rr = 0.0, bb = 0.0;
         float hi = 0.0f, lo = 0.0f;
-        for (int j = lane; j < bub[b].nth; j += 64) {
+        for (int j = lane; j < nth; j += 64) {
             rr += partR[r0 + j];
             bb += partR[stride + r0 + j];
             if (!coef) continue;
@@ -1887,9 +1886,11 @@ __global__ __launch_bounds__(1024) void k_gate(int nb, const BubbleDev* __restri
         bb = wave_sum(bb);
         hi = wave_max(hi);
         lo = wave_max(lo);
+        if ((stop & 3) == 3) continue;
         if (!accept && !(residual_norm(rr, bb, sp.absolute) <= sp.tol)) why |= kGateMissed;
         if (!((double)hi * (double)lo <= max_condition)) why |= kGateUneven;
     }
+    if (closed) return;
     if (lane == 0) bad[wid] = why;
     __syncthreads();
     why = 0;
@@ -3038,8 +3039,8 @@ void launch_sp_line(hipStream_t s, const int4* items, int nitems, int threads, s
 void launch_gate(hipStream_t s, int nb, const BubbleDev* bub, BubbleTime* bt, StepGate* g,
                  const float* coef, const SolveParams& sp, const double* partR, long stride,
                  double max_condition) {
-    hipLaunchKernelGGL(k_gate, dim3(1), dim3(1024), 0, s, nb, bub, bt, g, coef, sp, partR, stride,
-                       max_condition);
+    hipLaunchKernelGGL(k_gate, dim3(1), dim3(64 * std::min(nb, 16)), 0, s, nb, bub, bt, g, coef, sp,
+                       partR, stride, max_condition);
 }
 void launch_gate_read(hipStream_t s, const StepGate* d, StepGate* h) {
     hipLaunchKernelGGL(k_gate_read, dim3(1), dim3(64), 0, s, d, h);
