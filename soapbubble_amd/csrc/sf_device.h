@@ -805,13 +805,12 @@ struct P2d {
 };
 
 // Index coordinates (acos z, atan2(y, x)) / h of a unit vector a few cells
-// from the centre of cell (j, i): the
-// centre's index coordinates (j + 1/2, i) plus the angles turned from it,
-// each the asin of a sine that the (sin, cos) pair of the meridian half-plane
-// (a unit vector) or the equatorial plane (scale rho) gives, by its series
-// below 1/4; farther points take acos and
-// atan2. The same angles up to rounding, phi in the centre's period rather
-// than atan2's (-pi, pi] (the samplers wrap phi either way).
+// from the centre of cell (j, i): the centre's index coordinates (j + 1/2, i)
+// plus the angles turned from it, each the asin of a sine that the (sin, cos)
+// pair of the meridian half-plane (a unit vector) or the equatorial plane
+// (scale rho) gives, by its series below 1/4; farther points take atan2. The
+// same angles up to rounding, phi in the centre's period rather than atan2's
+// (-pi, pi] (the samplers wrap phi either way).
 struct CellRef {
     double gx, gy, sT, cT, sP, cP;
 };
@@ -846,7 +845,9 @@ __device__ __forceinline__ P2d index_near(double invh, const U3& r, const CellRe
     q.x = o.gx + asin_wide(nt) * invh;
     q.y = o.gy + asin_wide(np) * invh;
     if (!(ct > 0.0 && fabs(nt) < kAsinWide && cp > 0.0 && fabs(np) < kAsinWide)) {
-        q.x = safe_acos_d(r.z) * invh;
+        // (next to a pole, where phi turns far at once, the arc cosine of z
+        // would leave theta a rounding of z over sin(theta))
+        q.x = atan2(sqrt(r2), r.z) * invh;
         q.y = atan2(r.y, r.x) * invh;
     }
     return q;
