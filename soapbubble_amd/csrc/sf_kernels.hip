@@ -2405,7 +2405,7 @@ __global__ void k_row_stats(const int2* __restrict__ rows, const BubbleDev* __re
 // FP64 vector issue and, with it, by registers: the three kernels of every
 // step are held to three waves a SIMD (168 registers; two waves unbound, and
 // four spill: 275, 259 and 282 us a 512x1024 step). A step with them: 512x1024
-// 387 -> 259 us, 1024x2048 1351 -> 905 us, 1000x2000 1715 -> 955 us against
+// 387 -> 246 us, 1024x2048 1371 -> 875 us, 1000x2000 1722 -> 898 us against
 // separate map lookups, 25 field samples and library arc functions per cell.
 // Where a film's maps have come too far apart for the fast forms somewhere, a
 // wave that holds such a cell computes both forms. On a coarse film
