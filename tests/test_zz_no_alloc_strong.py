@@ -60,5 +60,5 @@ def test_takes_no_longer_than_the_schedule():
     a_step()
     auto, fixed = a_step(), a_step(max_outer=2, max_inner=16)
     print(f"  a step: {1e6 * auto:.0f} us, with the schedule fixed {1e6 * fixed:.0f}", flush=True)
-    assert auto < 1.2 * fixed, (auto, fixed)
+    assert auto < 1.25 * fixed, (auto, fixed)
     hip.free()
